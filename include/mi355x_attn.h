@@ -181,6 +181,16 @@ int ma_paged_verify(const void* q, int64_t q_stride_tok, int64_t q_stride_head, 
 size_t ma_extend_workspace_bytes(int64_t num_tokens, int num_q_heads, int num_kv_heads, int batch);
 
 /*
+ * Bytes of workspace with which ma_paged_extend can also cut row tiles into key pieces
+ * (at least ma_extend_workspace_bytes; equal to it where a call has row tiles enough to
+ * fill the chip several times). The pieces' partial results take 128 KB or less per piece
+ * and kv head, at most two pieces per compute unit. With a smaller workspace the call runs
+ * whole row tiles; the result is the same up to rounding. 0 for bad arguments.
+ */
+size_t ma_extend_split_workspace_bytes(int64_t num_tokens, int num_q_heads, int num_kv_heads, int batch,
+                                       int head_dim);
+
+/*
  * Prefix-aware paged extend (chunked prefill), MFMA tiles.
  * Replaces the reference's paged extend kernel (_kernels_paged.py:55-393 via
  * get_paged_kernel, _kernels_paged.py:414-436, called from paged_forward,
@@ -194,8 +204,9 @@ size_t ma_extend_workspace_bytes(int64_t num_tokens, int num_q_heads, int num_kv
  *   batch <= 16384. No host-side maximum of the query lengths is needed: a plan kernel
  *   lists the row tiles on the device (reference: max_seq_len from seq_lens.max().item(),
  *   _paged_adapter.py:605-606).
- *   workspace: ma_extend_workspace_bytes(num_tokens, ...) bytes, 256-byte aligned, no
- *   initialisation; calls that overlap in time must use different workspaces.
+ *   workspace: ma_extend_workspace_bytes(num_tokens, ...) bytes or more, 256-byte aligned,
+ *   no initialisation; with ma_extend_split_workspace_bytes(...) bytes a call with few row
+ *   tiles also splits their keys over workgroups. Calls that overlap in time must use different workspaces.
  *   The new tokens' K/V must already be in the pools.
  *   out [num_tokens, num_q_heads, head_dim] in out_dtype (q_dtype or MA_DT_F32).
  */

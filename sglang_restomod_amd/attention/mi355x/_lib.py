@@ -86,6 +86,7 @@ SIGNATURES = {
         c_void_p, c_void_p, c_void_p,                 # k_out, v_out, stream
     ]),
     "ma_extend_workspace_bytes": (c_size_t, [c_int64, c_int, c_int, c_int]),
+    "ma_extend_split_workspace_bytes": (c_size_t, [c_int64, c_int, c_int, c_int, c_int]),
     "ma_paged_extend": (c_int, [
         c_void_p, c_int64, c_int64, c_int, c_int64,   # q, strides, dtype, num_tokens
         c_void_p, c_void_p, c_int64, c_int64, c_int,  # k, v, strides, kv dtype

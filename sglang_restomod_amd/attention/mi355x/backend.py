@@ -123,6 +123,7 @@ class MI355XAttnBackend(_EngineBase):
         self.forward_metadata: Optional[MI355XForwardMetadata] = None
         self._workspace: Optional[torch.Tensor] = None
         self._extend_ws: Optional[torch.Tensor] = None
+        self._captured_ws: list = []  # extend workspaces whose addresses captured graphs hold
         # graph buffers (init_cuda_graph_state)
         self._cg_max_bs = 0
         self._cg_row_index: Optional[torch.Tensor] = None
@@ -259,20 +260,31 @@ class MI355XAttnBackend(_EngineBase):
         return self._workspace
 
     def _workspace_for(self, mode: str, num_tokens: int, hq: int, hkv: int, batch: int) -> torch.Tensor:
-        """The split-KV workspace, which also holds an extend call's work list (8 bytes
-        per row tile); a larger buffer only for a batch whose list does not fit."""
+        """The split-KV workspace for verify; for extend whichever buffer holds the call's
+        work list and key pieces (the split-KV workspace, or one of its own that grows). A
+        capture never allocates: it takes a buffer that holds at least the work list, and
+        that buffer then lives as long as the backend (the graph keeps its address)."""
         ws = self.splitkv_workspace()
         if mode == MODE_VERIFY:
             return ws
-        need = ops.extend_workspace_bytes(num_tokens, hq, hkv, batch)
-        if ws.numel() >= need:
+        want = ops.extend_split_workspace_bytes(num_tokens, hq, hkv, batch, self.head_dim)
+        if ws.numel() >= want:
             return ws
-        if self._extend_ws is None or self._extend_ws.numel() < need:
-            if torch.cuda.is_current_stream_capturing():
-                raise RuntimeError(f"an extend of {num_tokens} tokens needs {need} workspace bytes; "
-                                   "capture smaller batches")
-            self._extend_ws = ops.extend_workspace(self.device, num_tokens, hq, hkv, batch)
-        return self._extend_ws
+        own = self._extend_ws
+        capturing = torch.cuda.is_current_stream_capturing()
+        if own is None or own.numel() < want:
+            if capturing:
+                need = ops.extend_workspace_bytes(num_tokens, hq, hkv, batch)
+                if ws.numel() >= need and (own is None or own.numel() < ws.numel()):
+                    return ws
+                if own is None or own.numel() < need:
+                    raise RuntimeError(f"an extend of {num_tokens} tokens needs {need} workspace bytes; "
+                                       "capture smaller batches")
+            else:
+                own = self._extend_ws = torch.empty(want, dtype=torch.uint8, device=self.device)
+        if capturing and not any(own is kept for kept in self._captured_ws):
+            self._captured_ws.append(own)
+        return own
 
     def init_cuda_graph_state(self, max_bs: int, max_num_tokens: int, kv_indices_buf=None) -> None:
         dev = self.device

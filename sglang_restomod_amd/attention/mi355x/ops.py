@@ -212,11 +212,23 @@ def extend_workspace_bytes(num_tokens: int, num_q_heads: int, num_kv_heads: int,
                                                       int(batch)))
 
 
+def extend_split_workspace_bytes(num_tokens: int, num_q_heads: int, num_kv_heads: int, batch: int,
+                                 head_dim: int) -> int:
+    """Bytes with which an extend call can also split the keys of few row tiles over the
+    chip (``ma_extend_split_workspace_bytes``)."""
+    return int(_lib.load().ma_extend_split_workspace_bytes(int(num_tokens), int(num_q_heads), int(num_kv_heads),
+                                                            int(batch), int(head_dim)))
+
+
 def extend_workspace(device: torch.device, num_tokens: int, num_q_heads: int, num_kv_heads: int,
-                     batch: int) -> torch.Tensor:
+                     batch: int, head_dim: Optional[int] = None) -> torch.Tensor:
     """A fresh workspace for ``paged_extend_forward`` calls of up to ``num_tokens`` query
-    tokens in ``batch`` sequences (callers that capture graphs keep one)."""
-    nbytes = extend_workspace_bytes(num_tokens, num_q_heads, num_kv_heads, batch)
+    tokens in ``batch`` sequences (callers that capture graphs keep one). With ``head_dim``
+    it also holds the key pieces of a call of exactly these sizes."""
+    if head_dim is None:
+        nbytes = extend_workspace_bytes(num_tokens, num_q_heads, num_kv_heads, batch)
+    else:
+        nbytes = extend_split_workspace_bytes(num_tokens, num_q_heads, num_kv_heads, batch, head_dim)
     return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
 
 
@@ -499,14 +511,15 @@ def paged_extend_forward(
     pre = None if prefix_kv_lens is None else _i32(prefix_kv_lens)
     ridx = _i64(row_index)
     lib = _lib.load()
-    nbytes = lib.ma_extend_workspace_bytes(T, Hq, Hkv, B)
     stream = _stream_ptr(dev)
     if workspace is None:
+        nbytes = lib.ma_extend_split_workspace_bytes(T, Hq, Hkv, B, D)
         ws = workspace_buffer(dev, nbytes, stream)
     else:
+        nbytes = lib.ma_extend_workspace_bytes(T, Hq, Hkv, B)
         if workspace.dtype != torch.uint8 or workspace.device != dev or workspace.numel() < nbytes:
             raise ValueError(f"workspace must be a uint8 tensor of at least {nbytes} bytes on {dev}")
-        ws = workspace
+        ws, nbytes = workspace, workspace.numel()
     status = lib.ma_paged_extend(
         q.data_ptr(), q.stride(0), q.stride(1), q_dtype_code(q.dtype), T,
         k_cache.data_ptr(), v_cache.data_ptr(), row, head, kv_dtype_code(k_cache.dtype),

@@ -43,6 +43,8 @@
 // looked up S+1 tiles ahead. The loads are inline assembly with explicit wait counts,
 // and one barrier per tile both publishes a tile and retires the stage it replaces.
 
+#include <algorithm>
+#include <atomic>
 #include <type_traits>
 
 #include "common.h"
@@ -73,6 +75,29 @@ __host__ __device__ constexpr int64_t row_tile_item(int seq, int tile) {
   return (int64_t)(((uint64_t)(uint32_t)tile << 32) | (uint32_t)seq);
 }
 
+// Key pieces of row tiles, planned where a batch has too few row tiles to fill the chip or
+// to balance over it (plan_pieces below). A piece that is not a whole row tile leaves its
+// rows' normalised O and log2 LSE in slot `slot`; extend_merge combines the slots of a tile.
+struct ExtendPiece {
+  int seq, tile;     // sequence (-1: no piece) and row tile
+  int first, count;  // key tiles [first, first + count) of the row tile's range
+  int slot;          // partial slot, or -1 when the piece is the whole row tile
+  int pad[3];
+};
+struct ExtendMerge {
+  int seq, tile;   // sequence (-1: none) and row tile
+  int slot, parts; // its pieces' slots: slot .. slot + parts - 1
+};
+struct ExtendPieces {
+  const ExtendPiece* list;  // the plan kernel's list, or null: each workgroup plans (plan_direct)
+  ExtendMerge* merges;
+  int merge_capacity;
+  int shares;    // CUs per kv head; 0: whole row tiles from the work list
+  int capacity;  // pieces per kv head that the grid and the partial slots hold
+  float* o;      // [slot][kv head][row of the tile][D] fp32
+  float* lse;    // [slot][kv head][row of the tile]
+};
+
 struct ExtendArgs {
   const void* q;
   int64_t q_stride_tok, q_stride_head;
@@ -86,7 +111,8 @@ struct ExtendArgs {
   const int32_t* prefix;
   int num_tokens;        // rows of q and out: query rows are clamped into [0, num_tokens)
   int batch, hq, hkv, group;
-  const int64_t* items;  // work list (row_tile_item)
+  const int64_t* items;  // work list (row_tile_item), when pieces is null
+  ExtendPieces pieces;   // work list of key pieces (pieces.list null: whole row tiles)
   int causal, window;
   float scale_log2;
   float v_scale;
@@ -117,6 +143,22 @@ constexpr int kPlanBuckets = 1024;      // cost classes of the counting sort
 constexpr int kPlanMaxBatch = 16384;    // per-sequence tile offsets kept in LDS
 constexpr int kPlanFixedCost = 2;       // a row tile's set-up, in key tiles
 
+// ---- key pieces ----
+// One workgroup walking a row tile's whole key range leaves compute units idle when the
+// batch has few row tiles: a chunk of 1,021 tokens of one prompt at 32 / 8 heads has 128
+// workgroups for 256 CUs, four short turns about 50. So a call with at most one row tile
+// per CU (by its token count) may have them cut into key pieces. Per call, whole row tiles
+// against pieces: that chunk 28,001 tokens into its prompt 782 -> 455 us; 4 turns of 9-130
+// tokens over 64-1,500 36.4 -> 26.0 us; 800 tokens at 8 / 1 heads after 8,000 253 -> 60 us.
+// Beyond one round of row tiles the pieces gained nothing that their merge did not cost:
+// 16 sequences of 300 tokens (75 row tiles, 32 CUs per kv head) 127 us either way.
+constexpr int kSplitSlotRounds = 2;  // pieces per CU share: a partial takes 128 KB per kv head at D = 128
+constexpr int kSplitMinTiles = 4;    // least key tiles of a piece (a workgroup's start and end cost about 3)
+constexpr int kDirectItems = 128;    // row tiles up to which each workgroup plans for itself, two per lane
+constexpr int kDirectBatch = 64;     // ... and sequences, one per lane
+constexpr int kSplitMaxItems = 1024; // row tiles the plan holds one per thread
+
+
 struct ExtendPlanArgs {
   const int32_t* qsl;
   const int32_t* seq_lens;
@@ -124,8 +166,13 @@ struct ExtendPlanArgs {
   int num_tokens;
   int batch, group, causal, window;
   int tile_rows, tile_keys;  // the extend kernel's rows per workgroup and keys per tile
-  int capacity;              // entries of items
+  int capacity;              // entries of items (or of pieces)
   int64_t* items;
+  // key pieces (shares > 0): CUs per kv head, partial slots per kv head, and the lists
+  int shares, slots;
+  ExtendPiece* pieces;
+  ExtendMerge* merges;
+  int merge_capacity;
 };
 
 // Row tiles of bm rows of a sequence with ntok query tokens.
@@ -156,6 +203,292 @@ __device__ __forceinline__ int block_exclusive_scan(int x, int* sums, int* total
   __syncthreads();  // sums is free again
   *total = all;
   return before + incl - x;
+}
+
+// Estimated time, in key tiles, of n pieces of at most `longest` of `all` key tiles on
+// `shares` CUs per kv head: the longest piece, or the mean piece times the rounds the
+// pieces make, each with a workgroup's start and end, plus the writing and reading back of
+// the `split` pieces that leave partials.
+__device__ __forceinline__ float pieces_cost(float all, float n, float longest, float split, float shares) {
+  constexpr float kStart = 5.f;       // a workgroup's start and end: about 8 us, a key tile 1.2-1.9 us
+  constexpr float kMergeSlot = 8.f;   // one partial per CU, written and read back: about 14 us
+  const float mean = (all + kStart * n) / fmaxf(n, 1.f);
+  return fmaxf(longest + kStart, mean * ceilf(n / shares)) + kMergeSlot * split / shares;
+}
+// Inclusive prefix sum over the wave's lanes, and the wave's maximum, of values >= 0, by
+// DPP moves (a few cycles a step; a cross-lane read through LDS takes over a hundred).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp0(int x) {  // x of another lane, 0 where there is none
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ int wave_scan(int x) {
+  x += dpp0<0x111, 0xf>(x);  // row_shr:1, 2, 4, 8 within rows of 16 lanes
+  x += dpp0<0x112, 0xf>(x);
+  x += dpp0<0x114, 0xf>(x);
+  x += dpp0<0x118, 0xf>(x);
+  x += dpp0<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
+  x += dpp0<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+__device__ __forceinline__ int wave_max(int x) {
+  x = max(x, dpp0<0x111, 0xf>(x));
+  x = max(x, dpp0<0x112, 0xf>(x));
+  x = max(x, dpp0<0x114, 0xf>(x));
+  x = max(x, dpp0<0x118, 0xf>(x));
+  x = max(x, dpp0<0x142, 0xa>(x));
+  x = max(x, dpp0<0x143, 0xc>(x));
+  return __builtin_amdgcn_readlane(x, 63);
+}
+// Pieces of at most cap key tiles of a row tile of c (at least one): max(1, ceil(c / cap)),
+// exact below 2^24 (a reciprocal, then one step either way).
+__device__ __forceinline__ int piece_count(int c, int cap) {
+  const int x = c + cap - 1;
+  int q = (int)((float)x * __builtin_amdgcn_rcpf((float)cap));
+  const int r = x - q * cap;
+  q += r >= cap ? 1 : r < 0 ? -1 : 0;
+  return max(q, 1);
+}
+
+// Cut the m row tiles (m <= kSplitMaxItems, one per thread) into key pieces and list them,
+// longest first. The pieces of a tile are its key tiles in near-equal shares of at most
+// `cap`. Three caps are priced (pieces_cost): whole tiles, and the least caps with which
+// the pieces make one and two rounds on the CUs, each searched for by eight waves.
+template <typename Decode>
+__device__ __forceinline__ void plan_pieces(const ExtendPlanArgs& a, int m, int* hist, int* sums, Decode&& decode) {
+  constexpr int kWavesPerSearch = kPlanThreads / 64 / 2;
+  __shared__ int cost[kSplitMaxItems];
+  __shared__ int fits[2 * kWavesPerSearch];
+  __shared__ float found_est[2];
+  __shared__ int found_cap[2];
+  __shared__ int counters[2];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  int b = -1, rt = 0, c = 0;
+  if (tid < m) c = decode(tid, &b, &rt) - kPlanFixedCost;
+  cost[tid] = c;
+  if (tid < 2) counters[tid] = 0;
+  int all;
+  block_exclusive_scan(c, sums, &all);
+  int cmax = wave_max(c);
+  if (lane == 0) sums[wave] = cmax;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kPlanThreads / 64; ++w) cmax = max(cmax, sums[w]);
+
+  // pieces over all row tiles at a cap (one wave)
+  auto pieces_at = [&](int cap) -> int {
+    int n = 0;
+    for (int t = lane; t < m; t += 64) n += piece_count(cost[t], cap);
+    return __builtin_amdgcn_readlane(wave_scan(n), 63);
+  };
+  const int round = wave / kWavesPerSearch;  // 0, 1: the search for one and two rounds
+  const int probe = wave % kWavesPerSearch;
+  const int room = min((round + 1) * a.shares, a.slots);
+  int lo = kSplitMinTiles, hi = max(cmax, kSplitMinTiles);  // the least cap that fits is in [lo, hi]
+  for (int span = hi - lo; span > 0; span /= kWavesPerSearch) {  // the same passes in every wave
+    // probes cut lo .. hi into kWavesPerSearch parts, each probed at its last value
+    const int step = (hi - lo) / kWavesPerSearch + 1;
+    const int mid = min(lo + step * (probe + 1) - 1, hi);
+    const int fit = mid >= hi || pieces_at(mid) <= room;
+    if (lane == 0) fits[wave] = fit;
+    __syncthreads();
+    int first = kWavesPerSearch - 1;
+#pragma unroll
+    for (int w = kWavesPerSearch - 1; w >= 0; --w)
+      if (fits[round * kWavesPerSearch + w]) first = w;
+    const int new_lo = lo + step * first;
+    hi = min(lo + step * (first + 1) - 1, hi);
+    lo = min(new_lo, hi);
+    __syncthreads();
+  }
+  if (probe == 0) {
+    int n = 0, split = 0, longest = 0;
+    for (int t = lane; t < m; t += 64) {
+      const int parts = piece_count(cost[t], hi);
+      n += parts;
+      split += parts > 1 ? parts : 0;
+      longest = max(longest, piece_count(cost[t], parts));
+    }
+    n = __builtin_amdgcn_readlane(wave_scan(n), 63);
+    split = __builtin_amdgcn_readlane(wave_scan(split), 63);
+    longest = wave_max(longest);
+    if (lane == 0) {
+      found_cap[round] = hi;
+      found_est[round] = n > room ? INFINITY
+                                  : pieces_cost((float)all, (float)n, (float)longest, (float)split, (float)a.shares);
+    }
+  }
+  hist[tid] = 0;
+  __syncthreads();
+  int cap = max(cmax, 1);
+  float est = pieces_cost((float)all, (float)m, (float)cmax, 0.f, (float)a.shares);
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+    if (found_est[r] < est) {
+      est = found_est[r];
+      cap = found_cap[r];
+    }
+
+  // this thread's tile: its pieces, their partial slots and merge entry
+  const int parts = b >= 0 ? piece_count(c, cap) : 0;
+  int slot = -1;
+  if (parts > 1) {
+    slot = atomicAdd(&counters[0], parts);
+    const int e = atomicAdd(&counters[1], 1);
+    if (e < a.merge_capacity) {
+      int4 MA_GLOBAL* mp = reinterpret_cast<int4 MA_GLOBAL*>(gptr_mut(a.merges)) + e;
+      mp->x = b; mp->y = rt; mp->z = slot; mp->w = parts;
+    }
+  }
+  // longest pieces first: a counting sort by length class
+  const int len = parts > 0 ? piece_count(c, parts) : 0;
+  const int lmax = min(cmax, cap);
+  const int cls = kPlanBuckets - 1 - (int)(((int64_t)len * kPlanBuckets) / ((int64_t)lmax + 1));
+  if (parts > 0) atomicAdd(&hist[cls], parts);
+  __syncthreads();
+  int unused;
+  const int first = block_exclusive_scan(hist[tid], sums, &unused);
+  hist[tid] = first;
+  __syncthreads();
+  if (parts > 0) {
+    const int pos = atomicAdd(&hist[cls], parts);
+    for (int p = 0; p < parts; ++p) {
+      if (pos + p >= a.capacity) break;
+      const int lo = (int)((int64_t)c * p / parts);
+      const int hi = (int)((int64_t)c * (p + 1) / parts);
+      int4 MA_GLOBAL* ep = reinterpret_cast<int4 MA_GLOBAL*>(gptr_mut(a.pieces) + pos + p);
+      ep[0].x = b; ep[0].y = rt; ep[0].z = lo; ep[0].w = hi - lo;
+      ep[1].x = slot < 0 ? -1 : slot + p;
+    }
+  }
+  // the rest of the lists is empty
+  int n = 0;
+  block_exclusive_scan(parts, sums, &n);
+  for (int i = n + tid; i < a.capacity; i += kPlanThreads)
+    reinterpret_cast<int4 MA_GLOBAL*>(gptr_mut(a.pieces) + i)->x = -1;
+  for (int i = counters[1] + tid; i < a.merge_capacity; i += kPlanThreads)
+    reinterpret_cast<int4 MA_GLOBAL*>(gptr_mut(a.merges) + i)->x = -1;
+}
+
+// The piece of list position `w` (per kv head), planned by the wave itself: for batches of
+// at most kDirectItems row tiles and kDirectBatch sequences, which then need no plan kernel
+// (about 6 us of a call that takes 20). Every wave of every workgroup computes the same plan
+// from the same numbers. The first workgroup of
+// kv head 0 leave each row tile's slots in `merges`.
+template <int BM, int BN>
+__device__ __forceinline__ ExtendPiece plan_direct(const ExtendArgs& a, int w, int h) {
+  constexpr int kPer = kDirectItems / 64;
+  const int lane = lane_id();
+  int nt = 0, ntok = 0, seq = 0, prefix = 0;
+  if (lane < a.batch) {
+    ntok = clamp_query_rows(gptr(a.qsl)[lane], gptr(a.qsl)[lane + 1], a.num_tokens).ntok;
+    seq = gptr(a.seq_lens)[lane];
+    prefix = a.prefix ? gptr(a.prefix)[lane] : seq - ntok;
+    nt = seq_row_tiles(ntok, a.group, BM);
+  }
+  const int incl = wave_scan(nt);
+  const int start = incl - nt;
+  const int m = min(__builtin_amdgcn_readlane(incl, 63), min(kDirectItems, a.pieces.merge_capacity));
+  // row tiles kPer * lane + x: their sequences and key tiles
+  int b[kPer], rt[kPer], c[kPer];
+  int cmax = 0, csum = 0;
+#pragma unroll
+  for (int x = 0; x < kPer; ++x) b[x] = 0;
+  for (int s = 1; s < a.batch; ++s) {
+    const int first = __builtin_amdgcn_readlane(start, s);
+#pragma unroll
+    for (int x = 0; x < kPer; ++x)
+      if (kPer * lane + x >= first) b[x] = s;
+  }
+#pragma unroll
+  for (int x = 0; x < kPer; ++x) {
+    rt[x] = kPer * lane + x - shfl_i(start, b[x]);
+    const KeyRange kr = row_tile_keys(rt[x] * BM, BM, shfl_i(ntok, b[x]), a.group, shfl_i(prefix, b[x]),
+                                      shfl_i(seq, b[x]), a.causal, a.window);
+    c[x] = (kPer * lane + x < m && kr.hi > kr.lo) ? (kr.hi - kr.lo + BN - 1) / BN : 0;
+    cmax = max(cmax, c[x]);
+    csum += c[x];
+  }
+  cmax = wave_max(cmax);
+  const int all = __builtin_amdgcn_readlane(wave_scan(csum), 63);
+  // this lane's pieces at a cap
+  int parts[kPer];
+  auto cut = [&](int cap) __attribute__((always_inline)) -> int {
+    int n = 0;
+#pragma unroll
+    for (int x = 0; x < kPer; ++x) {
+      parts[x] = kPer * lane + x < m ? piece_count(c[x], cap) : 0;
+      n += parts[x];
+    }
+    return n;
+  };
+  // Three candidates: whole tiles, and the least caps with which the pieces make one and
+  // two rounds on the CUs.
+  int cap = max(cmax, 1);
+  float est = pieces_cost((float)all, (float)m, (float)cmax, 0.f, (float)a.pieces.shares);
+#pragma unroll 1
+  for (int r = 1; r <= 2; ++r) {
+    const int room = min(r * a.pieces.shares, a.pieces.capacity);
+    if (m > room || cmax <= kSplitMinTiles) continue;
+    int lo = kSplitMinTiles, hi = cmax;  // the least cap whose pieces fit; cmax does
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      const int n = __builtin_amdgcn_readlane(wave_scan(cut(mid)), 63);
+      if (n <= room) hi = mid;
+      else lo = mid + 1;
+    }
+    const int n = __builtin_amdgcn_readlane(wave_scan(cut(lo)), 63);
+    int split = 0, longest = 0;
+#pragma unroll
+    for (int x = 0; x < kPer; ++x) {
+      split += parts[x] > 1 ? parts[x] : 0;
+      longest = max(longest, parts[x] > 0 ? piece_count(c[x], parts[x]) : 0);
+    }
+    split = __builtin_amdgcn_readlane(wave_scan(split), 63);
+    longest = wave_max(longest);
+    const float e = pieces_cost((float)all, (float)n, (float)longest, (float)split, (float)a.pieces.shares);
+    if (e < est) {
+      est = e;
+      cap = lo;
+    }
+  }
+  // list position of each tile's first piece: the last tiles come first (in a causal batch
+  // the longer ones)
+  const int mine = cut(cap);
+  const int upto = wave_scan(mine);
+  int pos[kPer];
+  pos[kPer - 1] = __builtin_amdgcn_readlane(upto, 63) - upto;
+#pragma unroll
+  for (int x = kPer - 2; x >= 0; --x) pos[x] = pos[x + 1] + parts[x + 1];
+  ExtendPiece p;
+  p.seq = -1;
+  p.tile = p.first = p.count = 0;
+  p.slot = -1;
+#pragma unroll
+  for (int x = 0; x < kPer; ++x) {
+    if (w == 0 && h == 0 && (int)threadIdx.x < 64 && kPer * lane + x < a.pieces.merge_capacity) {
+      int4 MA_GLOBAL* mp = reinterpret_cast<int4 MA_GLOBAL*>(gptr_mut(a.pieces.merges)) + kPer * lane + x;
+      mp->x = parts[x] > 1 ? b[x] : -1;
+      mp->y = rt[x];
+      mp->z = pos[x];
+      mp->w = parts[x];
+    }
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(w >= pos[x] && w < pos[x] + parts[x]);
+    if (hit) {
+      const int L = __builtin_ctzll(hit);
+      const int cx = __builtin_amdgcn_readlane(c[x], L);
+      const int np = __builtin_amdgcn_readlane(parts[x], L);
+      const int k = w - __builtin_amdgcn_readlane(pos[x], L);
+      const int lo = (int)((int64_t)cx * k / np);
+      p.seq = __builtin_amdgcn_readlane(b[x], L);
+      p.tile = __builtin_amdgcn_readlane(rt[x], L);
+      p.first = lo;
+      p.count = (int)((int64_t)cx * (k + 1) / np) - lo;
+      p.slot = np > 1 ? w : -1;
+    }
+  }
+  return p;
 }
 
 // One workgroup: list every row tile of the batch as {sequence, tile}, the ones with the
@@ -205,6 +538,11 @@ __global__ __launch_bounds__(kPlanThreads, 1) void extend_plan_kernel(const Exte
     *rt_out = rt;
     return (k.hi > k.lo ? (k.hi - k.lo + a.tile_keys - 1) / a.tile_keys : 0) + kPlanFixedCost;
   };
+
+  if (a.shares > 0) {
+    plan_pieces(a, m, hist, sums, decode);
+    return;
+  }
 
   // 2. the largest cost, which scales the classes
   int cmax = 0;
@@ -311,10 +649,30 @@ __global__ __launch_bounds__(kXWaves * 64, 1) void extend_kernel(const ExtendArg
 
   const int item = (int)blockIdx.x / a.hkv;
   const int h = (int)blockIdx.x - item * a.hkv;
-  const int64_t work = cptr(a.items)[item];
-  const int b = (int)(uint32_t)work;
-  if (b < 0) return;
-  const int rt = (int)(work >> 32);
+  int b, rt, piece_first = 0, piece_count = -1, piece_slot = -1;
+  if (a.pieces.shares > 0) {
+    if (a.pieces.list) {
+      const int MA_CONST* e = cptr(reinterpret_cast<const int*>(a.pieces.list + item));
+      b = e[0];
+      rt = e[1];
+      piece_first = e[2];
+      piece_count = e[3];
+      piece_slot = e[4];
+    } else {
+      const ExtendPiece p = plan_direct<kXBM, kXBN>(a, item, h);
+      b = p.seq;
+      rt = p.tile;
+      piece_first = p.first;
+      piece_count = p.count;
+      piece_slot = p.slot;
+    }
+    if (b < 0) return;
+  } else {
+    const int64_t work = cptr(a.items)[item];
+    b = (int)(uint32_t)work;
+    if (b < 0) return;
+    rt = (int)(work >> 32);
+  }
   const QueryRows qr = clamp_query_rows(cptr(a.qsl)[b], cptr(a.qsl)[b + 1], a.num_tokens);
   const int tok0 = qr.tok0;
   const int ntok = qr.ntok;
@@ -357,11 +715,12 @@ __global__ __launch_bounds__(kXWaves * 64, 1) void extend_kernel(const ExtendArg
   const int t_first = r0 / a.group;
   const int t_last = min(ntok - 1, (r0 + kXBM - 1) / a.group);
   const KeyRange keys = row_tile_keys(r0, kXBM, ntok, a.group, prefix, seq, a.causal, a.window);
-  const int key_lo = keys.lo;
+  const int key_lo = keys.lo + piece_first * kXBN;
   const int key_hi = keys.hi;
   const int full_lo = a.window >= 0 ? max(0, prefix + t_last - a.window) : 0;
   const int full_hi = a.causal ? min(seq, prefix + t_first + 1) : seq;
-  const int ntiles = key_hi > key_lo ? (key_hi - key_lo + kXBN - 1) / kXBN : 0;
+  const int rest = key_hi > key_lo ? (key_hi - key_lo + kXBN - 1) / kXBN : 0;
+  const int ntiles = piece_count >= 0 ? min(piece_count, rest) : rest;
 
   float m_run[kXRB];
   f32x4 o[kXRB][DB];
@@ -674,6 +1033,17 @@ __global__ __launch_bounds__(kXWaves * 64, 1) void extend_kernel(const ExtendArg
     const int r = r0 + wave * (kXRB * 16) + rb * 16 + c;
     const int t = r / a.group;
     const int g = r - t * a.group;
+    if (piece_slot >= 0) {  // one piece of several: normalised O and log2 LSE for the merge
+      const int64_t prow = ((int64_t)piece_slot * a.hkv + h) * kXBM + wave * (kXRB * 16) + rb * 16 + c;
+      const float pinv = (lt > 0.f) ? 1.f / lt : 0.f;
+      float MA_GLOBAL* po = gptr_mut(a.pieces.o) + prow * D + 4 * j;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+        if (!PAD || db * 16 + 4 * j < a.head_dim) *reinterpret_cast<f32x4 MA_GLOBAL*>(po + db * 16) = o[rb][db] * pinv;
+      if (j == 0)
+        gptr_mut(a.pieces.lse)[prow] = (lt > 0.f) ? __builtin_amdgcn_logf(lt) + m_run[rb] * a.scale_log2 : -INFINITY;
+      continue;
+    }
     const float inv = (lt > 0.f) ? a.v_scale / lt : 0.f;
     const int64_t off = (int64_t)(tok0 + t) * a.out_stride_tok + (int64_t)(h * a.group + g) * a.out_stride_head;
 #pragma unroll
@@ -681,6 +1051,63 @@ __global__ __launch_bounds__(kXWaves * 64, 1) void extend_kernel(const ExtendArg
       if (!PAD || db * 16 + 4 * j < a.head_dim)
         store_out4<QBF16>(a.out, off + db * 16 + 4 * j, o[rb][db], inv, a.out_f32);
   }
+}
+
+// Merge of the row tiles that were cut into key pieces: 1024 / D rows of one tile and kv
+// head per workgroup, D / 4 threads per row, four dims each. A running maximum of the log2
+// LSEs rescales the sum of the pieces' normalised O, so one pass reads each piece once
+// (four pieces' loads in flight). Pieces in which a row saw no key (LSE -inf) weigh 0.
+
+template <int D, bool QBF16>
+__global__ __launch_bounds__(256) void extend_merge(const ExtendArgs args) {
+  const ExtendArgs a = args;
+  constexpr int kBM = XShape<D>::BM;
+  constexpr int kTPR = D / 4;              // threads per row
+  constexpr int kRows = 256 / kTPR;        // rows per workgroup
+  constexpr int kBlocks = kBM / kRows;     // workgroups per row tile and kv head
+  const int blk = (int)blockIdx.x % kBlocks;
+  const int rest = (int)blockIdx.x / kBlocks;
+  const int h = rest % a.hkv;
+  const int MA_CONST* e = cptr(reinterpret_cast<const int*>(a.pieces.merges + rest / a.hkv));
+  const int b = e[0];
+  if (b < 0) return;
+  const int rt = e[1], slot = e[2], parts = e[3];
+  const QueryRows qr = clamp_query_rows(cptr(a.qsl)[b], cptr(a.qsl)[b + 1], a.num_tokens);
+  const int d = ((int)threadIdx.x % kTPR) * 4;
+  const int r = blk * kRows + (int)threadIdx.x / kTPR;
+  const int R = rt * kBM + r;
+  const int t = R / a.group;
+  const int g = R - t * a.group;
+  if (d >= a.head_dim || t >= qr.ntok) return;
+  const int64_t pitch = (int64_t)a.hkv * kBM;  // rows of one slot
+  const int64_t row0 = ((int64_t)slot * a.hkv + h) * kBM + r;
+  const float MA_GLOBAL* lse = gptr(a.pieces.lse) + row0;
+  const float MA_GLOBAL* po = gptr(a.pieces.o) + row0 * D + d;
+  float m = -INFINITY, w = 0.f;
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int p = 0; p < parts; ++p) {
+    const float l = lse[p * pitch];
+    const f32x4 o = *reinterpret_cast<const f32x4 MA_GLOBAL*>(po + p * pitch * D);
+    const float m_new = fmaxf(m, l);
+    const float base = (m_new == -INFINITY) ? 0.f : m_new;
+    const float s_old = __builtin_amdgcn_exp2f(m - base);
+    const float s_new = __builtin_amdgcn_exp2f(l - base);
+    acc = acc * s_old + o * s_new;
+    w = w * s_old + s_new;
+    m = m_new;
+  }
+  const float inv = (w > 0.f) ? a.v_scale / w : 0.f;
+  const int64_t off = (int64_t)(qr.tok0 + t) * a.out_stride_tok + (int64_t)(h * a.group + g) * a.out_stride_head + d;
+  store_out4<QBF16>(a.out, off, acc, inv, a.out_f32);
+}
+
+template <int D>
+static hipError_t launch_merge_d(bool qbf16, int merges, hipStream_t st, const ExtendArgs& a) {
+  const dim3 grid((unsigned)(merges * a.hkv * (XShape<D>::BM * D / 1024)));
+  if (qbf16) hipLaunchKernelGGL((extend_merge<D, true>), grid, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((extend_merge<D, false>), grid, dim3(256), 0, st, a);
+  return hipGetLastError();
 }
 
 template <int D, bool QBF16, int HD>
@@ -741,6 +1168,60 @@ extern "C" size_t ma_extend_workspace_bytes(int64_t num_tokens, int num_q_heads,
   return ((size_t)n * sizeof(int64_t) + 255) & ~(size_t)255;
 }
 
+// Compute units of the current device, read once per device.
+static int compute_units() {
+  constexpr int kMaxDevices = 64;
+  static std::atomic<int> cus[kMaxDevices];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+  int n = cus[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    cus[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
+// Key pieces of a call: sizes and offsets in the workspace (whose first `list` bytes are the
+// work list of whole row tiles); shares 0 when the call has too many row tiles for them.
+struct PiecePlan {
+  bool direct;  // no plan kernel
+  int shares, slots, capacity, merges;
+  size_t pieces_at, merges_at, lse_at, o_at, bytes;
+};
+static PiecePlan piece_plan(int64_t items, int batch, int hkv, int kdim, size_t list) {
+  PiecePlan p{};
+  p.bytes = list;
+  const int cus = compute_units();
+  if (cus <= 0 || kdim == 0) return p;
+  const int shares = std::max(1, cus / hkv);
+  // `items` counts a partly filled tile per sequence; beyond one round of row tiles the plan
+  // kernel's ordering balances whole tiles within a few percent
+  if (items > kSplitMaxItems || items - batch > shares) return p;
+  p.direct = items <= kDirectItems && batch <= kDirectBatch;
+  const int bm = kdim == 64 ? XShape<64>::BM : kdim == 128 ? XShape<128>::BM : XShape<256>::BM;
+  p.shares = shares;
+  p.slots = std::max((int)items, kSplitSlotRounds * shares);
+  p.capacity = p.direct ? p.slots : (int)items + p.slots;
+  p.merges = p.direct ? (int)items : std::min((int)items, p.slots / 2);
+  auto align = [](size_t x) { return (x + 255) & ~(size_t)255; };
+  p.pieces_at = list;
+  p.merges_at = align(p.pieces_at + (p.direct ? 0 : (size_t)p.capacity * sizeof(ExtendPiece)));
+  p.lse_at = align(p.merges_at + (size_t)p.merges * sizeof(ExtendMerge));
+  p.o_at = align(p.lse_at + (size_t)p.slots * hkv * bm * sizeof(float));
+  p.bytes = align(p.o_at + (size_t)p.slots * hkv * bm * kdim * sizeof(float));
+  return p;
+}
+
+extern "C" size_t ma_extend_split_workspace_bytes(int64_t num_tokens, int num_q_heads, int num_kv_heads, int batch,
+                                                  int head_dim) {
+  const size_t list = ma_extend_workspace_bytes(num_tokens, num_q_heads, num_kv_heads, batch);
+  const int bm = extend_tile_rows(head_dim);
+  if (list == 0 || bm == 0) return list;
+  const int64_t items = extend_items(num_tokens, num_q_heads / num_kv_heads, batch, bm);
+  return piece_plan(items, batch, num_kv_heads, extend_kernel_dim(head_dim), list).bytes;
+}
+
 extern "C" int ma_paged_extend(
     const void* q, int64_t q_stride_tok, int64_t q_stride_head, int q_dtype, int64_t num_tokens,
     const void* k_cache, const void* v_cache, int64_t kv_stride_row, int64_t kv_stride_head, int kv_dtype,
@@ -795,8 +1276,27 @@ extern "C" int ma_paged_extend(
   p.tile_rows = bm;
   p.tile_keys = generic ? kAnyKeys : kdim == 256 ? XShape<256>::BN : XShape<128>::BN;
   p.capacity = (int)items; p.items = reinterpret_cast<int64_t*>(workspace);
-  hipLaunchKernelGGL(extend_plan_kernel, dim3(1), dim3(kPlanThreads), 0, (hipStream_t)stream, p);
-  hipError_t e = hipGetLastError();
+  // key pieces where the batch has few row tiles and the workspace holds their partials
+  PiecePlan pp{};
+  ExtendPieces pieces{};
+  if (!generic) pp = piece_plan(items, batch, num_kv_heads, kdim, need);
+  if (pp.shares > 0 && workspace_bytes >= pp.bytes &&
+      (int64_t)pp.capacity * num_kv_heads <= 0x7fffffff / (kXWaves * 64)) {
+    char* ws = reinterpret_cast<char*>(workspace);
+    p.shares = pp.shares; p.slots = pp.slots; p.capacity = pp.capacity; p.merge_capacity = pp.merges;
+    p.pieces = reinterpret_cast<ExtendPiece*>(ws + pp.pieces_at);
+    p.merges = reinterpret_cast<ExtendMerge*>(ws + pp.merges_at);
+    pieces.list = pp.direct ? nullptr : p.pieces;
+    pieces.merges = p.merges; pieces.merge_capacity = pp.merges;
+    pieces.shares = pp.shares; pieces.capacity = pp.capacity;
+    pieces.lse = reinterpret_cast<float*>(ws + pp.lse_at);
+    pieces.o = reinterpret_cast<float*>(ws + pp.o_at);
+  }
+  hipError_t e = hipSuccess;
+  if (pieces.shares == 0 || pieces.list) {
+    hipLaunchKernelGGL(extend_plan_kernel, dim3(1), dim3(kPlanThreads), 0, (hipStream_t)stream, p);
+    e = hipGetLastError();
+  }
   if (e != hipSuccess) return set_error(MA_ELAUNCH, "extend plan launch failed: %s", hipGetErrorString(e));
   if (generic) {
     AnyArgs g{};
@@ -822,11 +1322,12 @@ extern "C" int ma_paged_extend(
   a.num_tokens = (int)num_tokens;
   a.batch = batch; a.hq = num_q_heads; a.hkv = num_kv_heads; a.group = group;
   a.items = p.items;
+  a.pieces = pieces;
   a.causal = p.causal; a.window = p.window;
   a.scale_log2 = softmax_scale * k_scale * kLog2e; a.v_scale = v_scale;
   a.out = out; a.out_stride_tok = out_stride_tok; a.out_stride_head = out_stride_head;
   a.out_f32 = out_dtype == DT_F32;
-  const dim3 grid((unsigned)(items * num_kv_heads));
+  const dim3 grid((unsigned)((int64_t)p.capacity * num_kv_heads));
   const bool qbf16 = q_dtype == DT_BF16;
   a.head_dim = head_dim;
   a.chunks = head_dim * elt / 16;  // >= 1: head_dim is a multiple of 16
@@ -834,5 +1335,11 @@ extern "C" int ma_paged_extend(
       : kdim == 128 ? launch_extend_d<128>(qbf16, kv_dtype, grid, (hipStream_t)stream, a)
                     : launch_extend_d<256>(qbf16, kv_dtype, grid, (hipStream_t)stream, a);
   if (e != hipSuccess) return set_error(MA_ELAUNCH, "extend launch failed: %s", hipGetErrorString(e));
+  if (pieces.shares > 0) {
+    e = kdim == 64    ? launch_merge_d<64>(qbf16, pp.merges, (hipStream_t)stream, a)
+        : kdim == 128 ? launch_merge_d<128>(qbf16, pp.merges, (hipStream_t)stream, a)
+                      : launch_merge_d<256>(qbf16, pp.merges, (hipStream_t)stream, a);
+    if (e != hipSuccess) return set_error(MA_ELAUNCH, "extend merge launch failed: %s", hipGetErrorString(e));
+  }
   return MA_OK;
 }
