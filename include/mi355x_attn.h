@@ -174,7 +174,7 @@ int ma_paged_verify(const void* q, int64_t q_stride_tok, int64_t q_stride_head, 
 /*
  * Bytes of workspace ma_paged_extend needs for `num_tokens` query tokens in `batch`
  * sequences: the work list, one 8-byte entry per row tile. Row tiles have 256 rows at
- * head_dim 64 and 128 and 128 rows at 256; the size covers the smaller tile (at most
+ * head_dim up to 128 and 128 rows above; the size covers the smaller tile (at most
  * ceil(num_tokens * G / 128) + batch entries, G = num_q_heads / num_kv_heads), so one
  * workspace serves every head dim. 0 for bad arguments.
  */

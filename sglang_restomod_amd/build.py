@@ -51,7 +51,7 @@ def common_flags() -> list[str]:
 # between the two register files on every key tile (hundreds to thousands of
 # v_accvgpr moves per kernel).
 _VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
-SOURCE_FLAGS = {"paged_any": _VGPR_FORM, "splitkv": _VGPR_FORM}
+SOURCE_FLAGS = {"paged_any": _VGPR_FORM, "splitkv": _VGPR_FORM, "extend_wide": _VGPR_FORM}
 
 
 def _flags(src: Path, extra: list[str]) -> list[str]:

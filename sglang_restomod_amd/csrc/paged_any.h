@@ -1,6 +1,5 @@
-// Paged attention for the head dims the tuned kernels do not take (every multiple of 16
-// from 16 to 512 other than 64, 128 and 256): one kernel for decode, linear verify and
-// extend rows. Shared by the decode/verify and extend entry points.
+// Paged decode and linear verify for the head dims the tuned kernels do not take (every
+// multiple of 16 from 16 to 512 other than 64, 128 and 256), and for small decodes.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -13,7 +12,6 @@ namespace ma {
 constexpr int kAnyWaves = 4;        // waves per workgroup
 constexpr int kAnyRows = 16;        // query rows per wave
 constexpr int kAnyKeys = 16;        // keys per tile
-constexpr int kAnyPlanRows = 128;   // rows of one work-list entry (the extend plan's smallest tile)
 constexpr int kAnyMaxDim = 512;
 
 struct AnyArgs {
@@ -30,8 +28,7 @@ struct AnyArgs {
   int num_tokens;            // rows of q and out: query rows are clamped into [0, num_tokens)
   int batch, hq, hkv, group;
   int head_dim;              // D: the kernel's width is the next of 64, 128, 256, 512
-  const int64_t* items;      // work list of 128-row tiles (extend), or null: workgroup
-  int row_blocks;            //   item -> (kv head, key piece, 16-row block of row_blocks, sequence)
+  int row_blocks;            // workgroup -> (kv head, key piece, 16-row block of row_blocks, sequence)
   int pieces;                // decode: workgroups per row block, each over a contiguous piece of
                              //   the keys (1: one workgroup takes them all)
   float* part_o;             // pieces > 1: each piece's normalised O, [slot][16 rows][DP] fp32,
@@ -49,7 +46,7 @@ inline bool any_head_dim(int d) {
   return d >= 16 && d <= kAnyMaxDim && d % 16 == 0 && d != 64 && d != 128 && d != 256;
 }
 
-// Launch on `a` (validated by the caller, items already planned when set); returns the
+// Launch on `a` (validated by the caller); returns the
 // launch status. q_dtype DT_F16/DT_BF16, kv_dtype the same or fp8. With pieces > 1 (decode
 // only) the grid is row-block items x pieces and a merge kernel follows.
 hipError_t any_launch(const AnyArgs& a, int q_dtype, int kv_dtype, int64_t work_items, hipStream_t stream);

@@ -1,24 +1,20 @@
-// Paged attention at the head dims the tuned kernels do not take: every multiple of 16
-// from 16 to 512 other than 64, 128 and 256 (the reference's paged kernels take any head
-// dim, with a default tile configuration and a tuned one for 512:
+// Paged decode and linear verify at the head dims the tuned kernels do not take: every
+// multiple of 16 from 16 to 512 other than 64, 128 and 256 (the reference's paged kernels
+// take any head dim, with a default tile configuration and a tuned one for 512:
 // sglang_restomod/attention/v100/tilelang/_kernels_paged.py:397-418; above 256 its linear
-// verify also runs on the ordinary paged kernel, _paged_adapter.py:612-616).
+// verify also runs on the ordinary paged kernel, _paged_adapter.py:612-616), and small
+// decodes at every head dim.
 //
-// One kernel family serves decode, linear verify and extend rows. A wave computes the
-// scores of 16 query rows (token, GQA head) of one sequence and kv head, 16 keys at a
-// time:
+// A wave computes the scores of 16 query rows (token, GQA head) of one sequence and kv
+// head, 16 keys at a time:
 //   - scores S^T = K Q^T on 16x16x32 MFMAs (the query's 16-bit type; fp8 K converted),
 //     so each lane holds four keys of one row: the B operand of the 16x16x16 fp16 MFMA
 //     of O^T += V^T P^T, whose A operand is read transposed (ds_read_b64_tr_b16) from
 //     fp16 V rows in LDS,
 //   - an online softmax with the tuned kernels' lazy rescale (kLazyRescale).
-// Decode and verify (no work list): the four waves of a workgroup hold the same 16 rows
-// and take a quarter of their 16-key tiles each, K straight into operand registers and V
-// through the wave's own LDS rows, then merge through LDS. Extend (the work list, its own
-// instantiation): the four waves hold 64 consecutive rows and share each K/V tile (32
-// keys up to 128 dims, else 16) through a three-stage LDS ring; each wave publishes its
-// rows' P and accumulates O for a quarter of the dims of all 64 rows, one barrier per
-// tile.
+// The four waves of a workgroup hold the same 16 rows and take a quarter of their 16-key
+// tiles each, K straight into operand registers and V through the wave's own LDS rows,
+// then merge through LDS.
 // The kernel is as wide as the next of 64, 128, 256 and 512: lanes past the head dim
 // read the row's last dims again (every load is unconditional), which meet Q's zeros in
 // the scores and fill output dims that are never stored.
@@ -40,26 +36,20 @@ struct AnyVRaw<true> {
   typedef u32x2 type;
 };
 
-// the mode of one call of the row routine, fixed at compile time
-template <bool SHARED>
-struct AnyMode {
-  static constexpr bool shared = SHARED;
-};
 // a register buffer index, fixed at compile time
 template <int N>
 struct AnyIdx {
   static constexpr int v = N;
 };
 
-// SHARED: the extend kernel (work list, shared K/V ring); otherwise decode and verify
-// (split keys). Two workgroups share a CU where the registers allow it.
-template <bool SHARED, int DP>
+// Two workgroups share a CU where the registers allow it.
+template <int DP>
 constexpr int any_wg_per_cu() {
-  return (DP >= 512 || (DP >= 256 && !SHARED)) ? 1 : 2;
+  return DP >= 256 ? 1 : 2;
 }
 
-template <int DP, bool QBF16, int KV, bool SHARED>
-__global__ __launch_bounds__(kAnyWaves * 64, (any_wg_per_cu<SHARED, DP>())) void any_kernel(const AnyArgs args) {
+template <int DP, bool QBF16, int KV>
+__global__ __launch_bounds__(kAnyWaves * 64, any_wg_per_cu<DP>()) void any_kernel(const AnyArgs args) {
   const AnyArgs a = args;  // local copy: the lambdas capture by reference
   constexpr bool kFp8 = (KV == DT_E4M3 || KV == DT_E5M2);
   constexpr int KK = DP / 32;                   // QK MFMA steps
@@ -76,38 +66,13 @@ __global__ __launch_bounds__(kAnyWaves * 64, (any_wg_per_cu<SHARED, DP>())) void
 
   // Decode and verify at the widest head dim with fp16 Q and KV keep Q in LDS (rows padded
   // by 16 bytes so the 16 rows of an operand read fall in different banks): in registers
-  // it spilled. bf16 and fp8 KV, and extend, keep Q in registers (1-3% faster at D=320
-  // and 512 than reading it from LDS every tile).
+  // it spilled. bf16 and fp8 KV keep Q in registers (1-3% faster at D=320 and 512 than
+  // reading it from LDS every tile).
   constexpr bool kQLds = DP >= 512 && !kFp8 && !QBF16;
   constexpr int kQRow = DP * 2 + 16;
   constexpr int kVBlock = kAnyKeys * kRowL;            // one wave's V rows
   constexpr int kQBlock = kQLds ? kAnyRows * kQRow : 0;  // one wave's Q rows
-  // Extend rows: the four waves own 64 consecutive rows of one sequence and kv head and
-  // share every K/V tile (kKT keys: 32 up to 128 dims, else 16) through a three-stage LDS
-  // ring (16-bit K rows padded by 32 bytes, V rows padded as above: fp16, or bf16 that
-  // becomes fp16 as its fragments are read), loaded once per workgroup; kUW 16-byte
-  // units per thread. Each wave computes the scores and softmax of its own 16 rows, and
-  // O for a quarter of the dims (kCB 16-dim blocks) of all 64 rows: P, the rescale
-  // factors and their flags pass through the exchange memory behind the ring (two tiles
-  // deep). Decode and verify tiles have 16 keys.
-  constexpr int kKT = (SHARED && DP <= 128) ? 2 * kAnyKeys : kAnyKeys;
-  constexpr int kNS = kKT / kAnyKeys;  // 16-key score blocks per tile
-  // K row pitch: 32 bytes of padding. With 16, the score reads of the D = 512 extend batch
-  // took 139 million bank-conflict cycles per launch (a quarter of the LDS's active
-  // cycles); with 32, none, and the kernel ran 3.7% faster.
-  constexpr int kRowK = DP * 2 + 32;
-  constexpr int kKTile = kKT * kRowK;
-  constexpr int kStageB = kKTile + kKT * kRowL;
-  constexpr int kTileUnits = kKT * kUnits;  // 16-byte units of one K (or V) tile
-  constexpr int kUW = kTileUnits >= kAnyWaves * 64 ? kTileUnits / (kAnyWaves * 64) : 1;
-  constexpr int kCB = DB / kAnyWaves;
-  static_assert(kCB >= 1 && DB % kAnyWaves == 0, "whole dim blocks per wave");
-  constexpr int kXP = 0;                                   // P: [tile & 1][wave][block][lane] u32x2
-  constexpr int kXA = kXP + 2 * kAnyWaves * kNS * 64 * 8;  // factors: [tile & 1][wave][row] f32
-  constexpr int kXF = kXA + 2 * kAnyWaves * kAnyRows * 4;  // flags: [tile & 1][wave] u32
-  constexpr int kXBytes = kXF + 2 * kAnyWaves * 4;
-  constexpr int kRing = 3 * kStageB;
-  constexpr int kSmem = SHARED ? kRing + kXBytes : kAnyWaves * (kVBlock + kQBlock);
+  constexpr int kSmem = kAnyWaves * (kVBlock + kQBlock);
   // When the four waves split one row block's keys, their partial O meet in the same
   // memory after the loop, kBPR 16-column blocks (1 KiB per wave each) at a time.
   constexpr int kBPR = (DB * kAnyWaves * 1024 <= kSmem) ? DB
@@ -138,14 +103,9 @@ __global__ __launch_bounds__(kAnyWaves * 64, (any_wg_per_cu<SHARED, DP>())) void
   const uint32_t row_bytes32 = (uint32_t)(a.kv_stride_row * kElt);  // the hosts check it fits
   const int page_mask = (1 << a.tt.page_shift) - 1;
 
-  // One wave's 16 rows r0 .. r0 + 15 of sequence b, kv head h. Shared mode: the
-  // workgroup's four waves own consecutive row blocks (rows r0 - 16 * wave ..) and walk the
-  // keys any of them sees together, sharing each K/V tile. Otherwise the four waves own the
-  // same row block and take quarter `split` of its key tiles each, merging at the end.
-  auto rows = [&](auto mode, int b, int h, int r0, int split) __attribute__((always_inline)) {
-    constexpr bool shared = decltype(mode)::shared;
-    const int rg0 = shared ? r0 - wave * kAnyRows : r0;  // first row of the workgroup's rows
-    const int rgn = shared ? kAnyWaves * kAnyRows : kAnyRows;
+  // The 16 rows r0 .. r0 + 15 of sequence b, kv head h: the four waves take quarter `split`
+  // of their key tiles each, merging at the end.
+  auto rows = [&](int b, int h, int r0, int split) __attribute__((always_inline)) {
     int tok0, ntok;
     if (a.qsl) {
       const QueryRows qr = clamp_query_rows(cptr(a.qsl)[b], cptr(a.qsl)[b + 1], a.num_tokens);
@@ -155,7 +115,7 @@ __global__ __launch_bounds__(kAnyWaves * 64, (any_wg_per_cu<SHARED, DP>())) void
       tok0 = b;
       ntok = b < a.num_tokens ? 1 : 0;
     }
-    if (rg0 >= ntok * G) return;  // the same for every wave of the workgroup
+    if (r0 >= ntok * G) return;  // the same for every wave of the workgroup
     const int seq = max(cptr(a.seq_lens)[b], 0);
     const int prefix = a.prefix ? cptr(a.prefix)[b] : seq - ntok;
     const int64_t seq_row = a.row_index ? cptr(a.row_index)[b] : (int64_t)b;
@@ -169,8 +129,7 @@ __global__ __launch_bounds__(kAnyWaves * 64, (any_wg_per_cu<SHARED, DP>())) void
     const int qpos = prefix + t;
     const int lo_r = (real && a.window >= 0) ? max(0, qpos - a.window) : 0;
     const int hi_r = real ? (a.causal ? min(seq, qpos + 1) : seq) : 0;
-    constexpr bool kQInLds = kQLds && !shared;  // shared mode keeps Q in registers
-    u32x4 qv[kQInLds ? 1 : KK];
+    u32x4 qv[kQLds ? 1 : KK];
     const uint32_t qa = q_base + c * kQRow + j * 16;
     {
       const uint16_t MA_GLOBAL* qp = gptr(reinterpret_cast<const uint16_t*>(a.q)) +
@@ -178,22 +137,22 @@ __global__ __launch_bounds__(kAnyWaves * 64, (any_wg_per_cu<SHARED, DP>())) void
                                      (int64_t)(h * G + g) * a.q_stride_head;
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) {
-        const int d0 = shared ? kk * 32 + j * 8 : qdim(kk);
+        const int d0 = qdim(kk);
         const u32x4 qf = (real && d0 < D) ? *reinterpret_cast<const u32x4 MA_GLOBAL*>(qp + d0) : u32x4{0, 0, 0, 0};
-        if constexpr (kQInLds) *reinterpret_cast<__attribute__((address_space(3))) u32x4*>((uintptr_t)(qa + kk * 64)) = qf;
+        if constexpr (kQLds) *reinterpret_cast<__attribute__((address_space(3))) u32x4*>((uintptr_t)(qa + kk * 64)) = qf;
         else qv[kk] = qf;
       }
     }
-    // keys any of the rows (the wave's, or the workgroup's in shared mode) may see
-    const int t_first = rg0 / G;
-    const int t_last = min(ntok - 1, (rg0 + rgn - 1) / G);
+    // keys any of the rows may see
+    const int t_first = r0 / G;
+    const int t_last = min(ntok - 1, (r0 + kAnyRows - 1) / G);
     const int key_lo = a.window >= 0 ? max(0, prefix + t_first - a.window) : 0;
     const int key_hi = a.causal ? min(seq, prefix + t_last + 1) : seq;
-    const int nt = key_hi > key_lo ? (key_hi - key_lo + kKT - 1) / kKT : 0;
+    const int nt = key_hi > key_lo ? (key_hi - key_lo + kAnyKeys - 1) / kAnyKeys : 0;
     // split: this wave's quarter of the workgroup's key piece (pieces x 4 equal shares)
     const int parts = kAnyWaves * a.pieces;
-    const int i_lo = shared ? 0 : (int)((int64_t)split * nt / parts);
-    const int i_hi = shared ? nt : (int)((int64_t)(split + 1) * nt / parts);
+    const int i_lo = (int)((int64_t)split * nt / parts);
+    const int i_hi = (int)((int64_t)(split + 1) * nt / parts);
 
     float m_run = -INFINITY;
     float lsum = 0.f;  // this lane's share of its row's sum of p (keys 4j .. 4j + 3 of each tile)
@@ -201,9 +160,9 @@ __global__ __launch_bounds__(kAnyWaves * 64, (any_wg_per_cu<SHARED, DP>())) void
 #pragma unroll
     for (int db = 0; db < DB; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // lane l holds tile i's key l % kKT: its page, then its slot
+    // lane l holds tile i's key l % kAnyKeys: its page, then its slot
     auto key_pos = [&](int i) __attribute__((always_inline)) -> int {
-      return min(key_lo + i * kKT + (lane & (kKT - 1)), key_hi - 1);
+      return min(key_lo + i * kAnyKeys + (lane & (kAnyKeys - 1)), key_hi - 1);
     };
     auto page_load = [&](int i) __attribute__((always_inline)) -> int {
       return gptr(a.tt.table)[seq_row * a.tt.stride + (key_pos(i) >> a.tt.page_shift)];
@@ -268,7 +227,7 @@ __global__ __launch_bounds__(kAnyWaves * 64, (any_wg_per_cu<SHARED, DP>())) void
       } else {
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
-          if constexpr (kQInLds) {
+          if constexpr (kQLds) {
             const u32x4 qf = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>((uintptr_t)(qa + kk * 64));
             s = mfma16t<QBF16>(kr[kk], qf, s);
           } else
@@ -277,47 +236,16 @@ __global__ __launch_bounds__(kAnyWaves * 64, (any_wg_per_cu<SHARED, DP>())) void
       }
       return s;
     };
-    // scores of tile i from a K tile in LDS (shared mode, Q in registers)
-    // The operand reads run one batch of kFB steps ahead of the MFMAs; the scheduling
-    // barriers keep the compiler from sinking each read down to its MFMA, which left every
-    // MFMA waiting out a full LDS latency.
-    auto scores_lds = [&](uint32_t kt) __attribute__((always_inline)) -> f32x4 {
-      f32x4 s2[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};  // two MFMA chains
-      const uint32_t ka0 = kt + c * kRowK + j * 16;
-      constexpr int kFB = KK < 4 ? KK : 4;  // QK steps per batch
-      constexpr int kNB = KK / kFB;
-      u32x4 kf[2][kFB];
-      auto fetch = [&](int bb, int sl) __attribute__((always_inline)) {
+    // Online softmax of tile i's scores (lane (c, j): keys 4j .. 4j + 3 of row c). Gives p in
+    // fp16; `moved` (the same in every lane) says whether some row's exponent base moved, and
+    // then `alpha` is the factor the row's earlier O takes (1 for the others). The base moves
+    // only when a row's max grew by more than 2^kLazyRescale in p.
+    auto softmax = [&](int i, f32x4& s, u32x2& pk, float& alpha, bool& moved) __attribute__((always_inline)) {
+      const int kb0 = key_lo + i * kAnyKeys + 4 * j;
 #pragma unroll
-        for (int x = 0; x < kFB; ++x)
-          kf[sl][x] = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>((uintptr_t)(ka0 + (bb * kFB + x) * 64));
-      };
-      fetch(0, 0);
-#pragma unroll
-      for (int bb = 0; bb < kNB; ++bb) {
-        if (bb + 1 < kNB) fetch(bb + 1, (bb + 1) & 1);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int x = 0; x < kFB; ++x) s2[x & 1] = mfma16t<QBF16>(kf[bb & 1][x], qv[bb * kFB + x], s2[x & 1]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      return s2[0] + s2[1];
-    };
-    // Online softmax of tile i's scores, kNS blocks of 16 keys (lane (c, j): keys
-    // 16 sb + 4j .. + 3 of row c in block sb). Writes p in fp16; `moved` (the same in
-    // every lane) says whether some row's exponent base moved, and then `alpha` is the
-    // factor the row's earlier O takes (1 for the others). The base moves only when a
-    // row's max grew by more than 2^kLazyRescale in p.
-    auto softmax = [&](int i, f32x4 (&s)[kNS], u32x2 (&pk)[kNS], float& alpha, bool& moved) __attribute__((always_inline)) {
-      float mx = -INFINITY;
-#pragma unroll
-      for (int sb = 0; sb < kNS; ++sb) {
-        const int kb0 = key_lo + i * kKT + sb * kAnyKeys + 4 * j;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (kb0 + e < lo_r || kb0 + e >= hi_r) s[sb][e] = -INFINITY;
-        mx = fmaxf(mx, fmaxf(fmaxf(s[sb][0], s[sb][1]), fmaxf(s[sb][2], s[sb][3])));
-      }
+      for (int e = 0; e < 4; ++e)
+        if (kb0 + e < lo_r || kb0 + e >= hi_r) s[e] = -INFINITY;
+      float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
       alpha = 1.f;
       moved = __builtin_amdgcn_ballot_w64((mx - m_run) * a.scale_log2 > kLazyRescale) != 0;
       if (moved) {
@@ -330,23 +258,18 @@ __global__ __launch_bounds__(kAnyWaves * 64, (any_wg_per_cu<SHARED, DP>())) void
         lsum *= alpha;
       }
       const float msc = (m_run == -INFINITY ? 0.f : m_run) * a.scale_log2;
+      float p[4];
 #pragma unroll
-      for (int sb = 0; sb < kNS; ++sb) {
-        float p[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) p[e] = __builtin_amdgcn_exp2f(s[sb][e] * a.scale_log2 - msc);
-        lsum += (p[0] + p[1]) + (p[2] + p[3]);
-        pk[sb] = u32x2{pack_f16(p[0], p[1]), pack_f16(p[2], p[3])};
-      }
+      for (int e = 0; e < 4; ++e) p[e] = __builtin_amdgcn_exp2f(s[e] * a.scale_log2 - msc);
+      lsum += (p[0] + p[1]) + (p[2] + p[3]);
+      pk = u32x2{pack_f16(p[0], p[1]), pack_f16(p[2], p[3])};
     };
-    // softmax and PV of tile i in split mode (its V in this wave's LDS rows at vt)
+    // softmax and PV of tile i (its V in this wave's LDS rows at vt)
     auto finish = [&](int i, f32x4 s, uint32_t vt) __attribute__((always_inline)) {
       float alpha;
       bool moved;
-      f32x4 sa[kNS] = {s};
-      u32x2 pka[kNS];
-      softmax(i, sa, pka, alpha, moved);
-      const u32x2 pk = pka[0];
+      u32x2 pk;
+      softmax(i, s, pk, alpha, moved);
       if (moved) {
 #pragma unroll
         for (int db = 0; db < DB; ++db) o[db] *= alpha;
@@ -376,170 +299,7 @@ __global__ __launch_bounds__(kAnyWaves * 64, (any_wg_per_cu<SHARED, DP>())) void
       }
     };
 
-    // LDS words of the shared mode's exchange memory
-    const uint32_t xbase = smem_base + kRing;
-    auto xp = [&](int i, int w, int sb) -> uint32_t { return xbase + kXP + (((i & 1) * kAnyWaves + w) * kNS + sb) * 512; };
-    auto xa = [&](int i, int w) -> uint32_t { return xbase + kXA + ((i & 1) * kAnyWaves + w) * (kAnyRows * 4); };
-    auto xf = [&](int i) -> uint32_t { return xbase + kXF + (i & 1) * (kAnyWaves * 4); };
-    if (shared && nt > 0) {
-      // The workgroup's tile ring. Step i writes tile i+1 (its units loaded kRB steps
-      // earlier) to stage (i+1) % 3, loads tile i+kRB+1, computes the scores and softmax
-      // of tile i from stage i % 3 and publishes P, then meets the other waves, then
-      // accumulates PV for its dims from every wave's P. The barrier of step i publishes
-      // stage (i+1) % 3 and tile i's P; stage (i+2) % 3, which step i+1 writes, was last
-      // read before the barrier of step i-1, and so were the exchange words of tile i-2.
-      // Tiles past the last are the last again (key positions clamp), every load is
-      // unconditional.
-      // tile t's raw units live in register buffer t % kRB from the step that loads them
-      // (t - kRB - 1) to the step that writes them to LDS (t - 1): kRB tiles' compute to
-      // land in (three at the widest head dim, where one wave per SIMD leaves the registers)
-      constexpr int kRB = DP >= 512 ? 3 : 2;
-      u32x4 kraw[kRB][kUW];
-      VRaw vraw[kRB][kUW];
-      auto load_units = [&](int myslot, u32x4 (&kraw)[kUW], VRaw (&vraw)[kUW]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int x = 0; x < kUW; ++x) {
-          const int u = min((int)threadIdx.x + kAnyWaves * 64 * x, kTileUnits - 1);
-          const int key = u / kUnits;
-          const int q = min(u - key * kUnits, D / 8 - 1);
-          const int64_t off = (int64_t)((uint64_t)(uint32_t)shfl_i(myslot, key) * row_bytes32) + head_off + q * 8 * kElt;
-          if constexpr (kFp8) {
-            const u32x2 w = *reinterpret_cast<const u32x2 MA_GLOBAL*>(kbase + off);
-            kraw[x] = u32x4{w[0], w[1], 0u, 0u};
-          } else {
-            kraw[x] = *reinterpret_cast<const u32x4 MA_GLOBAL*>(kbase + off);
-          }
-          vraw[x] = *reinterpret_cast<const VRaw MA_GLOBAL*>(vbase + off);
-        }
-      };
-      auto write_units = [&](uint32_t st, const u32x4 (&kraw)[kUW], const VRaw (&vraw)[kUW]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int x = 0; x < kUW; ++x) {
-          const int u = (int)threadIdx.x + kAnyWaves * 64 * x;
-          if (kTileUnits % (kAnyWaves * 64) == 0 || u < kTileUnits) {
-            const int key = u / kUnits;
-            const int q = u - key * kUnits;
-            u32x4 kh, vh;
-            if constexpr (kFp8) {
-              kh = cvt8_fp8<KV, QBF16>(kraw[x][0], kraw[x][1]);
-              vh = cvt8_fp8<KV, false>(vraw[x][0], vraw[x][1]);
-            } else {
-              kh = kraw[x];
-              vh = vraw[x];  // bf16 V stays bf16 in LDS: its fragments are converted as read
-            }
-            *reinterpret_cast<__attribute__((address_space(3))) u32x4*>((uintptr_t)(st + key * kRowK + q * 16)) = kh;
-            *reinterpret_cast<__attribute__((address_space(3))) u32x4*>((uintptr_t)(st + kKTile + key * kRowL + q * 16)) = vh;
-          }
-        }
-      };
-      auto stage = [&](int i) -> uint32_t { return smem_base + (uint32_t)(i % 3) * kStageB; };
-      // Page lookups go out two steps before the units that use them: waiting for a lookup
-      // then waits only for loads issued before it, which have had kRB steps to land. The
-      // prologue issues its loads in the steps' order, so the loop starts with the load
-      // counts its back edge brings.
-      int pa = page_load(0);
-      int pb = page_load(1);
-      int pc = page_load(2);
-#pragma unroll
-      for (int t = 0; t < kRB; ++t) {
-        load_units(slot_of(t, pa), kraw[t], vraw[t]);
-        pa = pb;
-        pb = pc;
-        pc = page_load(t + 3);
-      }
-      write_units(stage(0), kraw[0], vraw[0]);
-      load_units(slot_of(kRB, pa), kraw[0], vraw[0]);
-      int pg1 = pb, pg2 = pc;  // the pages of tiles kRB + 1 and kRB + 2
-      __syncthreads();
-      // PV of tile t: the V^T fragments of this wave's kCB dim blocks (stage t % 3) meet
-      // the P fragments of all four row blocks, after the rows whose exponent base moved
-      // have taken their factor
-      auto pv = [&](int t) __attribute__((always_inline)) {
-        const uint32_t vb = stage(t) + kKTile + (4 * j + (c >> 2)) * kRowL + (c & 3) * 8 + wave * kCB * 32;
-        u32x2 vf[kNS][kCB], pf[kNS][kAnyWaves];
-#pragma unroll
-        for (int sb = 0; sb < kNS; ++sb)
-#pragma unroll
-          for (int cb = 0; cb < kCB; ++cb)
-            vf[sb][cb] = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) i16x4*)(uintptr_t)(vb + sb * kAnyKeys * kRowL + cb * 32)));
-        const u32x4 fl = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>((uintptr_t)xf(t));
-#pragma unroll
-        for (int sb = 0; sb < kNS; ++sb)
-#pragma unroll
-          for (int rb = 0; rb < kAnyWaves; ++rb)
-            pf[sb][rb] = *reinterpret_cast<const __attribute__((address_space(3))) u32x2*>((uintptr_t)(xp(t, rb, sb) + lane * 8));
-        if constexpr (QBF16 && !kFp8) {
-          // bf16 V fragments to fp16 (each V element is read by one wave only, so this is
-          // the same conversion count as converting the tile when it is written)
-#pragma unroll
-          for (int sb = 0; sb < kNS; ++sb)
-#pragma unroll
-            for (int cb = 0; cb < kCB; ++cb)
-#pragma unroll
-              for (int w = 0; w < 2; ++w)
-                vf[sb][cb][w] = pack_f16(__builtin_bit_cast(float, vf[sb][cb][w] << 16),
-                                         __builtin_bit_cast(float, vf[sb][cb][w] & 0xffff0000u));
-        }
-#pragma unroll
-        for (int rb = 0; rb < kAnyWaves; ++rb) {
-          if (__builtin_amdgcn_readfirstlane(fl[rb])) {
-            const float al = *reinterpret_cast<const __attribute__((address_space(3))) float*>((uintptr_t)(xa(t, rb) + c * 4));
-#pragma unroll
-            for (int cb = 0; cb < kCB; ++cb) o[rb * kCB + cb] *= al;
-          }
-        }
-#pragma unroll
-        for (int sb = 0; sb < kNS; ++sb)
-#pragma unroll
-          for (int cb = 0; cb < kCB; ++cb)
-#pragma unroll
-            for (int rb = 0; rb < kAnyWaves; ++rb)
-              o[rb * kCB + cb] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, vf[sb][cb]),
-                                                                       __builtin_bit_cast(f16x4, pf[sb][rb]),
-                                                                       o[rb * kCB + cb], 0, 0, 0);
-      };
-      // Step i: the scores of tile i, then PV of tile i-1 (independent work for the MFMA
-      // pipe while the scores land), then tile i's softmax, whose P the barrier publishes.
-      auto tile_step = [&](int i, auto buf_t) __attribute__((always_inline)) {
-        constexpr int cur = decltype(buf_t)::v;  // (i + 1) % kRB
-        write_units(stage(i + 1), kraw[cur], vraw[cur]);  // tile i+1
-        const int pn = page_load(i + kRB + 3);
-        load_units(slot_of(i + kRB + 1, pg1), kraw[cur], vraw[cur]);  // into the buffer just written
-        pg1 = pg2;
-        pg2 = pn;
-        float alpha;
-        bool moved;
-        f32x4 sc[kNS];
-        u32x2 pk[kNS];
-#pragma unroll
-        for (int sb = 0; sb < kNS; ++sb) sc[sb] = scores_lds(stage(i) + sb * kAnyKeys * kRowK);
-        if (i > 0) pv(i - 1);
-        softmax(i, sc, pk, alpha, moved);
-#pragma unroll
-        for (int sb = 0; sb < kNS; ++sb)
-          *reinterpret_cast<__attribute__((address_space(3))) u32x2*>((uintptr_t)(xp(i, wave, sb) + lane * 8)) = pk[sb];
-        if (lane == 0) *reinterpret_cast<__attribute__((address_space(3))) uint32_t*>((uintptr_t)(xf(i) + wave * 4)) = moved;
-        if (moved && j == 0) *reinterpret_cast<__attribute__((address_space(3))) float*>((uintptr_t)(xa(i, wave) + c * 4)) = alpha;
-        __syncthreads();
-      };
-      // the last steps short of a whole round of buffers run after the loop, so the loop's
-      // back edge is its only path to the next pass and the compiler's load counts stay
-      // exact there
-      int i = 0;
-#pragma unroll 1
-      for (; i + kRB - 1 < nt; i += kRB) {
-        tile_step(i, AnyIdx<1 % kRB>{});
-        tile_step(i + 1, AnyIdx<2 % kRB>{});
-        if constexpr (kRB == 3) tile_step(i + 2, AnyIdx<0>{});
-      }
-      if (i < nt) tile_step(i, AnyIdx<1 % kRB>{});
-      if constexpr (kRB == 3) {
-        if (i + 1 < nt) tile_step(i + 1, AnyIdx<2 % kRB>{});
-      }
-      pv(nt - 1);
-    }
-    if (!shared && DP <= 128 && i_hi > i_lo) {
+    if (DP <= 128 && i_hi > i_lo) {
       // Up to 128 dims a tile is small and its compute short, so each wave keeps two tiles
       // in flight: step i issues the slot lookup of tile i+3, writes tile i's V to LDS,
       // loads tile i+2 into the buffers tile i-1 has left, and computes tile i. The
@@ -577,7 +337,7 @@ __global__ __launch_bounds__(kAnyWaves * 64, (any_wg_per_cu<SHARED, DP>())) void
       if (i < i_hi) step3(i, AnyIdx<0>{});
       if (i + 1 < i_hi) step3(i + 1, AnyIdx<1>{});
     }
-    if (!shared && DP > 128 && i_hi > i_lo) {
+    if (DP > 128 && i_hi > i_lo) {
       // Step i issues the slot lookup of tile i+2, writes tile i's V to LDS and refills the
       // V registers with tile i+1, and loads tile i+1's K (into the other K buffer, or at
       // the widest head dims into the same one once tile i's scores have used it), so every
@@ -624,34 +384,6 @@ __global__ __launch_bounds__(kAnyWaves * 64, (any_wg_per_cu<SHARED, DP>())) void
     // normalise and store: row sums first
     float lt = lsum + shfl_xor_f(lsum, 16);
     lt += shfl_xor_f(lt, 32);
-    if constexpr (shared) {
-      // Each row's owner publishes its sum of p (in the factor words of tile nt, whose last
-      // readers were done before the barrier of step nt-1); this wave then stores its dims
-      // of all 64 rows. The second barrier keeps the words until every wave has read them.
-      if (j == 0) *reinterpret_cast<__attribute__((address_space(3))) float*>((uintptr_t)(xa(nt, wave) + c * 4)) = lt;
-      __syncthreads();
-      float ls[kAnyWaves];
-#pragma unroll
-      for (int rb = 0; rb < kAnyWaves; ++rb)
-        ls[rb] = *reinterpret_cast<const __attribute__((address_space(3))) float*>((uintptr_t)(xa(nt, rb) + c * 4));
-      __syncthreads();
-#pragma unroll
-      for (int rb = 0; rb < kAnyWaves; ++rb) {
-        const int rr = rg0 + rb * kAnyRows + c;
-        const int tr = rr / G;
-        if (tr < ntok) {
-          const int gr = rr - tr * G;
-          const int64_t offr = (int64_t)(tok0 + tr) * a.out_stride_tok + (int64_t)(h * G + gr) * a.out_stride_head;
-          const float inv = (ls[rb] > 0.f) ? a.v_scale / ls[rb] : 0.f;
-#pragma unroll
-          for (int cb = 0; cb < kCB; ++cb) {
-            const int d0 = (wave * kCB + cb) * 16;
-            if (d0 < D) store_out4<QBF16>(a.out, offr + d0 + 4 * j, o[rb * kCB + cb], inv, a.out_f32);
-          }
-        }
-      }
-      return;
-    }
     const int64_t off = (int64_t)(tok0 + t) * a.out_stride_tok + (int64_t)(h * G + g) * a.out_stride_head;
     // merge of the four quarters: each O and row sum is relative to its wave's exponent
     // base (its row max, 0 when it saw no key), rescaled to the largest
@@ -707,38 +439,25 @@ __global__ __launch_bounds__(kAnyWaves * 64, (any_wg_per_cu<SHARED, DP>())) void
     }
   };
 
-  if constexpr (SHARED) {
-    // one 128-row work-list entry per workgroup and kv head, in two passes of 64 rows
-    const int entry = (int)blockIdx.x / a.hkv;
-    const int h = (int)blockIdx.x - entry * a.hkv;
-    const int64_t work = cptr(a.items)[entry];
-    const int b = (int)(uint32_t)work;
-    if (b < 0) return;
-    const int rt = (int)(work >> 32);
+  // decode and verify: workgroup = (kv head, key piece, 16-row block, sequence), kv head
+  // fastest; its four waves take the four quarters of its piece of the rows' key tiles.
+  // A sequence with more rows than row_blocks blocks has its later blocks taken in turn
+  // (verify, whose calls have one piece).
+  const int64_t item = blockIdx.x;
+  const int h = (int)(item % a.hkv);
+  const int64_t rest = item / a.hkv;
+  const int piece = (int)(rest % a.pieces);
+  const int64_t blk_item = rest / a.pieces;
+  const int b = (int)(blk_item / a.row_blocks);
+  const int rb = (int)(blk_item - (int64_t)b * a.row_blocks);
+  if (b >= a.batch) return;
+  piece_slot = (blk_item * a.hkv + h) * a.pieces + piece;
+  int rows_b;
+  if (a.qsl) rows_b = clamp_query_rows(cptr(a.qsl)[b], cptr(a.qsl)[b + 1], a.num_tokens).ntok * a.group;
+  else rows_b = (b < a.num_tokens ? 1 : 0) * a.group;
 #pragma unroll 1
-    for (int pass = 0; pass < kAnyPlanRows / (kAnyWaves * kAnyRows); ++pass)
-      rows(AnyMode<true>{}, b, h, rt * kAnyPlanRows + pass * (kAnyWaves * kAnyRows) + wave * kAnyRows, -1);
-  } else {
-    // decode and verify: workgroup = (kv head, key piece, 16-row block, sequence), kv head
-    // fastest; its four waves take the four quarters of its piece of the rows' key tiles.
-    // A sequence with more rows than row_blocks blocks has its later blocks taken in turn
-    // (verify, whose calls have one piece).
-    const int64_t item = blockIdx.x;
-    const int h = (int)(item % a.hkv);
-    const int64_t rest = item / a.hkv;
-    const int piece = (int)(rest % a.pieces);
-    const int64_t blk_item = rest / a.pieces;
-    const int b = (int)(blk_item / a.row_blocks);
-    const int rb = (int)(blk_item - (int64_t)b * a.row_blocks);
-    if (b >= a.batch) return;
-    piece_slot = (blk_item * a.hkv + h) * a.pieces + piece;
-    int rows_b;
-    if (a.qsl) rows_b = clamp_query_rows(cptr(a.qsl)[b], cptr(a.qsl)[b + 1], a.num_tokens).ntok * a.group;
-    else rows_b = (b < a.num_tokens ? 1 : 0) * a.group;
-#pragma unroll 1
-    for (int r0 = rb * kAnyRows; r0 < rows_b; r0 += a.row_blocks * kAnyRows)
-      rows(AnyMode<false>{}, b, h, r0, piece * kAnyWaves + wave);
-  }
+  for (int r0 = rb * kAnyRows; r0 < rows_b; r0 += a.row_blocks * kAnyRows)
+    rows(b, h, r0, piece * kAnyWaves + wave);
 }
 
 // Merge of the key pieces of a decode (pieces > 1): one workgroup per (sequence, 16-row
@@ -834,25 +553,15 @@ __global__ __launch_bounds__(256) void any_merge(const AnyArgs args) {
   }
 }
 
-template <int DP, bool QBF16, bool SHARED>
-static hipError_t launch_any_m(int kv, dim3 grid, hipStream_t st, const AnyArgs& a) {
-  if (kv == DT_E4M3)
-    hipLaunchKernelGGL((any_kernel<DP, QBF16, DT_E4M3, SHARED>), grid, dim3(kAnyWaves * 64), 0, st, a);
-  else if (kv == DT_E5M2)
-    hipLaunchKernelGGL((any_kernel<DP, QBF16, DT_E5M2, SHARED>), grid, dim3(kAnyWaves * 64), 0, st, a);
-  else
-    hipLaunchKernelGGL((any_kernel<DP, QBF16, QBF16 ? DT_BF16 : DT_F16, SHARED>), grid, dim3(kAnyWaves * 64), 0, st, a);
-  return hipGetLastError();
-}
-
 template <int DP, bool QBF16>
 static hipError_t launch_any_q(int kv, dim3 grid, hipStream_t st, const AnyArgs& a) {
-  // extend rows reach this kernel above 256 dims only (the tiled extend kernels take the rest)
-  if (a.items) {
-    if constexpr (DP == 512) return launch_any_m<DP, QBF16, true>(kv, grid, st, a);
-    else return hipErrorInvalidValue;
-  }
-  return launch_any_m<DP, QBF16, false>(kv, grid, st, a);
+  if (kv == DT_E4M3)
+    hipLaunchKernelGGL((any_kernel<DP, QBF16, DT_E4M3>), grid, dim3(kAnyWaves * 64), 0, st, a);
+  else if (kv == DT_E5M2)
+    hipLaunchKernelGGL((any_kernel<DP, QBF16, DT_E5M2>), grid, dim3(kAnyWaves * 64), 0, st, a);
+  else
+    hipLaunchKernelGGL((any_kernel<DP, QBF16, QBF16 ? DT_BF16 : DT_F16>), grid, dim3(kAnyWaves * 64), 0, st, a);
+  return hipGetLastError();
 }
 
 template <int DP>

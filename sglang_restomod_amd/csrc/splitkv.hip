@@ -1095,7 +1095,7 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
     g.k = a.k; g.v = a.v; g.kv_stride_row = a.kv_stride_row; g.kv_stride_head = a.kv_stride_head;
     g.tt = a.tt; g.row_index = a.row_index; g.seq_lens = a.seq_lens; g.qsl = a.qsl; g.prefix = a.prefix;
     g.num_tokens = a.num_tokens; g.batch = a.batch; g.hq = a.hq; g.hkv = a.hkv; g.group = a.group;
-    g.head_dim = head_dim; g.items = nullptr;
+    g.head_dim = head_dim;
     g.row_blocks = (int)(((int64_t)max_q_per_seq * a.group + kAnyRows - 1) / kAnyRows);
     g.causal = a.causal; g.window = a.window; g.scale_log2 = a.scale_log2; g.v_scale = a.v_scale;
     g.out = a.out; g.out_stride_tok = a.out_stride_tok; g.out_stride_head = a.out_stride_head; g.out_f32 = a.out_f32;

@@ -66,6 +66,11 @@ CASES = [  # prefix, ext, heads, kv heads, dim, q dtype, kv dtype, causal, windo
     ([2500, 10], [40, 90], 32, 8, 96, BF16, E4M3, True, -1),   # padded head dims
     ([2500], [40], 16, 4, 192, F16, F16, True, -1),
     ([1700], [25], 16, 4, 48, BF16, BF16, True, -1),
+    ([1500, 0, 31], [70, 0, 200], 16, 4, 512, BF16, BF16, True, -1),  # the wide kernel
+    ([900], [33], 16, 4, 512, F16, F16, True, 100),
+    ([900, 64], [40, 97], 8, 2, 512, BF16, E4M3, False, -1),
+    ([700], [50], 8, 1, 320, F16, E5M2, True, -1),
+    ([700, 5], [50, 300], 16, 4, 272, BF16, BF16, True, -1),
     ([255, 0], [1, 256], 32, 8, 128, BF16, BF16, True, -1),    # pieces of the least length
     ([500], [2100], 8, 1, 128, BF16, BF16, True, -1),          # over 64 row tiles: the plan kernel lists the pieces
     ([3000] * 40 + [0] * 30, [5] * 40 + [0, 2] * 15, 16, 2, 128, F16, F16, True, -1),  # over 64 sequences
