@@ -14,6 +14,7 @@ namespace ma {
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+typedef __attribute__((__vector_size__(2 * sizeof(float)))) float f32x2;
 typedef __attribute__((__vector_size__(2 * sizeof(_Float16)))) _Float16 f16x2;
 typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
 typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
@@ -212,16 +213,16 @@ __device__ __forceinline__ float h2f(uint32_t bits16) {
   else return (float)__builtin_bit_cast(_Float16, (uint16_t)bits16);
 }
 
+// Two floats -> packed 16-bit output values, rounded to nearest even (bf16: one
+// v_cvt_pk_bf16_f32, against sixteen instructions of integer rounding before).
 template <bool BF16>
-__device__ __forceinline__ uint16_t f2h(float x) {
+__device__ __forceinline__ uint32_t pack_out(float a, float b) {
   if constexpr (BF16) {
-    // round to nearest even; NaN stays NaN
-    uint32_t u = __builtin_bit_cast(uint32_t, x);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
+    const f32x2 v = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
   } else {
-    return __builtin_bit_cast(uint16_t, (_Float16)x);
+    const f16x2 v = {(_Float16)a, (_Float16)b};
+    return __builtin_bit_cast(uint32_t, v);
   }
 }
 
@@ -233,8 +234,8 @@ __device__ __forceinline__ void store_out4(void* out, int64_t off, f32x4 v, floa
     *reinterpret_cast<f32x4 MA_GLOBAL*>(gptr_mut(reinterpret_cast<float*>(out)) + off) = v * s;
   } else {
     u32x2 w;
-    w[0] = (uint32_t)f2h<BF16>(v[0] * s) | ((uint32_t)f2h<BF16>(v[1] * s) << 16);
-    w[1] = (uint32_t)f2h<BF16>(v[2] * s) | ((uint32_t)f2h<BF16>(v[3] * s) << 16);
+    w[0] = pack_out<BF16>(v[0] * s, v[1] * s);
+    w[1] = pack_out<BF16>(v[2] * s, v[3] * s);
     *reinterpret_cast<u32x2 MA_GLOBAL*>(gptr_mut(reinterpret_cast<uint16_t*>(out)) + off) = w;
   }
 }

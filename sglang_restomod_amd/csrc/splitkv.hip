@@ -73,7 +73,7 @@ constexpr int kTileKeys() {
   return (D == 256 && !FP8) ? 16 : 32;
 }
 constexpr int kMinTiles = 2;  // least tiles per active wave
-constexpr int kDescInts = 8;  // per wave: valid, sequence, kv head, row group, first wave, its slot
+constexpr int kDescInts = 8;  // per wave: valid, sequence, kv head, row group, first wave, its slot, absent
 
 struct SplitKVArgs {
   const void* q;
@@ -94,7 +94,8 @@ struct SplitKVArgs {
   float scale_log2;          // softmax_scale * k_scale * log2(e)
   float v_scale;
   int nwaves;                // waves of the persistent grid
-  int merge_split;           // merge workgroups per wave: 1, or one per row set of a row group
+  int merge_split;           // merge workgroups per descriptor group: 1, or one per row set of a row group
+  int merge_waves;           // waves (descriptors) per merge workgroup
   int* desc;                 // [nwaves][kDescInts] shared segment ending in each wave's first piece
   float* part_o;             // [nwaves][2][kMaxRows][D]
   float* part_lse;           // [nwaves][2][kMaxRows]
@@ -131,8 +132,9 @@ __device__ __forceinline__ Geom geom(const SplitKVArgs& a, int b) {
   g.lo_min = min(g.lo_min, g.seq);
   g.span = g.seq - g.lo_min;
   g.nt = (g.span + (1 << TS) - 1) / (1 << TS);
-  const int real_rows = max(g.ntok, 0) * a.group;
-  g.rg_real = (int)(((int64_t)real_rows + a.rows - 1) / a.rows);  // every query row, whatever the host's hint
+  // every query row, whatever the host's hint; rows is 16 or 32 (token x group stays below 2^31)
+  const uint32_t real_rows = (uint32_t)(max(g.ntok, 0) * a.group);
+  g.rg_real = (int)((real_rows + (uint32_t)(a.rows - 1)) >> (a.rows == 32 ? 5 : 4));
   g.seq_row = a.row_index ? cptr(a.row_index)[b] : (int64_t)b;
   return g;
 }
@@ -150,46 +152,47 @@ __device__ __forceinline__ int64_t seq_work(const SplitKVArgs& a, int b) {
   return (int64_t)g.nt * g.rg_real * a.hkv;
 }
 
-__device__ __forceinline__ int64_t shfl_up_i64(int64_t v, int delta) {
-  const int lane = lane_id();
-  const int src = (lane >= delta ? lane - delta : lane) << 2;
-  const int lo = __builtin_amdgcn_ds_bpermute(src, (int)(uint32_t)v);
-  const int hi = __builtin_amdgcn_ds_bpermute(src, (int)(v >> 32));
-  return (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
-}
-
 __device__ __forceinline__ int64_t readlane_i64(int64_t v, int lane) {
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
   const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), lane);
   return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
-// Total tiles, and (when t >= 0) the sequence holding global tile t and t's offset in it.
+// Inclusive prefix sum over the wave's lanes, by DPP moves.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int64_t dpp0_i64(int64_t x) {  // x of another lane, 0 where there is none
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, CTRL, ROWS, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(x >> 32), CTRL, ROWS, 0xf, false);
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ int64_t wave_scan_i64(int64_t x) {
+  x += dpp0_i64<0x111, 0xf>(x);  // row_shr:1, 2, 4, 8 within rows of 16 lanes
+  x += dpp0_i64<0x112, 0xf>(x);
+  x += dpp0_i64<0x114, 0xf>(x);
+  x += dpp0_i64<0x118, 0xf>(x);
+  x += dpp0_i64<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
+  x += dpp0_i64<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+
+// The sequence holding global tile t and t's offset in it.
 template <int TS>
-__device__ __forceinline__ void scan_work(const SplitKVArgs& a, int64_t t, int64_t& total, int& b_at, int64_t& off_at) {
+__device__ __forceinline__ void scan_work(const SplitKVArgs& a, int64_t t, int& b_at, int64_t& off_at) {
   const int lane = lane_id();
   int64_t base = 0;
-  b_at = -1;
-  off_at = 0;
   for (int b0 = 0; b0 < a.batch; b0 += 64) {
     const int b = b0 + lane;
     const int64_t w = b < a.batch ? seq_work<TS>(a, b) : 0;
-    int64_t inc = w;
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) {
-      const int64_t y = shfl_up_i64(inc, m);
-      if (lane >= m) inc += y;
-    }
+    const int64_t inc = wave_scan_i64(w);
     const int64_t chunk = readlane_i64(inc, 63);
-    if (b_at < 0 && t >= 0 && base + chunk > t) {
-      const uint64_t hit = __builtin_amdgcn_ballot_w64(base + inc > t);
-      const int L = __builtin_ctzll(hit);
+    if (base + chunk > t) {
+      const int L = __builtin_ctzll(__builtin_amdgcn_ballot_w64(base + inc > t));
       b_at = b0 + L;
       off_at = t - (base + readlane_i64(inc - w, L));
+      return;
     }
     base += chunk;
   }
-  total = base;
 }
 
 // Zeros for every real row of sequence b (a sequence whose rows see no key: no tile
@@ -210,28 +213,23 @@ __device__ __forceinline__ void write_zero_rows(const SplitKVArgs& a, int b) {
 }
 
 // Total tiles over all sequences. Wave W also zeroes the rows of the key-less sequences
-// b with b mod nwaves == W.
+// b with b mod nwaves == W. `work` and `upto`: this lane's sequence of the last 64 (of a
+// batch of at most 64: of all), its tiles and the tiles up to and with it.
 template <int D, int TS>
-__device__ __forceinline__ int64_t scan_total(const SplitKVArgs& a, int W) {
+__device__ __forceinline__ int64_t scan_total(const SplitKVArgs& a, int W, int64_t& work, int64_t& upto) {
   const int lane = lane_id();
   int64_t base = 0;
   for (int b0 = 0; b0 < a.batch; b0 += 64) {
     const int b = b0 + lane;
-    int64_t w = 0;
+    work = 0;
     bool zero = false;
     if (b < a.batch) {
       const Geom g = geom<TS>(a, b);
-      w = (int64_t)g.nt * g.rg_real * a.hkv;
+      work = (int64_t)g.nt * g.rg_real * a.hkv;
       zero = g.nt == 0 && g.ntok > 0 && (b % a.nwaves) == W;
     }
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) {
-      const int src = (lane ^ m) << 2;
-      const int lo = __builtin_amdgcn_ds_bpermute(src, (int)(uint32_t)w);
-      const int hi = __builtin_amdgcn_ds_bpermute(src, (int)(w >> 32));
-      w += (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
-    }
-    base += readlane_i64(w, 0);
+    upto = base + wave_scan_i64(work);
+    base = readlane_i64(upto, 63);
     uint64_t zm = __builtin_amdgcn_ballot_w64(zero);
     while (zm) {
       const int L = __builtin_ctzll(zm);
@@ -355,24 +353,26 @@ __global__ __launch_bounds__(256, 1) void splitkv_partial(const SplitKVArgs args
     else return kk * 32 + j * 8;
   };
 
-  const int64_t total = scan_total<D, kTS>(a, W);
+  int64_t work = 0, upto = 0;
+  const int64_t total = scan_total<D, kTS>(a, W, work, upto);
   const int nA = active_waves(total, a.nwaves);
   int MA_GLOBAL* my_desc = gptr_mut(a.desc) + (int64_t)W * kDescInts;
-  if (W >= nA) {
-    if (lane == 0) my_desc[0] = 0;
+  if (W >= nA || total == 0) {
+    if (lane == 0) {
+      my_desc[0] = 0;
+      my_desc[6] = 1;
+    }
     return;
   }
   const int64_t t0 = wave_begin(W, total, nA);
   const int count = (int)(wave_begin(W + 1, total, nA) - t0);
-  if (count <= 0) {
-    if (lane == 0) my_desc[0] = 0;
-    return;
-  }
-  int b0;
-  int64_t off0;
-  {
-    int64_t tot_again;
-    scan_work<kTS>(a, t0, tot_again, b0, off0);
+  int b0 = 0;
+  int64_t off0 = 0;
+  if (a.batch <= 64) {  // one pass over the lengths was enough
+    b0 = __builtin_ctzll(__builtin_amdgcn_ballot_w64(upto > t0));
+    off0 = t0 - readlane_i64(upto - work, b0);
+  } else {
+    scan_work<kTS>(a, t0, b0, off0);
   }
 
   const unsigned char MA_GLOBAL* kbase = gptr(reinterpret_cast<const unsigned char*>(a.k));
@@ -531,18 +531,23 @@ __global__ __launch_bounds__(256, 1) void splitkv_partial(const SplitKVArgs args
     }
   };
 
-  // Write this piece: the final output when it covers the whole segment, else a partial.
-  auto end_segment = [&](const Cursor& cu, bool whole, int slot_sel) __attribute__((always_inline)) {
+  // Row sums of the current piece over the lanes of a row.
+  auto row_sums = [&](float (&lt)[NB]) __attribute__((always_inline)) {
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-      float lt = l_run[nb];
-      lt += shfl_xor_f(lt, 16);
-      lt += shfl_xor_f(lt, 32);
+      lt[nb] = l_run[nb] + shfl_xor_f(l_run[nb], 16);
+      lt[nb] += shfl_xor_f(lt[nb], 32);
+    }
+  };
+  // Write this piece: the final output when it covers the whole segment, else a partial.
+  auto end_segment = [&](const Cursor& cu, const float (&lt)[NB], bool whole, int slot_sel) __attribute__((always_inline)) {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
       if (!real[nb]) continue;
       const int R = cu.rg * kRows + nb * 16 + c;
       const int t = R / a.group;
       const int g = R - t * a.group;
-      const float inv = lt > 0.f ? 1.f / lt : 0.f;
+      const float inv = lt[nb] > 0.f ? 1.f / lt[nb] : 0.f;
       if (whole) {
         const int64_t off = (int64_t)(cu.g.tok0 + t) * a.out_stride_tok + (int64_t)(cu.h * a.group + g) * a.out_stride_head;
         const float sc = inv * a.v_scale;
@@ -555,12 +560,14 @@ __global__ __launch_bounds__(256, 1) void splitkv_partial(const SplitKVArgs args
         for (int db = 0; db < DB; ++db) *reinterpret_cast<f32x4 MA_GLOBAL*>(po + db * 16 + 4 * j) = o[nb][db] * inv;
         if (j == 0) {
           const float mu = (m_run[nb] == -INFINITY) ? 0.f : m_run[nb];
-          gptr_mut(a.part_lse)[pidx] = lt > 0.f ? __builtin_amdgcn_logf(lt) + mu * a.scale_log2 : kEmptyLse;
+          gptr_mut(a.part_lse)[pidx] = lt[nb] > 0.f ? __builtin_amdgcn_logf(lt[nb]) + mu * a.scale_log2 : kEmptyLse;
         }
       }
     }
-    if (!whole && slot_sel == 0 && cu.tile == cu.g.nt - 1) {
-      // first piece of this range and last tile of its segment, which began earlier
+  };
+  // The piece ends its segment, which began in an earlier wave: this wave's descriptor names it.
+  auto note_end = [&](const Cursor& cu) __attribute__((always_inline)) {
+    if (first_piece && cu.tile == cu.g.nt - 1) {
       ends_shared = true;
       end_b = cu.g.b;
       end_h = cu.h;
@@ -574,32 +581,59 @@ __global__ __launch_bounds__(256, 1) void splitkv_partial(const SplitKVArgs args
     const unsigned char* vt = vring[wave][stage];
     // ---- K operand: the tile's rows from the K ring, unswizzled into operand order ----
     const unsigned char* ks = kring[wave][stage];
-    u32x4 kr[TB][KK];
-#pragma unroll
-    for (int tb = 0; tb < TB; ++tb) {
+    auto chunk = [&](int tb, int q) -> u32x4 {
       const int t = tb * 16 + c;
-      auto chunk = [&](int q) -> u32x4 {
-        return *reinterpret_cast<const u32x4*>(ks + t * kRowB + (((4 * q + j) ^ swzk(t)) << 4));
-      };
-      if constexpr (kFp8) {
-#pragma unroll
-        for (int half = 0; half < KK / 2; ++half) cvt16_fp8<KV, QBF16>(chunk(half), kr[tb][2 * half], kr[tb][2 * half + 1]);
-      } else {
-#pragma unroll
-        for (int kk = 0; kk < KK; ++kk) kr[tb][kk] = chunk(kk);
-      }
-    }
+      return *reinterpret_cast<const u32x4*>(ks + t * kRowB + (((4 * q + j) ^ swzk(t)) << 4));
+    };
     // ---- S^T = K Q^T ----
     f32x4 s[NB][TB];
+    if constexpr (D == 256 && NB == 2) {
+      // two row blocks at 256 dims: each K fragment meets both at once, so that the tile's
+      // fragments (64 registers) are not all held next to Q (64) and O (128)
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) s[nb][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int q = 0; q < (kFp8 ? KK / 2 : KK); ++q)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) {
+          const u32x4 raw = chunk(tb, q);
+          if constexpr (kFp8) {
+            u32x4 k0, k1;
+            cvt16_fp8<KV, QBF16>(raw, k0, k1);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+              s[nb][tb] = mfma16t<QBF16>(k0, qv[nb][2 * q], s[nb][tb]);
+              s[nb][tb] = mfma16t<QBF16>(k1, qv[nb][2 * q + 1], s[nb][tb]);
+            }
+          } else {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) s[nb][tb] = mfma16t<QBF16>(raw, qv[nb][q], s[nb][tb]);
+          }
+        }
+    } else {
+      u32x4 kr[TB][KK];
 #pragma unroll
       for (int tb = 0; tb < TB; ++tb) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (kFp8) {
 #pragma unroll
-        for (int kk = 0; kk < KK; ++kk) acc = mfma16t<QBF16>(kr[tb][kk], qv[nb][kk], acc);
-        s[nb][tb] = acc;
+          for (int half = 0; half < KK / 2; ++half) cvt16_fp8<KV, QBF16>(chunk(tb, half), kr[tb][2 * half], kr[tb][2 * half + 1]);
+        } else {
+#pragma unroll
+          for (int kk = 0; kk < KK; ++kk) kr[tb][kk] = chunk(tb, kk);
+        }
       }
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) {
+          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int kk = 0; kk < KK; ++kk) acc = mfma16t<QBF16>(kr[tb][kk], qv[nb][kk], acc);
+          s[nb][tb] = acc;
+        }
+    }
     // ---- online softmax ----
     const bool full = (tb0 >= lmax) && (tb0 + kTile <= hmin);
     u32x4 pb[NB], pl[NB];
@@ -751,16 +785,21 @@ __global__ __launch_bounds__(256, 1) void splitkv_partial(const SplitKVArgs args
     (vstep(std::integral_constant<int, Is>{}), ...);
   }(std::make_integer_sequence<int, A>{});
 
+  // I: n % S, a constant where the steps of a round are unrolled. With two stages the slot
+  // lookup of a step serves that step's issue (one register), and the step is not unrolled:
+  // one copy of its code, which is most of a small call's instruction fetches.
   auto step = [&](auto I_, int n) __attribute__((always_inline)) {
-    constexpr int I = decltype(I_)::value;
-    constexpr int RI = (I + S - 1) % S;
+    const int I = I_;
+    const int SL = S == 2 ? 0 : (I + A) % S;
+    const int RI = (I + S - 1) % S;
+    const int RS = S == 2 ? 0 : RI;
     // slot of tile n+A -> sreg[(n+A) % S] (that register's previous tile is already issued)
-    sreg[(I + A) % S] = load_slot(cs);
+    sreg[SL] = load_slot(cs);
     cursor_next<kTS>(a, cs, count);
     // K/V of tile n+S-1, once its slot lookup (A-S+1 steps ago) has landed
     wait_vm(std::integral_constant<int, OPS * (A - S + 1)>{});
-    __asm__ volatile("" : "+v"(sreg[RI]));
-    issue(ci, slot_of(ci, sreg[RI]), RI);
+    __asm__ volatile("" : "+v"(sreg[RS]));
+    issue(ci, slot_of(ci, sreg[RS]), RI);
     cursor_next<kTS>(a, ci, count);
     if (n < count) {
       if (cc.t == 0 || cc.tile == 0) {
@@ -777,12 +816,13 @@ __global__ __launch_bounds__(256, 1) void splitkv_partial(const SplitKVArgs args
       // only tile n, so S-1 tiles stay in flight, which is 12% faster than waiting for all.
       wait_vm(std::integral_constant<int, (kFp8 || S < 4) ? (S - 1) * OPS : kInFlight16 * OPS>{});
       compute(cc, I);
-      const bool seg_last = (cc.tile == cc.g.nt - 1);
-      const bool range_last = (n == count - 1);
-      if (seg_last || range_last) {
-        const bool whole = seg_last && (cc.tile == cc.t - piece_start_t);
-        // slot 0: the first piece of the range (also a single-piece range); slot 1: the last
-        end_segment(cc, whole, first_piece ? 0 : 1);
+      // a segment that ends before the range does (the range's last piece: below the loop)
+      if (cc.tile == cc.g.nt - 1 && n < count - 1) {
+        const bool whole = cc.tile == cc.t - piece_start_t;
+        float lt[NB];
+        row_sums(lt);
+        end_segment(cc, lt, whole, 0);  // cut only at its start: the first piece of the range
+        if (!whole) note_end(cc);
         first_piece = false;
       }
       cursor_next<kTS>(a, cc, count);
@@ -792,11 +832,84 @@ __global__ __launch_bounds__(256, 1) void splitkv_partial(const SplitKVArgs args
   auto group = [&]<int... Is>(std::integer_sequence<int, Is...>, int n) __attribute__((always_inline)) {
     (step(std::integral_constant<int, Is>{}, n + Is), ...);
   };
-  for (int n = 0; n < count; n += S) group(std::make_integer_sequence<int, S>{}, n);
+  if constexpr (S == 2) {
+#pragma unroll 1
+    for (int n = 0; n < count; ++n) step(n & 1, n);
+  } else {
+    for (int n = 0; n < count; n += S) group(std::make_integer_sequence<int, S>{}, n);
+  }
+
+  wait_vm(std::integral_constant<int, OPS - 1>{});  // the last slot lookups land before their registers are used again
+#pragma unroll
+  for (int i = 0; i < S; ++i) __asm__ volatile("" : "+v"(sreg[i]));
+
+  // ---- the range's last piece ----
+  // A workgroup whose four waves hold one piece each of one segment merges them through LDS
+  // first (waves 1 into 0 and 3 into 2, then 2 into 0) and leaves one partial instead of
+  // four: few sequences over long contexts cut a segment into a piece per wave, and writing
+  // and re-reading those (25 MB on 6 sequences of 16k keys, 2 kv heads, 24 rows, D = 256)
+  // cost more than the merge itself.
+  const bool seg_last = cc.tile == cc.g.nt - 1;
+  const bool whole = seg_last && cc.tile == cc.t - piece_start_t;
+  float lt[NB];
+  row_sums(lt);
+  bool absent = false;
+  {
+    __shared__ float mrow[kWaves][kRows], lrow[kWaves][kRows];
+    static_assert(16 * D * 4 <= S * kStage, "a row block's output fits a wave's ring");
+    // the workgroup's tiles lie in this wave's last segment: true for one wave, true for all
+    const int wg0 = (int)blockIdx.x * kWaves;
+    const int64_t seg0 = t0 + cc.t - cc.tile;
+    if (wg0 + kWaves <= nA && seg0 <= wave_begin(wg0, total, nA) &&
+        wave_begin(wg0 + kWaves, total, nA) <= seg0 + cc.g.nt) {
+      wait_vm(std::integral_constant<int, 0>{});  // no DMA may land in the rings from here on
+      __syncthreads();
+      auto part = [&](int w, int nb) __attribute__((always_inline)) -> f32x4* {
+        return reinterpret_cast<f32x4*>(nb == 0 ? kring[w][0] : vring[w][0]);
+      };
+#pragma unroll
+      for (int step_w = 1; step_w < kWaves; step_w <<= 1) {
+        const int low = wave & (2 * step_w - 1);
+        if (low == step_w) {
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) {
+            f32x4* dst = part(wave, nb);
+#pragma unroll
+            for (int db = 0; db < DB; ++db) dst[db * 64 + lane] = o[nb][db];
+            if (j == 0) {
+              mrow[wave][nb * 16 + c] = m_run[nb];
+              lrow[wave][nb * 16 + c] = lt[nb];
+            }
+          }
+        }
+        __syncthreads();
+        if (low == 0) {
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) {
+            const float m2 = mrow[wave + step_w][nb * 16 + c];
+            const float m_new = fmaxf(m_run[nb], m2);
+            const float mu = m_new == -INFINITY ? 0.f : m_new;
+            const float s1 = __builtin_amdgcn_exp2f((m_run[nb] - mu) * a.scale_log2);
+            const float s2 = __builtin_amdgcn_exp2f((m2 - mu) * a.scale_log2);
+            const f32x4* src = part(wave + step_w, nb);
+#pragma unroll
+            for (int db = 0; db < DB; ++db) o[nb][db] = o[nb][db] * s1 + src[db * 64 + lane] * s2;
+            lt[nb] = lt[nb] * s1 + lrow[wave + step_w][nb * 16 + c] * s2;
+            m_run[nb] = m_new;
+          }
+        }
+      }
+      absent = wave != 0;
+    }
+  }
+  // slot 0: the first piece of the range (also a single-piece range); slot 1: the last
+  if (!absent) end_segment(cc, lt, whole, first_piece ? 0 : 1);
+  if (!whole) note_end(cc);
 
   // ---- descriptor of the shared segment ending here (read by splitkv_merge) ----
   if (lane == 0) {
     int MA_GLOBAL* dsc = my_desc;
+    dsc[6] = absent;
     if (ends_shared) {
       const int w1 = wave_of(end_first, total, nA);
       dsc[1] = end_b;
@@ -836,73 +949,82 @@ template <int D, int NB, bool QBF16>
 __global__ __launch_bounds__(256) void splitkv_merge(const SplitKVArgs args) {
   const SplitKVArgs a = args;
   constexpr int kRows = 16 * NB;
-  const int split = a.merge_split;  // workgroups per partial-kernel wave: 1 or kPass
-  const int W = blockIdx.x / split;
-  const int part = blockIdx.x - W * split;
-  const int MA_CONST* dsc = cptr(a.desc) + (int64_t)W * kDescInts;
-  if (dsc[0] == 0) return;
-  const int b = dsc[1], h = dsc[2], rg = dsc[3], w1 = dsc[4], sel1 = dsc[5];
-  const Geom g = geom_u<5>(a, b);  // only its token range is read here, not the tile count
-  const float MA_GLOBAL* plse = gptr(a.part_lse);
-  const float MA_GLOBAL* po = gptr(a.part_o);
   constexpr int kTPR = D / 4;       // threads per row, four head-dim entries each
   constexpr int kRPP = 256 / kTPR;  // rows per pass of the workgroup
-  const int d4 = (threadIdx.x % kTPR) * 4;
-  const int r_base = threadIdx.x / kTPR;
-  // thread: rows r_base + kRPP i, head-dim entries d4..d4+3. Each row set has a workgroup
-  // of its own (one whose rows are all GQA padding returns at once). Within a row set the pieces
-  // are the outer loop (unrolled by four), so the loads of four pieces are in flight
-  // together. Measured at D=128 on a verify batch of 32 x 4 tokens: 13 us with one row
-  // set at a time in one workgroup, 10 us with all four together, 8.0 us with a
-  // workgroup per row set; about 5 us on a decode batch of 64.
   constexpr int kPass = merge_passes<D, NB>();
   static_assert(kPass == (kRows / kRPP > 0 ? kRows / kRPP : 1), "a row set is one pass");
-  constexpr int kChunk = 1;
-  for (int c0 = split == 1 ? 0 : part; c0 < (split == 1 ? kPass : part + 1); c0 += kChunk) {
-    bool live = false;  // rows past the last query token (GQA padding) are not read
-#pragma unroll
-    for (int i = 0; i < kChunk; ++i) {
-      const int row = r_base + kRPP * (c0 + i);
-      live |= row < kRows && (rg * kRows + row) / a.group < g.ntok;
-    }
-    if (!live) continue;
-    float m[kChunk], wsum[kChunk];
-    f32x4 acc[kChunk];
-#pragma unroll
-    for (int i = 0; i < kChunk; ++i) {
-      m[i] = -INFINITY;
-      wsum[i] = 0.f;
-      acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll 4
-    for (int w = w1; w <= W; ++w) {
-      const int64_t pbase = ((int64_t)w * 2 + (w == w1 ? sel1 : 0)) * kMaxRows + r_base + kRPP * c0;
-      float lse[kChunk];
-      f32x4 o[kChunk];
-#pragma unroll
-      for (int i = 0; i < kChunk; ++i) {
-        lse[i] = plse[pbase + kRPP * i];
-        o[i] = *reinterpret_cast<const f32x4 MA_GLOBAL*>(po + (pbase + kRPP * i) * D + d4);
-      }
-#pragma unroll
-      for (int i = 0; i < kChunk; ++i) {
-        const float m_new = fmaxf(m[i], lse[i]);  // every LSE is finite (empty pieces: -2^30)
-        const float s_old = __builtin_amdgcn_exp2f(m[i] - m_new);
-        const float s_new = __builtin_amdgcn_exp2f(lse[i] - m_new);
-        acc[i] = acc[i] * s_old + o[i] * s_new;
-        wsum[i] = wsum[i] * s_old + s_new;
-        m[i] = m_new;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < kChunk; ++i) {
-      const int row = r_base + kRPP * (c0 + i);
+  const int split = a.merge_split;  // workgroups per descriptor group: 1 or kPass
+  const int group0 = ((int)blockIdx.x / split) * a.merge_waves;
+  const int part = (int)blockIdx.x % split;
+  const float MA_GLOBAL* plse = gptr(a.part_lse);
+  const float MA_GLOBAL* po = gptr(a.part_o);
+  const int lane = threadIdx.x & 63;
+  const int d4 = (threadIdx.x % kTPR) * 4;
+  const int r_base = threadIdx.x / kTPR;
+  for (int W = group0; W < group0 + a.merge_waves; ++W) {
+    const int MA_CONST* dsc = cptr(a.desc) + (int64_t)W * kDescInts;
+    if (dsc[0] == 0) continue;
+    const int b = dsc[1], h = dsc[2], rg = dsc[3], w1 = dsc[4], sel1 = dsc[5];
+    const Geom g = geom_u<5>(a, b);  // only its token range is read here, not the tile count
+    // thread: row r_base of a row set, head-dim entries d4..d4+3. Each row set has a
+    // workgroup of its own when more than one holds real rows. Measured at D=128 on a verify
+    // batch of 32 x 4 tokens: 13 us with one row set at a time in one workgroup, 8.0 us with
+    // a workgroup per row set; about 5 us on a decode batch of 64.
+    for (int c0 = split == 1 ? 0 : part; c0 < (split == 1 ? kPass : part + 1); ++c0) {
+      const int row = r_base + kRPP * c0;
       const int R = rg * kRows + row;
       const int t = R / a.group;
+      // rows past the last query token (GQA padding) are not read (a wave's rows differ at
+      // D = 64 and 128 only; the loop below stays wave-uniform)
+      const bool live = row < kRows && t < g.ntok;
+      if (!__builtin_amdgcn_ballot_w64(live)) continue;
+      float m = -INFINITY, wsum = 0.f;
+      f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+      const int64_t rrow = live ? row : 0;
+      // pieces of the waves in `mask` (bit i: wave w0 + i), the N lowest: all loads in flight
+      // together; past the last, the last one again with weight 0
+      auto batch = [&](auto N_, int w0, uint64_t& mask) __attribute__((always_inline)) {
+        constexpr int N = decltype(N_)::value;
+        float lse[N];
+        f32x4 o[N];
+        const int n = __builtin_popcountll(mask);
+        int w = w0;
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+          if (mask) {
+            w = w0 + __builtin_ctzll(mask);
+            mask &= mask - 1;
+          }
+          const int64_t p = ((int64_t)w * 2 + (w == w1 ? sel1 : 0)) * kMaxRows + rrow;
+          lse[u] = plse[p];
+          o[u] = *reinterpret_cast<const f32x4 MA_GLOBAL*>(po + p * D + d4);
+        }
+        float m_new = m;
+#pragma unroll
+        for (int u = 0; u < N; ++u) m_new = fmaxf(m_new, lse[u]);  // every LSE is finite (empty pieces: -2^30)
+        const float s_old = __builtin_amdgcn_exp2f(m - m_new);
+        acc = acc * s_old;
+        wsum = wsum * s_old;
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+          const float s_new = u < n ? __builtin_amdgcn_exp2f(lse[u] - m_new) : 0.f;
+          acc = acc + o[u] * s_new;
+          wsum += s_new;
+        }
+        m = m_new;
+      };
+      for (int w0 = w1; w0 <= W; w0 += 64) {
+        const int w = min(w0 + lane, W);
+        uint64_t mask = __builtin_amdgcn_ballot_w64(w0 + lane <= W && gptr(a.desc)[(int64_t)w * kDescInts + 6] == 0);
+        while (mask) {
+          if (__builtin_popcountll(mask) <= 4) batch(std::integral_constant<int, 4>{}, w0, mask);
+          else batch(std::integral_constant<int, 8>{}, w0, mask);
+        }
+      }
+      if (!live) continue;
       const int gg = R - t * a.group;
-      if (row >= kRows || t >= g.ntok) continue;
       const int64_t off = (int64_t)(g.tok0 + t) * a.out_stride_tok + (int64_t)(h * a.group + gg) * a.out_stride_head + d4;
-      store_out4<QBF16>(a.out, off, acc[i], a.v_scale / wsum[i], a.out_f32);
+      store_out4<QBF16>(a.out, off, acc, a.v_scale / wsum, a.out_f32);
     }
   }
 }
@@ -917,31 +1039,21 @@ static hipError_t launch_partial_kv(int kv, dim3 grid, hipStream_t st, const Spl
   return hipGetLastError();
 }
 
-// Row blocks per row group: at D = 256 only one (two would spill registers that in-flight
-// loads still target); the host then uses more row groups of 16 rows.
-template <int D>
-constexpr int kMaxNB = D == 256 ? 1 : 2;
-
 template <int D>
 static hipError_t launch_partial_d(int nb, bool qbf16, int kv, dim3 grid, hipStream_t st, const SplitKVArgs& a) {
-  if constexpr (kMaxNB<D> == 1) {
-    return qbf16 ? launch_partial_kv<D, 1, true>(kv, grid, st, a) : launch_partial_kv<D, 1, false>(kv, grid, st, a);
-  } else {
-    if (qbf16) return nb == 1 ? launch_partial_kv<D, 1, true>(kv, grid, st, a) : launch_partial_kv<D, 2, true>(kv, grid, st, a);
-    return nb == 1 ? launch_partial_kv<D, 1, false>(kv, grid, st, a) : launch_partial_kv<D, 2, false>(kv, grid, st, a);
-  }
+  if (qbf16) return nb == 1 ? launch_partial_kv<D, 1, true>(kv, grid, st, a) : launch_partial_kv<D, 2, true>(kv, grid, st, a);
+  return nb == 1 ? launch_partial_kv<D, 1, false>(kv, grid, st, a) : launch_partial_kv<D, 2, false>(kv, grid, st, a);
 }
 
 template <int D>
 static hipError_t launch_merge_d(int nb, bool qbf16, int nwaves, hipStream_t st, const SplitKVArgs& a) {
-  constexpr int NB2 = kMaxNB<D>;
-  const dim3 grid((unsigned)(nwaves * a.merge_split));
+  const dim3 grid((unsigned)(nwaves / a.merge_waves * a.merge_split));
   if (qbf16) {
     if (nb == 1) hipLaunchKernelGGL((splitkv_merge<D, 1, true>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((splitkv_merge<D, NB2, true>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((splitkv_merge<D, 2, true>), grid, dim3(256), 0, st, a);
   } else {
     if (nb == 1) hipLaunchKernelGGL((splitkv_merge<D, 1, false>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((splitkv_merge<D, NB2, false>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((splitkv_merge<D, 2, false>), grid, dim3(256), 0, st, a);
   }
   return hipGetLastError();
 }
@@ -1126,13 +1238,16 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
     return MA_OK;
   }
   const int rows_total = max_q_per_seq * a.group;
-  const int nb = (rows_total <= 16 || head_dim == 256) ? 1 : 2;
+  const int nb = rows_total <= 16 ? 1 : 2;
   a.rows = 16 * nb;
   a.row_groups = (rows_total + a.rows - 1) / a.rows;
   a.nwaves = num_workgroups * kWaves;
   a.merge_split = head_dim == 64    ? (nb == 1 ? merge_split<64, 1>(rows_total) : merge_split<64, 2>(rows_total))
                   : head_dim == 128 ? (nb == 1 ? merge_split<128, 1>(rows_total) : merge_split<128, 2>(rows_total))
-                                    : merge_split<256, 1>(rows_total);
+                                    : nb == 1 ? merge_split<256, 1>(rows_total) : merge_split<256, 2>(rows_total);
+  // few segments: few waves end one, and a merge workgroup looks at a workgroup's four
+  // descriptors (8,192 workgroups that mostly find nothing took 10 us by themselves)
+  a.merge_waves = (int64_t)a.batch * a.hkv * a.row_groups * 16 <= a.nwaves ? kWaves : 1;
   const size_t need = ma_splitkv_workspace_bytes(num_workgroups, head_dim);
   if (!workspace || workspace_bytes < need)
     return set_error(MA_EINVAL, "workspace too small: %zu < %zu bytes", workspace_bytes, need);
