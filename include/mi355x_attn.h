@@ -81,9 +81,8 @@ int ma_device_workgroups(void);
  * `num_workgroups` workgroups (1..16384): one descriptor per wave, then the partial
  * results of segments shared by several waves. No initialisation is needed; calls
  * that overlap in time must use different workspaces. At the head dims other than 64,
- * 128 and 256 it holds only the key pieces of a split decode (2 * num_workgroups
- * pieces of 16 rows); there a decode given no workspace runs without the split, and
- * verify uses none.
+ * 128 and 256 it holds only the key pieces of a split row block (2 * num_workgroups
+ * pieces of 16 rows); there a call given no workspace runs without the split.
  */
 size_t ma_splitkv_workspace_bytes(int num_workgroups, int head_dim);
 
@@ -170,6 +169,21 @@ int ma_paged_verify(const void* q, int64_t q_stride_tok, int64_t q_stride_head, 
                     int num_workgroups, float softmax_scale, float k_scale, float v_scale,
                     void* workspace, size_t workspace_bytes, void* out, int out_dtype,
                     int64_t out_stride_tok, int64_t out_stride_head, void* stream);
+
+/*
+ * ma_paged_verify with `max_seq_len`: an upper bound of seq_lens the caller knows without
+ * reading the device, or 0 for none, as for ma_grouped_decode: it only chooses the kernels.
+ */
+int ma_paged_verify_bounded(const void* q, int64_t q_stride_tok, int64_t q_stride_head, int q_dtype,
+                            int64_t num_tokens, const void* k_cache, const void* v_cache,
+                            int64_t kv_stride_row, int64_t kv_stride_head, int kv_dtype,
+                            const int32_t* table, int64_t table_stride, const int64_t* row_index,
+                            int page_size, const int32_t* seq_lens, const int32_t* query_start_loc,
+                            const int32_t* prefix_lens, int batch, int max_q_per_seq, int num_q_heads,
+                            int num_kv_heads, int head_dim, int causal, int sliding_window,
+                            int num_workgroups, float softmax_scale, float k_scale, float v_scale,
+                            int max_seq_len, void* workspace, size_t workspace_bytes, void* out,
+                            int out_dtype, int64_t out_stride_tok, int64_t out_stride_head, void* stream);
 
 /*
  * Bytes of workspace ma_paged_extend needs for `num_tokens` query tokens in `batch`

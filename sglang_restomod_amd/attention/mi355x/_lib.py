@@ -62,6 +62,17 @@ SIGNATURES = {
         c_float, c_float, c_float, c_void_p, c_size_t,  # scales, workspace, bytes
         c_void_p, c_int, c_int64, c_int64, c_void_p,  # out, out dtype, strides, stream
     ]),
+    "ma_paged_verify_bounded": (c_int, [
+        c_void_p, c_int64, c_int64, c_int, c_int64,   # q, strides, dtype, num_tokens
+        c_void_p, c_void_p, c_int64, c_int64, c_int,  # k, v, strides, kv dtype
+        c_void_p, c_int64, c_void_p, c_int,           # table, stride, row_index, page size
+        c_void_p, c_void_p, c_void_p,                 # seq_lens, qsl, prefix
+        c_int, c_int, c_int, c_int, c_int,            # batch, max_q, hq, hkv, dim
+        c_int, c_int, c_int,                          # causal, window, num_workgroups
+        c_float, c_float, c_float, c_int,             # scales, max_seq_len
+        c_void_p, c_size_t,                           # workspace, bytes
+        c_void_p, c_int, c_int64, c_int64, c_void_p,  # out, out dtype, strides, stream
+    ]),
     "ma_set_kv_buffer": (c_int, [
         c_void_p, c_void_p, c_int64, c_int64, c_int,  # k, v, strides, source dtype
         c_void_p, c_int64, c_int, c_int,              # loc, num_tokens, hkv, dim

@@ -480,6 +480,7 @@ class MI355XAttnBackend(_EngineBase):
                 softmax_scale=float(layer.scaling), causal=causal, sliding_window_size=window,
                 linear_verify=md.mode == MODE_VERIFY, k_scale=ks, v_scale=vs, row_index=rows,
                 max_q_len_hint=md.max_q_per_seq if md.mode == MODE_VERIFY else None,
+                max_seq_len_hint=md.max_seq_len or None,
                 workspace=self._workspace_for(md.mode, q3.shape[0], hq, int(layer.tp_k_head_num),
                                               md.seq_lens.shape[0]))
         out = out.reshape(q3.shape[0], hq * d)

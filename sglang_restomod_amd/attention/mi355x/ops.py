@@ -378,19 +378,19 @@ def paged_verify_forward(
     qsl = _i32(query_start_loc)
     pre = None if prefix_kv_lens is None else _i32(prefix_kv_lens)
     ridx = _i64(row_index)
-    del max_seq_len_hint
+    max_len = 0 if max_seq_len_hint is None else max(0, int(max_seq_len_hint))  # picks kernels only
     nwg = int(num_workgroups) if num_workgroups else splitkv_workgroups(dev)
     lib = _lib.load()
     stream = _stream_ptr(dev)
     ws, nbytes = _splitkv_ws(lib, dev, nwg, D, workspace, stream)
-    status = lib.ma_paged_verify(
+    status = lib.ma_paged_verify_bounded(
         q.data_ptr(), q.stride(0), q.stride(1), q_dtype_code(q.dtype), T,
         k_cache.data_ptr(), v_cache.data_ptr(), row, head, kv_dtype_code(k_cache.dtype),
         table.data_ptr(), table.stride(0), _ptr(ridx), ps,
         seq.data_ptr(), qsl.data_ptr(), _ptr(pre),
         B, int(max_q_per_seq), Hq, Hkv, D,
         1 if causal else 0, int(sliding_window_size), nwg,
-        float(softmax_scale), float(k_scale), float(v_scale), _ptr(ws), nbytes,
+        float(softmax_scale), float(k_scale), float(v_scale), max_len, _ptr(ws), nbytes,
         out.data_ptr(), out_code, out.stride(0), out.stride(1), stream,
     )
     _lib.check(status, "ma_paged_verify")

@@ -13,6 +13,7 @@ constexpr int kAnyWaves = 4;        // waves per workgroup
 constexpr int kAnyRows = 16;        // query rows per wave
 constexpr int kAnyKeys = 16;        // keys per tile
 constexpr int kAnyMaxDim = 512;
+constexpr int kAnyMaxPieces = 512;  // key pieces of one row block (the merge keeps their weights in LDS)
 
 struct AnyArgs {
   const void* q;
@@ -29,8 +30,9 @@ struct AnyArgs {
   int batch, hq, hkv, group;
   int head_dim;              // D: the kernel's width is the next of 64, 128, 256, 512
   int row_blocks;            // workgroup -> (kv head, key piece, 16-row block of row_blocks, sequence)
-  int pieces;                // decode: workgroups per row block, each over a contiguous piece of
-                             //   the keys (1: one workgroup takes them all)
+  int pieces;                // workgroups per row block, each over a contiguous piece of the
+                             //   keys (1: one workgroup takes them all)
+  int merge_rows;            // rows of a row block the merge visits (1 .. 16)
   float* part_o;             // pieces > 1: each piece's normalised O, [slot][16 rows][DP] fp32,
   float* part_lse;           //   and its log2 LSE [slot][16], slot = (row block item) * pieces + piece
   int causal, window;
@@ -47,8 +49,8 @@ inline bool any_head_dim(int d) {
 }
 
 // Launch on `a` (validated by the caller); returns the
-// launch status. q_dtype DT_F16/DT_BF16, kv_dtype the same or fp8. With pieces > 1 (decode
-// only) the grid is row-block items x pieces and a merge kernel follows.
+// launch status. q_dtype DT_F16/DT_BF16, kv_dtype the same or fp8. With pieces > 1 the
+// grid is row-block items x pieces and a merge kernel follows.
 hipError_t any_launch(const AnyArgs& a, int q_dtype, int kv_dtype, int64_t work_items, hipStream_t stream);
 
 // The padded width of the kernel at head dim d (64, 128, 256 or 512).

@@ -105,7 +105,7 @@ __global__ __launch_bounds__(kAnyWaves * 64, any_wg_per_cu<DP>()) void any_kerne
 
   // The 16 rows r0 .. r0 + 15 of sequence b, kv head h: the four waves take quarter `split`
   // of their key tiles each, merging at the end.
-  auto rows = [&](int b, int h, int r0, int split) __attribute__((always_inline)) {
+  auto rows = [&](int b, int h, int r0, int pieces, int split) __attribute__((always_inline)) {
     int tok0, ntok;
     if (a.qsl) {
       const QueryRows qr = clamp_query_rows(cptr(a.qsl)[b], cptr(a.qsl)[b + 1], a.num_tokens);
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(kAnyWaves * 64, any_wg_per_cu<DP>()) void any_kerne
     const int key_hi = a.causal ? min(seq, prefix + t_last + 1) : seq;
     const int nt = key_hi > key_lo ? (key_hi - key_lo + kAnyKeys - 1) / kAnyKeys : 0;
     // split: this wave's quarter of the workgroup's key piece (pieces x 4 equal shares)
-    const int parts = kAnyWaves * a.pieces;
+    const int parts = kAnyWaves * pieces;
     const int i_lo = (int)((int64_t)split * nt / parts);
     const int i_hi = (int)((int64_t)(split + 1) * nt / parts);
 
@@ -407,7 +407,7 @@ __global__ __launch_bounds__(kAnyWaves * 64, any_wg_per_cu<DP>()) void any_kerne
     // one piece of several (pieces > 1): this workgroup's rows normalised over its keys,
     // in fp32, and their log2 LSE, for the merge kernel; every row is written (a row that
     // saw no key gets O = 0 and LSE -inf)
-    const bool piece_out = a.pieces > 1;
+    const bool piece_out = pieces > 1;
     float MA_GLOBAL* po = nullptr;
     if (piece_out) {
       po = gptr_mut(a.part_o) + (int64_t)piece_slot * (16 * DP) + c * DP + 4 * j;
@@ -439,10 +439,10 @@ __global__ __launch_bounds__(kAnyWaves * 64, any_wg_per_cu<DP>()) void any_kerne
     }
   };
 
-  // decode and verify: workgroup = (kv head, key piece, 16-row block, sequence), kv head
-  // fastest; its four waves take the four quarters of its piece of the rows' key tiles.
-  // A sequence with more rows than row_blocks blocks has its later blocks taken in turn
-  // (verify, whose calls have one piece).
+  // workgroup = (kv head, key piece, 16-row block, sequence), kv head fastest; its four waves
+  // take the four quarters of its piece of the rows' key tiles. A sequence with more rows
+  // than row_blocks blocks (a verify past its hint) has its later blocks taken in turn, whole
+  // (the pieces' slots hold row_blocks blocks), by the workgroups of its first piece.
   const int64_t item = blockIdx.x;
   const int h = (int)(item % a.hkv);
   const int64_t rest = item / a.hkv;
@@ -455,102 +455,105 @@ __global__ __launch_bounds__(kAnyWaves * 64, any_wg_per_cu<DP>()) void any_kerne
   int rows_b;
   if (a.qsl) rows_b = clamp_query_rows(cptr(a.qsl)[b], cptr(a.qsl)[b + 1], a.num_tokens).ntok * a.group;
   else rows_b = (b < a.num_tokens ? 1 : 0) * a.group;
+  int pieces = a.pieces;
 #pragma unroll 1
-  for (int r0 = rb * kAnyRows; r0 < rows_b; r0 += a.row_blocks * kAnyRows)
-    rows(b, h, r0, piece * kAnyWaves + wave);
+  for (int r0 = rb * kAnyRows; r0 < rows_b; r0 += a.row_blocks * kAnyRows) {
+    rows(b, h, r0, pieces, (pieces > 1 ? piece * kAnyWaves : 0) + wave);
+    if (piece > 0) return;
+    pieces = 1;
+  }
 }
 
-// Merge of the key pieces of a decode (pieces > 1): one workgroup per (sequence, 16-row
-// block, kv head), 16 threads per row, each thread four dims of every 64. The row's 16
-// threads read the pieces' log2 LSEs 16 at a time and reduce them across lanes, so every
-// load of a round is in flight together; a piece's weight is 2^(lse - max), and its O
-// chunks are then read eight pieces at a time. Pieces that saw no key have weight 0.
+// Merge of the key pieces (pieces > 1): one workgroup per row of a (sequence, 16-row block,
+// kv head). The threads read the pieces' log2 LSEs together; a piece's weight is
+// 2^(lse - max), kept in LDS. Then DP / 4 threads, four dims each, read a piece's row, the
+// 1024 / DP groups of them every 1024 / DP-th piece, sixteen loads in flight each, and the
+// groups' sums meet in LDS. Pieces that saw no key weigh 0. One workgroup per 16 rows with
+// eight loads in flight took 156 us on the 352 pieces of one sequence of 22k keys at 8 / 1
+// heads and 107 us at D = 256, 12 / 2 heads; this takes ANYMERGE.
 template <int DP, bool QBF16>
 __global__ __launch_bounds__(256) void any_merge(const AnyArgs args) {
   const AnyArgs a = args;
-  constexpr int kNC = DP / 64;  // f32x4 chunks per thread
-  const int item = (int)blockIdx.x;  // (b * row_blocks + rb) * hkv + h
+  constexpr int kTPR = DP / 4;        // threads of one piece's row
+  constexpr int kGroups = 256 / kTPR;
+  constexpr int kFlight = 16;
+  __shared__ float wt[kAnyMaxPieces];
+  __shared__ float red[8];
+  __shared__ __attribute__((aligned(16))) f32x4 sum[kGroups][kTPR];
+  const int item = (int)blockIdx.x / a.merge_rows;  // (b * row_blocks + rb) * hkv + h
+  const int row = (int)blockIdx.x - item * a.merge_rows;
   const int h = item % a.hkv;
   const int blk_item = item / a.hkv;
   const int b = blk_item / a.row_blocks;
   const int rb = blk_item - b * a.row_blocks;
-  const int row = threadIdx.x >> 4;
-  const int part = threadIdx.x & 15;
-  const int lane16 = (threadIdx.x & 63) & ~15;  // first lane of this row's 16 in the wave
-  const int R = rb * kAnyRows + row;  // decode: rows 0 .. G-1 of one token
-  // the row's 16 threads stay together (rows are whole 16-lane groups of a wave)
-  const bool live = b < a.batch && b < a.num_tokens && R < a.group;
+  const int R = rb * kAnyRows + row;
+  const int t = R / a.group;
+  int tok0 = b, ntok = b < a.num_tokens ? 1 : 0;
+  if (a.qsl) {
+    const QueryRows qr = clamp_query_rows(cptr(a.qsl)[b], cptr(a.qsl)[b + 1], a.num_tokens);
+    tok0 = qr.tok0;
+    ntok = qr.ntok;
+  }
+  if (t >= ntok) return;
   const int np = a.pieces;
   const int64_t slot0 = (int64_t)item * np;
   const float MA_GLOBAL* lse = gptr(a.part_lse) + slot0 * 16 + row;
-  const float MA_GLOBAL* po = gptr(a.part_o) + slot0 * (16 * DP) + row * DP + part * 4;
-  // 1. max LSE over the pieces: thread `part` reads pieces part, part + 16, ...
-  float lv[4];  // up to 64 pieces per row in registers
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  // 1. the largest LSE, 2. the weights and their sum
+  float lv[kAnyMaxPieces / 256];
   float m = -INFINITY;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int p = part + 16 * k;
-    lv[k] = (live && p < np) ? lse[(int64_t)p * 16] : -INFINITY;
+  for (int k = 0; k < kAnyMaxPieces / 256; ++k) {
+    const int p = tid + 256 * k;
+    lv[k] = p < np ? lse[(int64_t)p * 16] : -INFINITY;
     m = fmaxf(m, lv[k]);
   }
-  for (int p = part + 64; p < np; p += 16) m = fmaxf(m, live ? lse[(int64_t)p * 16] : -INFINITY);
 #pragma unroll
-  for (int d = 1; d < 16; d <<= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
-  // 2. weights of this thread's pieces and their sum over the row
-  float wv[4];
-  float wsum = 0.f;
+  for (int d = 32; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+  if (lane == 0) red[wave] = m;
+  __syncthreads();
+  m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  float ws = 0.f;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    wv[k] = (lv[k] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(lv[k] - m);
-    wsum += wv[k];
-  }
-  for (int p = part + 64; p < np; p += 16) {
-    const float l = live ? lse[(int64_t)p * 16] : -INFINITY;
-    wsum += (l == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(l - m);
+  for (int k = 0; k < kAnyMaxPieces / 256; ++k) {
+    const int p = tid + 256 * k;
+    const float w = lv[k] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(lv[k] - m);
+    wt[p] = w;
+    ws += w;
   }
 #pragma unroll
-  for (int d = 1; d < 16; d <<= 1) wsum += __shfl_xor(wsum, d, 64);
-  // 3. the weighted sum of the pieces' O, eight pieces' loads in flight at a time
-  f32x4 acc[kNC];
+  for (int d = 32; d >= 1; d >>= 1) ws += __shfl_xor(ws, d, 64);
+  if (lane == 0) red[4 + wave] = ws;
+  __syncthreads();
+  ws = (red[4] + red[5]) + (red[6] + red[7]);
+  // 3. the weighted sum of the pieces' rows
+  const int part = tid % kTPR;
+  const int grp = tid / kTPR;
+  const float MA_GLOBAL* po = gptr(a.part_o) + slot0 * (16 * DP) + row * DP + part * 4;
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int p0 = grp; p0 < np; p0 += kGroups * kFlight) {
+    f32x4 o[kFlight];
 #pragma unroll
-  for (int x = 0; x < kNC; ++x) acc[x] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if (live && wsum > 0.f) {
-    for (int p0 = 0; p0 < np; p0 += 8) {
-      f32x4 ov[8][kNC];
-      float w8[8];
+    for (int u = 0; u < kFlight; ++u) {
+      const int p = p0 + u * kGroups;
+      o[u] = p < np ? *reinterpret_cast<const f32x4 MA_GLOBAL*>(po + (int64_t)p * (16 * DP)) : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int p = p0 + u;
-        // the weight of piece p sits in lane (p % 16) of the row's group, register p / 16
-        const int k = (p >> 4) & 3;
-        const float wk = k == 0 ? wv[0] : k == 1 ? wv[1] : k == 2 ? wv[2] : wv[3];
-        float w = __shfl(wk, lane16 + (p & 15), 64);
-        if (p >= 64) {
-          const float l = p < np ? lse[(int64_t)p * 16] : -INFINITY;
-          w = (l == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(l - m);
-        }
-        w8[u] = p < np ? w : 0.f;
-#pragma unroll
-        for (int x = 0; x < kNC; ++x)
-          ov[u][x] = (p < np && w8[u] > 0.f)
-                         ? *reinterpret_cast<const f32x4 MA_GLOBAL*>(po + (int64_t)p * (16 * DP) + x * 64)
-                         : f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-#pragma unroll
-        for (int x = 0; x < kNC; ++x) acc[x] += ov[u][x] * w8[u];
+    for (int u = 0; u < kFlight; ++u) {
+      const int p = p0 + u * kGroups;
+      acc += o[u] * (p < np ? wt[p] : 0.f);
     }
   }
-  if (!live) return;
-  const float inv = (wsum > 0.f) ? a.v_scale / wsum : 0.f;
-  const int g = R;
-  const int64_t off = (int64_t)b * a.out_stride_tok + (int64_t)(h * a.group + g) * a.out_stride_head;
+  sum[grp][part] = acc;
+  __syncthreads();
+  if (grp > 0) return;
 #pragma unroll
-  for (int x = 0; x < kNC; ++x) {
-    const int d0 = x * 64 + part * 4;
-    if (d0 < a.head_dim) store_out4<QBF16>(a.out, off + d0, acc[x], inv, a.out_f32);
-  }
+  for (int k = 1; k < kGroups; ++k) acc += sum[k][part];
+  const float inv = (ws > 0.f) ? a.v_scale / ws : 0.f;
+  const int64_t off = (int64_t)(tok0 + t) * a.out_stride_tok + (int64_t)(h * a.group + R - t * a.group) * a.out_stride_head;
+  if (part * 4 < a.head_dim) store_out4<QBF16>(a.out, off + part * 4, acc, inv, a.out_f32);
 }
 
 template <int DP, bool QBF16>
@@ -568,7 +571,7 @@ template <int DP>
 static hipError_t launch_any_d(bool qbf16, int kv, dim3 grid, hipStream_t st, const AnyArgs& a) {
   hipError_t e = qbf16 ? launch_any_q<DP, true>(kv, grid, st, a) : launch_any_q<DP, false>(kv, grid, st, a);
   if (e != hipSuccess || a.pieces <= 1) return e;
-  const dim3 mgrid(grid.x / (unsigned)a.pieces);
+  const dim3 mgrid(grid.x / (unsigned)a.pieces * (unsigned)a.merge_rows);
   if (qbf16) hipLaunchKernelGGL((any_merge<DP, true>), mgrid, dim3(256), 0, st, a);
   else hipLaunchKernelGGL((any_merge<DP, false>), mgrid, dim3(256), 0, st, a);
   return hipGetLastError();

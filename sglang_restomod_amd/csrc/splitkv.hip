@@ -1200,7 +1200,7 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
   }
   if (generic || small) {
     // one workgroup per 16 rows (token, GQA head), its four waves splitting the keys and
-    // merging through LDS; a decode also splits each row block's keys over `pieces`
+    // merging through LDS, which also splits each row block's keys over `pieces`
     // workgroups when the grid would leave compute units idle, merged by a second kernel
     AnyArgs g{};
     g.q = a.q; g.q_stride_tok = a.q_stride_tok; g.q_stride_head = a.q_stride_head;
@@ -1214,7 +1214,7 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
     g.pieces = 1;
     const int64_t base = (int64_t)a.batch * a.hkv * g.row_blocks;  // one workgroup per row block
     const int64_t cap_slots = (int64_t)num_workgroups * kPieceWgPerCu;
-    if (decode && base < num_workgroups && workspace && workspace_bytes >= any_piece_bytes(cap_slots, head_dim) &&
+    if (base < num_workgroups && workspace && workspace_bytes >= any_piece_bytes(cap_slots, head_dim) &&
         !(reinterpret_cast<uintptr_t>(workspace) & 255)) {
       // pieces: enough workgroups to cover the chip twice, no more than one 16-key tile per
       // wave at the longest length known (the caller's bound, else the table's width),
@@ -1223,9 +1223,11 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
       const int64_t width = max_seq_len > 0 ? (int64_t)max_seq_len : (a.tt.stride << a.tt.page_shift);
       const int64_t by_len = (width + kAnyWaves * kAnyKeys - 1) / (kAnyWaves * kAnyKeys);
       const int64_t want = (cap_slots + base - 1) / base;
-      const int64_t pieces = width > kPieceMinKeys ? std::min(std::min(want, by_len), cap_slots / base) : 1;
+      const int64_t pieces =
+          width > kPieceMinKeys ? std::min(std::min(want, by_len), std::min<int64_t>(cap_slots / base, kAnyMaxPieces)) : 1;
       if (pieces > 1) {
         g.pieces = (int)pieces;
+        g.merge_rows = decode ? std::min(kAnyRows, a.group) : kAnyRows;  // a verify may have more rows than its hint
         char* ws = reinterpret_cast<char*>(workspace);
         g.part_o = reinterpret_cast<float*>(ws);
         g.part_lse = reinterpret_cast<float*>(ws + any_piece_o_bytes(cap_slots, head_dim));
@@ -1297,14 +1299,14 @@ extern "C" int ma_grouped_decode(
                      (hipStream_t)stream);
 }
 
-extern "C" int ma_paged_verify(
+extern "C" int ma_paged_verify_bounded(
     const void* q, int64_t q_stride_tok, int64_t q_stride_head, int q_dtype, int64_t num_tokens,
     const void* k_cache, const void* v_cache, int64_t kv_stride_row, int64_t kv_stride_head, int kv_dtype,
     const int32_t* table, int64_t table_stride, const int64_t* row_index, int page_size,
     const int32_t* seq_lens, const int32_t* query_start_loc, const int32_t* prefix_lens,
     int batch, int max_q_per_seq, int num_q_heads, int num_kv_heads, int head_dim,
     int causal, int sliding_window, int num_workgroups,
-    float softmax_scale, float k_scale, float v_scale, void* workspace, size_t workspace_bytes,
+    float softmax_scale, float k_scale, float v_scale, int max_seq_len, void* workspace, size_t workspace_bytes,
     void* out, int out_dtype, int64_t out_stride_tok, int64_t out_stride_head, void* stream) {
   if ((q_dtype == DT_F16 || q_dtype == DT_BF16) && out_dtype != q_dtype && out_dtype != DT_F32)
     return set_error(MA_EINVAL, "out dtype %d must be the query dtype or f32", out_dtype);
@@ -1323,8 +1325,24 @@ extern "C" int ma_paged_verify(
   a.scale_log2 = softmax_scale * k_scale * kLog2e; a.v_scale = v_scale;
   a.out = out; a.out_stride_tok = out_stride_tok; a.out_stride_head = out_stride_head;
   a.out_f32 = out_dtype == DT_F32;
-  return splitkv_run(a, head_dim, q_dtype, kv_dtype, max_q_per_seq, num_workgroups, 0, workspace, workspace_bytes,
+  return splitkv_run(a, head_dim, q_dtype, kv_dtype, max_q_per_seq, num_workgroups, max_seq_len, workspace, workspace_bytes,
                      (hipStream_t)stream);
+}
+
+extern "C" int ma_paged_verify(
+    const void* q, int64_t q_stride_tok, int64_t q_stride_head, int q_dtype, int64_t num_tokens,
+    const void* k_cache, const void* v_cache, int64_t kv_stride_row, int64_t kv_stride_head, int kv_dtype,
+    const int32_t* table, int64_t table_stride, const int64_t* row_index, int page_size,
+    const int32_t* seq_lens, const int32_t* query_start_loc, const int32_t* prefix_lens,
+    int batch, int max_q_per_seq, int num_q_heads, int num_kv_heads, int head_dim,
+    int causal, int sliding_window, int num_workgroups,
+    float softmax_scale, float k_scale, float v_scale, void* workspace, size_t workspace_bytes,
+    void* out, int out_dtype, int64_t out_stride_tok, int64_t out_stride_head, void* stream) {
+  return ma_paged_verify_bounded(q, q_stride_tok, q_stride_head, q_dtype, num_tokens, k_cache, v_cache, kv_stride_row,
+                                 kv_stride_head, kv_dtype, table, table_stride, row_index, page_size, seq_lens,
+                                 query_start_loc, prefix_lens, batch, max_q_per_seq, num_q_heads, num_kv_heads, head_dim,
+                                 causal, sliding_window, num_workgroups, softmax_scale, k_scale, v_scale, 0, workspace,
+                                 workspace_bytes, out, out_dtype, out_stride_tok, out_stride_head, stream);
 }
 
 extern "C" int ma_grouped_decode_noalloc(

@@ -1,0 +1,87 @@
+"""Verify and decode calls of few sequences, whose keys are split over many waves: pieces of
+a workgroup merged in LDS and long piece lists (split-KV kernel), and key pieces with their
+merge (any-head-dim kernel), against float64."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import torch_f64
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+BF16, F16, E4M3, E5M2 = torch.bfloat16, torch.float16, torch.float8_e4m3fn, torch.float8_e5m2
+
+CASES = [  # prefix, new tokens, heads, kv heads, dim, q dtype, kv dtype, window, hint of the longest chain
+    # split-KV: one sequence (every workgroup inside one segment), two row blocks at D = 256
+    ([9000], [4], 12, 2, 256, BF16, E5M2, -1, 4),
+    ([9000], [4], 12, 2, 256, F16, F16, -1, 4),
+    ([5000, 0, 3], [4, 1, 0], 16, 4, 256, BF16, BF16, -1, 4),
+    ([7000, 40], [3, 7], 12, 2, 256, BF16, E4M3, 900, 7),
+    ([9000], [4], 32, 8, 128, BF16, BF16, -1, 4),
+    ([700, 9000, 12], [5, 5, 5], 40, 8, 128, F16, E4M3, -1, 5),
+    ([4000], [4], 8, 1, 64, BF16, E5M2, -1, 4),
+    ([3, 5, 2], [1, 2, 3], 8, 8, 128, BF16, BF16, -1, 3),          # fewer tiles than a workgroup has waves
+    ([31] * 70, [2] * 70, 8, 2, 128, F16, F16, -1, 2),             # over 64 sequences: two scans
+    # any-head-dim pieces: rows within and past the hint, empty sequences, windows
+    ([6000], [4], 16, 4, 512, BF16, BF16, -1, 4),
+    ([6000, 0, 70], [4, 3, 0], 16, 4, 512, F16, F16, -1, 4),
+    ([3000], [9], 8, 2, 512, BF16, E4M3, -1, 2),
+    ([3000, 100], [6, 2], 32, 8, 96, BF16, E5M2, 500, 6),
+    ([3000], [4], 16, 4, 192, F16, F16, -1, 4),
+    ([2500], [5], 6, 1, 48, BF16, BF16, -1, 5),
+    ([2500], [40], 8, 2, 320, BF16, BF16, -1, 8),
+]
+
+
+@pytest.mark.parametrize("hinted", [True, False])
+@pytest.mark.parametrize("prefix,new,heads,hkv,dim,q_dtype,kv,window,hint", CASES)
+def test_verify_matches_float64(prefix, new, heads, hkv, dim, q_dtype, kv, window, hint, hinted):
+    from sglang_restomod_amd.attention.mi355x import ops
+
+    print(f"[case] verify split prefix={prefix[:4]} new={new[:4]} h={heads}/{hkv} d={dim} q={q_dtype} kv={kv} "
+          f"window={window} hint={hint} hinted={hinted}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(11)
+    seq = [p + n for p, n in zip(prefix, new)]
+    slots = sum(seq) + 1
+    perm = torch.randperm(slots - 1, generator=g, device=DEV) + 1
+    table = torch.zeros(len(seq), max(seq) + 3, dtype=torch.int32, device=DEV)
+    off = 0
+    for b, n in enumerate(seq):
+        table[b, :n] = perm[off:off + n].to(torch.int32)
+        off += n
+    k, v = (torch.randn(slots, hkv, dim, generator=g, device=DEV).to(kv) for _ in range(2))
+    q = (3 * torch.randn(sum(new), heads, dim, generator=g, device=DEV)).to(q_dtype)
+    qsl = [sum(new[:i]) for i in range(len(new) + 1)]
+    i32 = dict(dtype=torch.int32, device=DEV)
+    out = torch.full(q.shape, float("nan"), dtype=torch.float32, device=DEV)
+    ops.paged_verify_forward(
+        q, k, v, table, torch.tensor(seq, **i32), torch.tensor(qsl, **i32), torch.tensor(prefix, **i32),
+        max_q_per_seq=hint, softmax_scale=dim ** -0.5, k_scale=0.5, v_scale=2.0, sliding_window_size=window, out=out,
+        page_size=1, max_seq_len_hint=max(seq) if hinted else None)
+    torch.cuda.synchronize()
+    ref = torch_f64.attend(q, k.float(), v.float(), [table[b] for b in range(len(seq))], qsl, prefix, seq,
+                           softmax_scale=dim ** -0.5, k_scale=0.5, v_scale=2.0, sliding_window=window)
+    # 2e-3 is the repository's bound for v_scale near 1
+    assert float((out.double() - ref).abs().max()) < 4e-3
+
+
+@pytest.mark.parametrize("heads,hkv,dim,kv", [(8, 1, 128, BF16), (12, 2, 256, E4M3), (16, 4, 512, F16), (5, 1, 80, BF16)])
+def test_decode_of_one_long_sequence(heads, hkv, dim, kv):
+    """Hundreds of key pieces of one row block: more than one round of the merge's loads."""
+    from sglang_restomod_amd.attention.mi355x import ops
+
+    print(f"[case] decode pieces h={heads}/{hkv} d={dim} kv={kv}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    n = 33001
+    table = (torch.randperm(n, generator=g, device=DEV) + 1).to(torch.int32).view(1, n)
+    k, v = (torch.randn(n + 1, hkv, dim, generator=g, device=DEV).to(kv) for _ in range(2))
+    q = (3 * torch.randn(1, heads, dim, generator=g, device=DEV)).to(F16 if kv == F16 else BF16)
+    out = torch.empty(q.shape, dtype=torch.float32, device=DEV)
+    ops.grouped_decode_forward(q, k, v, table, torch.tensor([n], dtype=torch.int32, device=DEV),
+                               softmax_scale=dim ** -0.5, out=out, max_seq_len_hint=n, page_size=1)
+    torch.cuda.synchronize()
+    ref = torch_f64.attend(q, k.float(), v.float(), [table[0]], [0, 1], [n - 1], [n], softmax_scale=dim ** -0.5)
+    assert float((out.double() - ref).abs().max()) < 2e-3
