@@ -33,8 +33,8 @@ HEAD_DIM_MULTIPLE = 16
 
 
 # A decode with at most this many 32-key split-KV tiles (over every sequence, kv head and
-# 32-row group, at the caller's length bound) runs as key pieces on the any-head-dim kernel
-# (MA_SMALL_DECODE_TILES in csrc/splitkv.hip).
+# 32-row group, at the caller's length bound; a tile of 256 dims counts twice) runs as key
+# pieces on the any-head-dim kernel (MA_SMALL_DECODE_TILES in csrc/splitkv.hip).
 SMALL_DECODE_TILES = 16384
 
 
@@ -49,7 +49,7 @@ def decode_kernel(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int
         return "splitkv_partial"
     group = int(num_q_heads) // int(num_kv_heads)
     tiles = int(batch) * int(num_kv_heads) * ((group + 31) // 32) * ((int(max_seq_len_hint) + 31) // 32)
-    return "any_kernel" if tiles <= SMALL_DECODE_TILES else "splitkv_partial"
+    return "any_kernel" if tiles * (2 if int(head_dim) > 128 else 1) <= SMALL_DECODE_TILES else "splitkv_partial"
 
 
 def head_dim_supported(head_dim: int) -> bool:

@@ -1110,7 +1110,10 @@ extern "C" size_t ma_splitkv_workspace_bytes(int num_workgroups, int head_dim) {
 // cost more than they save. Measured at D = 128, 32 / 8 heads, B 1-32 and contexts of
 // 512-8192: the pieces are faster up to 16384 tiles (B = 8 at 8192 keys: 51.8 against
 // 61.5 us per call; B = 32 at 2048: 45.6 against 59.4) and slower beyond (B = 16 at 8192:
-// 110 against 101); B = 1 at 512 keys takes 16.5 us per call either way.
+// 110 against 101); B = 1 at 512 keys takes 16.5 us per call either way. A tile of 256
+// dims counts twice: 12 / 2 heads 4 x 22k keys (5.6k tiles) 27 against 34 us, 16 / 4 heads
+// 16 x 6k keys (12k tiles) 92 against 81. A verify of one 16-row block over fp16 or fp8 KV
+// is the same work: 32 / 8 heads, 16 x 1.5k keys 24.8 against 32.0 us.
 #ifndef MA_SMALL_DECODE_TILES
 #define MA_SMALL_DECODE_TILES 16384
 #endif
@@ -1190,13 +1193,14 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
   if ((int64_t)a.num_tokens * a.group > 0x7fffffff) return set_error(MA_EINVAL, "num_tokens x GQA group exceeds 2^31");
   if (max_seq_len < 0) return set_error(MA_EINVAL, "max_seq_len must be >= 0 (0: not known)");
   const bool decode = a.qsl == nullptr;
-  // a small decode: the split-KV tiles at the longest length the caller knows
+  // a small decode, or a small verify of one 16-row block: the split-KV tiles at the longest
+  // length the caller knows, in tiles of 128 dims. A verify over bf16 KV stays on the
+  // persistent kernel, which keeps P to 16 bits (two bf16 halves) and bf16 V exact.
   bool small = false;
-  if (!generic && decode && max_seq_len > 0) {
-    const int rows_total = a.group;
-    const int64_t row_groups = (rows_total + 31) / 32;
+  if (!generic && max_seq_len > 0 && (decode || (kv_dtype != DT_BF16 && (int64_t)max_q_per_seq * a.group <= kAnyRows))) {
+    const int64_t row_groups = (a.group + 31) / 32;
     const int64_t tiles = (int64_t)a.batch * a.hkv * row_groups * ((max_seq_len + 31) / 32);
-    small = tiles <= kSmallDecodeTiles;
+    small = tiles * (head_dim > 128 ? 2 : 1) <= kSmallDecodeTiles;
   }
   if (generic || small) {
     // one workgroup per 16 rows (token, GQA head), its four waves splitting the keys and
@@ -1214,7 +1218,9 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
     g.pieces = 1;
     const int64_t base = (int64_t)a.batch * a.hkv * g.row_blocks;  // one workgroup per row block
     const int64_t cap_slots = (int64_t)num_workgroups * kPieceWgPerCu;
-    if (base < num_workgroups && workspace && workspace_bytes >= any_piece_bytes(cap_slots, head_dim) &&
+    // a verify up to 128 dims (two workgroups a CU) below half the CUs only: at half of them
+    // (16 sequences of 6k keys, 8 kv heads, D = 96, e4m3) the split measured 69.5 against 64.1 us
+    if ((decode || head_dim > 128 ? base : 2 * base) < num_workgroups && workspace && workspace_bytes >= any_piece_bytes(cap_slots, head_dim) &&
         !(reinterpret_cast<uintptr_t>(workspace) & 255)) {
       // pieces: enough workgroups to cover the chip twice, no more than one 16-key tile per
       // wave at the longest length known (the caller's bound, else the table's width),
