@@ -197,6 +197,13 @@ __device__ __forceinline__ uint32_t pack_f16(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
 }
 
+// Two probabilities -> packed fp16, rounded to nearest even: after the row sum of the same
+// rounded values divides it out, truncation's error is about 5% larger.
+__device__ __forceinline__ uint32_t pack_p16(float a, float b) {
+  const f32x2 v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2));
+}
+
 // Two floats -> packed bf16 by truncation, and the two truncation remainders.
 __device__ __forceinline__ void split_bf16(float a, float b, uint32_t& hi, uint32_t& lo) {
   uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);

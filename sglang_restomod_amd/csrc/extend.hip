@@ -382,7 +382,7 @@ __global__ __launch_bounds__(kXWaves * 64, 1) void extend_kernel(const ExtendArg
   __shared__ __attribute__((aligned(1024))) unsigned char vring[S][kStageB];
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // scalar: 0.6% on the D = 128 batches
   const int c = lane & 15;
   const int j = lane >> 4;
   // Head-dim order of the QK contraction: MFMA step kk of lane group j holds dims
@@ -672,7 +672,7 @@ __global__ __launch_bounds__(kXWaves * 64, 1) void extend_kernel(const ExtendArg
 #pragma unroll
       for (int st2 = 0; st2 < HF; ++st2)
 #pragma unroll
-        for (int w = 0; w < 4; ++w) pk[rb][st2][w] = pack_f16(p[8 * st2 + 2 * w], p[8 * st2 + 2 * w + 1]);
+        for (int w = 0; w < 4; ++w) pk[rb][st2][w] = pack_p16(p[8 * st2 + 2 * w], p[8 * st2 + 2 * w + 1]);
     }
     if (__builtin_amdgcn_ballot_w64(grew)) {
 #pragma unroll

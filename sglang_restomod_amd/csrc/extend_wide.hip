@@ -13,7 +13,7 @@
 // 1,700 cycles) under 2,048 cycles of MFMA per SIMD; the tile's 32 keys are one 16x16x32
 // contraction of the PV product. The kernel before it (four waves of 16 rows, one per SIMD,
 // 16-key tiles with 16x16x16 PV MFMAs) took 1,018 us on a batch of 4 (prefixes 0-4,096, 256
-// to 2,048 new tokens, 16 / 4 heads, bf16) where this one takes 576 (630 TFLOP/s).
+// to 2,048 new tokens, 16 / 4 heads, bf16) where this one takes 460 (790 TFLOP/s).
 //
 // Numerics as in the tiled kernel: K in the query dtype (fp8 converted exactly), V and P in
 // fp16 (bf16 V converted as its fragments are read, each by one wave), fp32 accumulation,
@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kWideWaves * 64, 1) void extend_wide_kernel(const E
   __shared__ __attribute__((aligned(16))) uint32_t fbuf[2][NRB];   // row block has moved rows
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // in scalar registers, with all that derives from it
   const int c = lane & 15;
   const int j = lane >> 4;
   auto qdim = [&](int kk) -> int {  // first dim of QK step kk for lane group j (as in the tiled kernel)
@@ -110,22 +110,18 @@ __global__ __launch_bounds__(kWideWaves * 64, 1) void extend_wide_kernel(const E
   const int prefix = a.prefix ? cptr(a.prefix)[b] : seq - ntok;
   const int64_t seq_row = a.row_index ? cptr(a.row_index)[b] : (int64_t)b;
 
-  // ---- this lane's score row ----
-  const int r = r0 + wave * 16 + c;
-  const int t = r / a.group;
-  const int g = r - t * a.group;
-  const bool real = t < ntok;
-  const int qpos = prefix + t;
-  const int lo_r = (real && a.window >= 0) ? max(0, qpos - a.window) : 0;
-  const int hi_r = real ? (a.causal ? min(seq, qpos + 1) : seq) : 0;
+  // ---- Q of this lane's score row (row c of the wave's block) ----
   u32x4 qv[KK];
   {
+    const int r = r0 + wave * 16 + c;
+    const int t = r / a.group;
+    const int g = r - t * a.group;
     const uint16_t MA_GLOBAL* qp = gptr(reinterpret_cast<const uint16_t*>(a.q)) + (int64_t)(tok0 + t) * a.q_stride_tok +
                                    (int64_t)(h * a.group + g) * a.q_stride_head;
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk)
-      qv[kk] = (real && qdim(kk) < a.head_dim) ? *reinterpret_cast<const u32x4 MA_GLOBAL*>(qp + qdim(kk))
-                                               : u32x4{0, 0, 0, 0};
+      qv[kk] = (t < ntok && qdim(kk) < a.head_dim) ? *reinterpret_cast<const u32x4 MA_GLOBAL*>(qp + qdim(kk))
+                                                   : u32x4{0, 0, 0, 0};
   }
   // waited for here, once (the compiler cannot count the inline-assembly loads below)
 #pragma unroll
@@ -225,25 +221,40 @@ __global__ __launch_bounds__(kWideWaves * 64, 1) void extend_wide_kernel(const E
   auto barrier = [&]() __attribute__((always_inline)) { __asm__ volatile("s_barrier" : : : "memory"); };
 
   // ---- scores of tile k from K stage st: lane (c, j) holds keys 16 kb + 4j .. + 3 of row c ----
+  // The K fragments are read kAhead before the MFMAs that use them; without the scheduling
+  // barriers the compiler put each read right before its MFMA, which then waited out the LDS
+  // latency (576 us on the D = 512 batch, 460 with them and with every wave-uniform value in scalar
+  // registers, which ended the spills).
   f32x4 s[KB];
   auto scores = [&](int st) __attribute__((always_inline)) {
-    const unsigned char* kt = kring[st] + lane * 16;
+    constexpr int kAhead = kFp8 ? 4 : 6;
+    constexpr int N = kKSub * KB;
+    int ln = lane;
+    __asm__ volatile("" : "+v"(ln));
+    const unsigned char* kt = kring[st] + ln * 16;
+    auto frag = [&](int i) __attribute__((always_inline)) -> u32x4 {  // block kb = i % KB, chunks i / KB
+      return *reinterpret_cast<const u32x4*>(kt + ((i % KB) * kKSub + i / KB) * 1024);
+    };
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) s[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    u32x4 kf[kAhead];
 #pragma unroll
-    for (int sub = 0; sub < kKSub; ++sub)
+    for (int i = 0; i < kAhead; ++i) kf[i] = frag(i);
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        const u32x4 kf = *reinterpret_cast<const u32x4*>(kt + (kb * kKSub + sub) * 1024);
-        if constexpr (kFp8) {
-          u32x4 k0, k1;
-          cvt16_fp8<KV, QBF16>(kf, k0, k1);
-          s[kb] = mfma16t<QBF16>(k0, qv[2 * sub], s[kb]);
-          s[kb] = mfma16t<QBF16>(k1, qv[2 * sub + 1], s[kb]);
-        } else {
-          s[kb] = mfma16t<QBF16>(kf, qv[sub], s[kb]);
-        }
+    for (int i = 0; i < N; ++i) {
+      __builtin_amdgcn_sched_barrier(0);
+      const int kb = i % KB, sub = i / KB;
+      if constexpr (kFp8) {
+        u32x4 k0, k1;
+        cvt16_fp8<KV, QBF16>(kf[i % kAhead], k0, k1);
+        s[kb] = mfma16t<QBF16>(k0, qv[2 * sub], s[kb]);
+        s[kb] = mfma16t<QBF16>(k1, qv[2 * sub + 1], s[kb]);
+      } else {
+        s[kb] = mfma16t<QBF16>(kf[i % kAhead], qv[sub], s[kb]);
       }
+      if (i + kAhead < N) kf[i % kAhead] = frag(i + kAhead);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   };
   // ---- softmax of tile k; P, and the factors of rows whose base moved, to LDS half pk ----
   auto softmax = [&](int k, int pk) __attribute__((always_inline)) {
@@ -251,6 +262,12 @@ __global__ __launch_bounds__(kWideWaves * 64, 1) void extend_wide_kernel(const E
     int ln = lane;
     __asm__ volatile("" : "+v"(ln));
     if (!(base >= full_lo && base + BN <= full_hi)) {
+      // the lane's visible keys, computed again on the few masked tiles: its row's bounds kept
+      // through the loop would spill
+      const int t = (r0 + wave * 16 + (ln & 15)) / a.group;
+      const int qpos = prefix + t;
+      const int lo_r = a.window >= 0 ? qpos - a.window : 0;
+      const int hi_r = t < ntok ? (a.causal ? min(seq, qpos + 1) : seq) : 0;
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
@@ -263,8 +280,9 @@ __global__ __launch_bounds__(kWideWaves * 64, 1) void extend_wide_kernel(const E
                      max3f(s[1][2], s[1][3], -INFINITY));
     const bool moved = __builtin_amdgcn_ballot_w64((mx - m_run) * a.scale_log2 > kLazyRescale) != 0;
     if (moved) {
-      mx = fmaxf(mx, shfl_xor_f(mx, 16));
-      mx = fmaxf(mx, shfl_xor_f(mx, 32));
+      const int sw = ln << 2;  // byte index of the lane for the cross-lane reads
+      mx = fmaxf(mx, __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(sw ^ 64, __builtin_bit_cast(int, mx))));
+      mx = fmaxf(mx, __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(sw ^ 128, __builtin_bit_cast(int, mx))));
       const float m_new = fmaxf(m_run, mx);
       const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
       const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * a.scale_log2);
@@ -281,7 +299,7 @@ __global__ __launch_bounds__(kWideWaves * 64, 1) void extend_wide_kernel(const E
       for (int w = 0; w < 2; ++w) {
         const float p0 = __builtin_amdgcn_exp2f(s[kb][2 * w] * a.scale_log2 - msc);
         const float p1 = __builtin_amdgcn_exp2f(s[kb][2 * w + 1] * a.scale_log2 - msc);
-        const uint32_t pw = pack_f16(p0, p1);
+        const uint32_t pw = pack_p16(p0, p1);
         pf[2 * kb + w] = pw;
         // the row sum takes the rounded p, so that rounding cancels in the quotient
         const f16x2 one = {(_Float16)1.f, (_Float16)1.f};
@@ -297,6 +315,12 @@ __global__ __launch_bounds__(kWideWaves * 64, 1) void extend_wide_kernel(const E
     int ln = lane;
     __asm__ volatile("" : "+v"(ln));
     const uint32_t vl = v_first(ln);
+    uint32_t fl = 0;
+#pragma unroll
+    for (int rb = 0; rb < NRB; rb += 4) {
+      const u32x4 f = *reinterpret_cast<const u32x4*>(&fbuf[pk][rb]);
+      fl |= f[0] | f[1] | f[2] | f[3];
+    }
     const unsigned char* vt = vring[st];
     u32x4 va[DB];
 #pragma unroll
@@ -321,27 +345,24 @@ __global__ __launch_bounds__(kWideWaves * 64, 1) void extend_wide_kernel(const E
         }
       }
     }
-    uint32_t fl = 0;
-#pragma unroll
-    for (int rb = 0; rb < NRB; rb += 4) {
-      const u32x4 f = *reinterpret_cast<const u32x4*>(&fbuf[pk][rb]);
-      fl |= f[0] | f[1] | f[2] | f[3];
-    }
+    u32x4 pf[2] = {pbuf[pk][0][ln], pbuf[pk][1][ln]};
     if (__builtin_amdgcn_readfirstlane(fl)) {
 #pragma unroll
       for (int rb = 0; rb < NRB; ++rb) {
         if (__builtin_amdgcn_readfirstlane(fbuf[pk][rb])) {
-          const float al = abuf[pk][rb * 16 + c];
+          const float al = abuf[pk][rb * 16 + (ln & 15)];
 #pragma unroll
           for (int db = 0; db < DB; ++db) o[rb][db] *= al;
         }
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int rb = 0; rb < NRB; ++rb) {
-      const u32x4 pf = pbuf[pk][rb][lane];
+    for (int rb = 0; rb < NRB; ++rb) {  // P fragments two row blocks ahead
 #pragma unroll
-      for (int db = 0; db < DB; ++db) o[rb][db] = mfma16t<false>(va[db], pf, o[rb][db]);
+      for (int db = 0; db < DB; ++db) o[rb][db] = mfma16t<false>(va[db], pf[rb & 1], o[rb][db]);
+      if (rb + 2 < NRB) pf[rb & 1] = pbuf[pk][rb + 2][ln];
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
@@ -385,26 +406,29 @@ __global__ __launch_bounds__(kWideWaves * 64, 1) void extend_wide_kernel(const E
   }
 
   // ---- epilogue: row sums meet in LDS, then each wave stores its dims of every row ----
+  int ln = lane;
+  __asm__ volatile("" : "+v"(ln));
+  const int lc = ln & 15;
   float lt = lsum + shfl_xor_f(lsum, 16);
   lt += shfl_xor_f(lt, 32);
   __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   barrier();  // every wave is past its last read of abuf
-  if (j == 0) abuf[0][wave * 16 + c] = lt;
+  if (ln < 16) abuf[0][wave * 16 + lc] = lt;
   __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   barrier();
-  if (piece_slot >= 0 && real && j == 0) {
-    const int64_t prow = ((int64_t)piece_slot * a.hkv + h) * BM + wave * 16 + c;
+  if (piece_slot >= 0 && ln < 16 && (r0 + wave * 16 + lc) / a.group < ntok) {
+    const int64_t prow = ((int64_t)piece_slot * a.hkv + h) * BM + wave * 16 + lc;
     gptr_mut(a.pieces.lse)[prow] = (lt > 0.f) ? __builtin_amdgcn_logf(lt) + m_run * a.scale_log2 : -INFINITY;
   }
 #pragma unroll
   for (int rb = 0; rb < NRB; ++rb) {
-    const int R = r0 + rb * 16 + c;
+    const int R = r0 + rb * 16 + lc;
     const int tr = R / a.group;
     if (tr >= ntok) continue;
-    const float l = abuf[0][rb * 16 + c];
-    const int d0 = wave * DW + 4 * j;
+    const float l = abuf[0][rb * 16 + lc];
+    const int d0 = wave * DW + 4 * (ln >> 4);
     if (piece_slot >= 0) {
-      const int64_t prow = ((int64_t)piece_slot * a.hkv + h) * BM + rb * 16 + c;
+      const int64_t prow = ((int64_t)piece_slot * a.hkv + h) * BM + rb * 16 + lc;
       const float inv = (l > 0.f) ? 1.f / l : 0.f;
 #pragma unroll
       for (int db = 0; db < DB; ++db)
