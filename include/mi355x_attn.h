@@ -270,6 +270,19 @@ int ma_translate_slots(const int32_t* table, int64_t table_stride, const int64_t
                        int32_t* out, int64_t out_stride, int width, void* stream);
 
 /*
+ * Lengths of an extend or verify batch in the types the attention calls take, on the device
+ * (replaces flash_attn_v100_backend.py:440-470's tensor operations):
+ *   seq_out[b] = max(seq_lens[b], prefix_lens[b] + extend[b])   (seq_lens NULL: the sum)
+ *   prefix_out[b] = prefix_lens[b] (prefix_out may be NULL)
+ *   query_start_loc[0] = 0, query_start_loc[b + 1] = extend[0] + .. + extend[b]
+ * extend[b] is extend_lens[b], or extend_const when extend_lens is NULL. Inputs are int32,
+ * or int64 where their flag is nonzero; outputs int32 [batch], [batch], [batch + 1].
+ */
+int ma_extend_lengths(const void* seq_lens, int seq_is_64, const void* extend_lens, int extend_is_64,
+                      int extend_const, const void* prefix_lens, int prefix_is_64, int batch, int32_t* seq_out,
+                      int32_t* prefix_out, int32_t* query_start_loc, void* stream);
+
+/*
  * Key rows of a multi-step speculative draft, on the device.
  * Replaces the per-step draft KV-index build of the reference's draft container
  * (draft_decode.py:172-208, the engine container's common_template)

@@ -84,6 +84,11 @@ SIGNATURES = {
         c_void_p, c_int64,                            # mapping, mapping_len
         c_void_p, c_int64, c_int, c_void_p,           # out, stride, width, stream
     ]),
+    "ma_extend_lengths": (c_int, [
+        c_void_p, c_int, c_void_p, c_int, c_int,      # seq_lens, is64, extend_lens, is64, extend_const
+        c_void_p, c_int, c_int,                       # prefix_lens, is64, batch
+        c_void_p, c_void_p, c_void_p, c_void_p,       # seq_out, prefix_out, query_start_loc, stream
+    ]),
     "ma_draft_table": (c_int, [
         c_void_p, c_int64, c_int, c_void_p,           # table, stride, width, row_index
         c_void_p, c_int, c_int, c_int,                # seq_lens, batch, topk, num_steps

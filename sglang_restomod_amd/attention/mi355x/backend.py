@@ -180,20 +180,26 @@ class MI355XAttnBackend(_EngineBase):
         seq_lens_cpu=None,
     ) -> MI355XForwardMetadata:
         row_index = req_pool_indices.to(torch.int64)
-        seq = seq_lens.to(torch.int32)
+        native = mode != MODE_DECODE and seq_lens.is_cuda
+        seq = seq_lens if native else seq_lens.to(torch.int32)
         md = MI355XForwardMetadata(mode=mode, table=self.req_to_token, row_index=row_index, seq_lens=seq)
         if seq_lens_cpu is not None and len(seq_lens_cpu):
-            md.max_seq_len = max(0, int(max(int(x) for x in seq_lens_cpu)))
+            lens = seq_lens_cpu.tolist() if isinstance(seq_lens_cpu, torch.Tensor) else seq_lens_cpu
+            md.max_seq_len = max(0, int(max(lens)))
         if mode != MODE_DECODE:
-            ext = extend_seq_lens.to(torch.int32)
-            pre = extend_prefix_lens.to(torch.int32)
             # a warm-up batch may carry a decode fill value in seq_lens; prefix + extend
             # is the length the kernels must see (reference :452-455)
-            md.seq_lens = torch.maximum(seq, pre + ext)
-            md.prefix_kv_lens = pre
-            qsl = torch.zeros(seq.shape[0] + 1, dtype=torch.int32, device=seq.device)
-            torch.cumsum(ext, dim=0, dtype=torch.int32, out=qsl[1:])
-            md.query_start_loc = qsl
+            if native:
+                md.seq_lens, md.prefix_kv_lens, md.query_start_loc = ops.extend_lengths(
+                    seq, extend_seq_lens, extend_prefix_lens)
+            else:
+                ext = extend_seq_lens.to(torch.int32)
+                pre = extend_prefix_lens.to(torch.int32)
+                md.seq_lens = torch.maximum(seq, pre + ext)
+                md.prefix_kv_lens = pre
+                qsl = torch.zeros(seq.shape[0] + 1, dtype=torch.int32, device=seq.device)
+                torch.cumsum(ext, dim=0, dtype=torch.int32, out=qsl[1:])
+                md.query_start_loc = qsl
             # the extend kernel lists its row tiles on the device; only the verifier's
             # grid needs the longest chain, which callers pass (0: not known)
             md.max_q_per_seq = int(max_q_per_seq) if max_q_per_seq is not None else 0
@@ -214,10 +220,11 @@ class MI355XAttnBackend(_EngineBase):
             self._check_linear_verify()
             n = int(forward_batch.spec_info.draft_token_num)
             prefix = forward_batch.seq_lens
-            ext = torch.full_like(prefix, n)
+            # on the device the lengths come from one launch: prefix + n is its maximum's other side
+            seq, ext = (prefix, n) if prefix.is_cuda else (prefix + n, torch.full_like(prefix, n))
             cpu = None if seq_lens_cpu is None else [int(s) + n for s in seq_lens_cpu]
             self.forward_metadata = self.build_metadata(
-                MODE_VERIFY, forward_batch.req_pool_indices, prefix + n, ext, prefix,
+                MODE_VERIFY, forward_batch.req_pool_indices, seq, ext, prefix,
                 max_q_per_seq=n, seq_lens_cpu=cpu)
             return
         ext_cpu = getattr(forward_batch, "extend_seq_lens_cpu", None)

@@ -613,6 +613,37 @@ def translate_slots(
     return out
 
 
+def _lens(t: torch.Tensor) -> torch.Tensor:
+    if t.dtype not in (torch.int32, torch.int64):
+        t = t.to(torch.int64)
+    return t if t.is_contiguous() else t.contiguous()
+
+
+def extend_lengths(seq_lens: Optional[torch.Tensor], extend_lens, prefix_lens: torch.Tensor):
+    """``(seq_lens, prefix_lens, query_start_loc)`` of an extend batch as int32 device tensors,
+    in one launch: ``max(seq_lens, prefix_lens + extend_lens)`` (``seq_lens`` None: the sum),
+    the prefix lengths, and the running sum of ``extend_lens`` with a leading 0.
+    ``extend_lens``: a tensor, or one int for every sequence."""
+    pre = _lens(prefix_lens)
+    seq = None if seq_lens is None else _lens(seq_lens)
+    ext = _lens(extend_lens) if isinstance(extend_lens, torch.Tensor) else None
+    dev = _check_device(pre, seq, ext)
+    B = int(pre.shape[0])
+    if (seq is not None and seq.shape[0] != B) or (ext is not None and ext.shape[0] != B):
+        raise ValueError("the lengths must have one entry per sequence")
+    wide = torch.int64
+    pad = (B + 63) & ~63  # each result 256-byte aligned
+    buf = torch.empty(2 * pad + B + 1, dtype=torch.int32, device=dev)
+    seq_out, qsl = buf[:B], buf[2 * pad:]
+    pre_out = pre if pre.dtype == torch.int32 else buf[pad:pad + B]
+    status = _lib.load().ma_extend_lengths(
+        _ptr(seq), seq is not None and seq.dtype == wide, _ptr(ext), ext is not None and ext.dtype == wide,
+        0 if ext is not None else int(extend_lens), pre.data_ptr(), pre.dtype == wide, B, seq_out.data_ptr(),
+        None if pre_out is pre else pre_out.data_ptr(), qsl.data_ptr(), _stream_ptr(dev))
+    _lib.check(status, "ma_extend_lengths")
+    return seq_out, pre_out, qsl
+
+
 def draft_table(
     table: torch.Tensor,
     seq_lens: torch.Tensor,

@@ -104,6 +104,69 @@ __global__ __launch_bounds__(kXlateThreads) void draft_table_kernel(const DraftT
   }
 }
 
+// ---- lengths of an extend or verify batch ----
+// The engine's lengths (int32 or int64) as the kernels read them, in one launch where the
+// torch operations took five (conversions, prefix + extend, maximum, zeros, cumsum: 22 us
+// of device time and 25 us of host time per forward; this kernel 4.8 us). One workgroup:
+// 1024 sequences per pass, an inclusive scan over waves of DPP scans.
+struct LengthsArgs {
+  const void* seq;     // or null: prefix + extend
+  const void* extend;  // or null: extend_const each
+  const void* prefix;
+  int seq64, extend64, prefix64;
+  int extend_const;
+  int batch;
+  int32_t* seq_out;     // max(seq, prefix + extend)
+  int32_t* prefix_out;  // or null
+  int32_t* qsl_out;     // [batch + 1]
+};
+constexpr int kLenThreads = 1024;
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int len_dpp(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false);
+}
+
+__global__ __launch_bounds__(kLenThreads) void lengths_kernel(const LengthsArgs a) {
+  __shared__ int sums[kLenThreads / 64];
+  const int tid = threadIdx.x;
+  const int wave = tid >> 6;
+  auto get = [&](const void* p, int is64, int b) -> int {
+    return is64 ? (int)gptr(reinterpret_cast<const int64_t*>(p))[b] : gptr(reinterpret_cast<const int32_t*>(p))[b];
+  };
+  int carry = 0;
+  if (tid == 0) gptr_mut(a.qsl_out)[0] = 0;
+  for (int b0 = 0; b0 < a.batch; b0 += kLenThreads) {
+    const int b = b0 + tid;
+    int ext = 0;
+    if (b < a.batch) {
+      ext = a.extend ? get(a.extend, a.extend64, b) : a.extend_const;
+      const int pre = get(a.prefix, a.prefix64, b);
+      const int n = pre + ext;
+      gptr_mut(a.seq_out)[b] = a.seq ? max(get(a.seq, a.seq64, b), n) : n;
+      if (a.prefix_out) gptr_mut(a.prefix_out)[b] = pre;
+    }
+    int x = ext;
+    x += len_dpp<0x111, 0xf>(x);  // row_shr:1, 2, 4, 8, then row_bcast:15 and 31
+    x += len_dpp<0x112, 0xf>(x);
+    x += len_dpp<0x114, 0xf>(x);
+    x += len_dpp<0x118, 0xf>(x);
+    x += len_dpp<0x142, 0xa>(x);
+    x += len_dpp<0x143, 0xc>(x);
+    if ((tid & 63) == 63) sums[wave] = x;
+    __syncthreads();
+    int before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < kLenThreads / 64; ++w) {
+      before += w < wave ? sums[w] : 0;
+      all += sums[w];
+    }
+    __syncthreads();  // sums is free for the next pass
+    if (b < a.batch) gptr_mut(a.qsl_out)[b + 1] = carry + before + x;
+    carry += all;
+  }
+}
+
 }  // namespace ma
 
 using namespace ma;
@@ -146,5 +209,22 @@ extern "C" int ma_draft_table(const int32_t* table, int64_t table_stride, int ta
   hipLaunchKernelGGL(draft_table_kernel, grid, dim3(kXlateThreads), 0, (hipStream_t)stream, a);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(MA_ELAUNCH, "draft table launch failed: %s", hipGetErrorString(e));
+  return MA_OK;
+}
+
+extern "C" int ma_extend_lengths(const void* seq_lens, int seq_is_64, const void* extend_lens, int extend_is_64,
+                                 int extend_const, const void* prefix_lens, int prefix_is_64, int batch,
+                                 int32_t* seq_out, int32_t* prefix_out, int32_t* query_start_loc, void* stream) {
+  if (batch < 0) return set_error(MA_EINVAL, "batch %d must be >= 0", batch);
+  if (!query_start_loc) return set_error(MA_EINVAL, "null pointer argument");
+  if (batch > 0 && (!prefix_lens || !seq_out)) return set_error(MA_EINVAL, "null pointer argument");
+  LengthsArgs a{};
+  a.seq = seq_lens; a.extend = extend_lens; a.prefix = prefix_lens;
+  a.seq64 = seq_is_64; a.extend64 = extend_is_64; a.prefix64 = prefix_is_64;
+  a.extend_const = extend_const; a.batch = batch;
+  a.seq_out = seq_out; a.prefix_out = prefix_out; a.qsl_out = query_start_loc;
+  hipLaunchKernelGGL(lengths_kernel, dim3(1), dim3(kLenThreads), 0, (hipStream_t)stream, a);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return set_error(MA_ELAUNCH, "extend lengths launch failed: %s", hipGetErrorString(e));
   return MA_OK;
 }

@@ -156,3 +156,26 @@ def test_fp8_gather_rejects_a_16_bit_cache():
     with pytest.raises(ValueError, match="E4M3 or E5M2"):
         _ops().gather_fp8_paged_kv(x, x, torch.zeros(1, 1, dtype=torch.int32, device=DEV),
                                    torch.ones(1, dtype=torch.int32, device=DEV), x, x)
+
+
+@pytest.mark.parametrize("batch", [0, 1, 63, 64, 65, 1023, 1024, 1025, 3000])
+@pytest.mark.parametrize("dtypes", [(torch.int64, torch.int32, torch.int32), (torch.int32, torch.int64, torch.int64)])
+def test_extend_lengths_match_torch(batch, dtypes):
+    """One launch against the tensor operations it replaces: whole numbers, both input types,
+    the edges of the scan's passes, a constant extend and strided inputs."""
+    from sglang_restomod_amd.attention.mi355x import ops
+
+    print(f"[case] extend lengths batch={batch} {dtypes}", flush=True)
+    g = torch.Generator().manual_seed(batch)
+    seq, ext, pre = (torch.randint(0, hi, (2 * batch,), generator=g).to("cuda:0", dt)[::2]
+                     for hi, dt in zip((5000, 70, 4000), dtypes))
+    for extend in (ext, 4):
+        e = ext if extend is ext else torch.full_like(pre, 4)
+        for s in (seq, None):
+            got_seq, got_pre, qsl = ops.extend_lengths(s, extend, pre)
+            want = (pre + e).to(torch.int32)
+            if s is not None:
+                want = torch.maximum(s.to(torch.int32), want)
+            assert got_seq.dtype == got_pre.dtype == qsl.dtype == torch.int32
+            assert torch.equal(got_seq, want) and torch.equal(got_pre, pre.to(torch.int32))
+            assert qsl.tolist() == [0] + torch.cumsum(e.to(torch.int64), 0).tolist()
