@@ -460,7 +460,6 @@ def _roofline(r, kernel, bound_hbm):
                   + (("any-head-dim kernel; above 512 keys per row over key pieces + merge" if r["mode"] == "decode"
                       else "any-head-dim kernel")
                      if kernel == "any_kernel" and bound_hbm
-                     else "any-head-dim kernel, after the work-list plan" if kernel == "any_kernel"
                      else "split-KV partial + merge" if bound_hbm else "plan + extend kernel") + ")",
     }
     if bound_hbm:
@@ -554,11 +553,11 @@ def main():
         ter = 0 if args.no_cpu_baseline else args.cpu_seconds_tertiary
         line["kv_write"] = _measure_kv_write(steps, args.warmup, ter)
         # the other head dims of the reference's tuned configurations: 256 on the split-KV and
-        # tiled extend kernels, 512 on the any-head-dim kernel
+        # tiled extend kernels, 512 on the any-head-dim (decode) and wide extend kernels
         line["head_dim_256"] = {"decode": _family(_measure(5, steps, args.warmup, ter), "splitkv_partial", True),
                                 "extend": _family(_measure(6, steps, args.warmup, ter), "extend_kernel", False)}
         line["head_dim_512"] = {"decode": _family(_measure(7, steps, args.warmup, ter), "any_kernel", True),
-                                "extend": _family(_measure(8, steps, args.warmup, ter), "any_kernel", False)}
+                                "extend": _family(_measure(8, steps, args.warmup, ter), "extend_wide_kernel", False)}
         # head dims without a tiled kernel of their own, padded onto the next one
         line["padded_head_dims"] = {"d96_extend": _family(_measure(9, steps, args.warmup, ter), "extend_kernel", False),
                                     "d192_extend": _family(_measure(10, steps, args.warmup, ter), "extend_kernel", False)}

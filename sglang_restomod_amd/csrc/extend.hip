@@ -17,7 +17,8 @@
 // first (a longest-processing-time order over the CUs), so no host-side maximum of the
 // query lengths is needed. The extend grid is 1-D, (list entry) x (kv head) with the kv
 // head fastest: workgroup i runs on XCD i % 8, so with 8 kv heads each XCD streams one
-// head's K/V through its own L2.
+// head's K/V through its own L2. A call with at most one row tile per CU may have its row
+// tiles cut into key pieces (extend.h), planned in the workgroups or by the plan kernel.
 //
 // Per 64-key tile, per wave (scores of all its keys, then one online-softmax update, then
 // PV), MFMA 16x16x32 with fp32 accumulate; the softmax's VALU work is what bounds the
