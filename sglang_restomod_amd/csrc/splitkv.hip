@@ -1252,7 +1252,14 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
     return MA_OK;
   }
   const int rows_total = max_q_per_seq * a.group;
-  const int nb = rows_total <= 16 ? 1 : 2;
+  // Two row blocks per group read K and V once for all rows. Over fp8 KV at D = 256 that
+  // kernel is long, and up to two tiles per wave at the caller's bound one-block groups end
+  // first. Per call, one block against two (12 / 2 heads, 4 rows, e5m2): 16 sequences of 190
+  // keys 20.0 / 22.8 us, 4 of 6k 27.5 / 29.4, one of 22k 35.7 / 41.7; beyond, 16 of 6k 43.9 /
+  // 43.4 and 64 of 1.5k 45.7 / 45.4.
+  const bool few256 = head_dim == 256 && kv_dtype >= DT_E4M3 && max_seq_len > 0 &&
+                      (int64_t)a.batch * a.hkv * ((max_seq_len + 31) / 32) <= (int64_t)num_workgroups * kWaves * 2;
+  const int nb = rows_total <= 16 || few256 ? 1 : 2;
   a.rows = 16 * nb;
   a.row_groups = (rows_total + a.rows - 1) / a.rows;
   a.nwaves = num_workgroups * kWaves;

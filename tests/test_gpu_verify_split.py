@@ -20,6 +20,7 @@ CASES = [  # prefix, new tokens, heads, kv heads, dim, q dtype, kv dtype, window
     ([9000], [4], 12, 2, 256, F16, F16, -1, 4),
     ([5000, 0, 3], [4, 1, 0], 16, 4, 256, BF16, BF16, -1, 4),
     ([7000, 40], [3, 7], 12, 2, 256, BF16, E4M3, 900, 7),
+    ([9000] * 5 + [30], [4] * 6, 12, 2, 256, BF16, E5M2, -1, 4),    # past the one-block rule at D = 256
     ([9000], [4], 32, 8, 128, BF16, BF16, -1, 4),
     ([700, 9000, 12], [5, 5, 5], 40, 8, 128, F16, E4M3, -1, 5),
     ([4000], [4], 8, 1, 64, BF16, E5M2, -1, 4),
