@@ -30,10 +30,10 @@ struct ExtendMerge {
 };
 struct ExtendPieces {
   const ExtendPiece* list;  // the plan kernel's list, or null: each workgroup plans (plan_direct)
-  ExtendMerge* merges;
+  ExtendMerge* merges;      // the cut row tiles, then entries with sequence -1
   int merge_capacity;
   int shares;    // CUs per kv head; 0: whole row tiles from the work list
-  int capacity;  // pieces per kv head that the grid and the partial slots hold
+  int capacity;  // pieces per kv head that the list, the grid and the partial slots hold
   float* o;      // [slot][kv head][row of the tile][D] fp32
   float* lse;    // [slot][kv head][row of the tile]
 };
@@ -145,8 +145,7 @@ __device__ __forceinline__ int piece_count(int c, int cap) {
 // The piece of list position `w` (per kv head), planned by the wave itself: for batches of
 // at most kDirectItems row tiles and kDirectBatch sequences, which then need no plan kernel
 // (about 6 us of a call that takes 20). Every wave of every workgroup computes the same plan
-// from the same numbers. The first workgroup of
-// kv head 0 leave each row tile's slots in `merges`.
+// from the same numbers. The first workgroup of kv head 0 lists the cut tiles in `merges`.
 template <int BM, int BN>
 __device__ __forceinline__ ExtendPiece plan_direct(const ExtendArgs& a, int w, int h) {
   constexpr int kPer = kDirectItems / 64;
@@ -160,7 +159,7 @@ __device__ __forceinline__ ExtendPiece plan_direct(const ExtendArgs& a, int w, i
   }
   const int incl = wave_scan(nt);
   const int start = incl - nt;
-  const int m = min(__builtin_amdgcn_readlane(incl, 63), min(kDirectItems, a.pieces.merge_capacity));
+  const int m = min(__builtin_amdgcn_readlane(incl, 63), min(kDirectItems, a.pieces.capacity));
   // row tiles kPer * lane + x: their sequences and key tiles
   int b[kPer], rt[kPer], c[kPer];
   int cmax = 0, csum = 0;
@@ -236,15 +235,27 @@ __device__ __forceinline__ ExtendPiece plan_direct(const ExtendArgs& a, int w, i
   p.seq = -1;
   p.tile = p.first = p.count = 0;
   p.slot = -1;
+  if (w == 0 && h == 0 && (int)threadIdx.x < 64) {
+    int4 MA_GLOBAL* mp = reinterpret_cast<int4 MA_GLOBAL*>(gptr_mut(a.pieces.merges));
+    int ncut = 0;
+#pragma unroll
+    for (int x = 0; x < kPer; ++x) ncut += parts[x] > 1 ? 1 : 0;
+    const int upto_cut = wave_scan(ncut);
+    int e = upto_cut - ncut;
+#pragma unroll
+    for (int x = 0; x < kPer; ++x) {
+      if (parts[x] > 1 && e < a.pieces.merge_capacity) {
+        mp[e].x = b[x];
+        mp[e].y = rt[x];
+        mp[e].z = pos[x];
+        mp[e].w = parts[x];
+      }
+      e += parts[x] > 1 ? 1 : 0;
+    }
+    for (int i = __builtin_amdgcn_readlane(upto_cut, 63) + lane; i < a.pieces.merge_capacity; i += 64) mp[i].x = -1;
+  }
 #pragma unroll
   for (int x = 0; x < kPer; ++x) {
-    if (w == 0 && h == 0 && (int)threadIdx.x < 64 && kPer * lane + x < a.pieces.merge_capacity) {
-      int4 MA_GLOBAL* mp = reinterpret_cast<int4 MA_GLOBAL*>(gptr_mut(a.pieces.merges)) + kPer * lane + x;
-      mp->x = parts[x] > 1 ? b[x] : -1;
-      mp->y = rt[x];
-      mp->z = pos[x];
-      mp->w = parts[x];
-    }
     const uint64_t hit = __builtin_amdgcn_ballot_w64(w >= pos[x] && w < pos[x] + parts[x]);
     if (hit) {
       const int L = __builtin_ctzll(hit);
@@ -263,51 +274,58 @@ __device__ __forceinline__ ExtendPiece plan_direct(const ExtendArgs& a, int w, i
 }
 
 // Merge of the row tiles that were cut into key pieces: 1024 / D rows of one tile and kv
-// head per workgroup, D / 4 threads per row, four dims each. A running maximum of the log2
-// LSEs rescales the sum of the pieces' normalised O, so one pass reads each piece once
-// (four pieces' loads in flight). Pieces in which a row saw no key (LSE -inf) weigh 0.
+// head at a time per workgroup, D / 4 threads per row, four dims each. A running maximum of
+// the log2 LSEs rescales the sum of the pieces' normalised O, so one pass reads each piece
+// once (four pieces' loads in flight). Pieces in which a row saw no key (LSE -inf) weigh 0.
+// The host does not know which tiles are cut, so the grid is one the chip holds at once, and
+// its workgroups walk the listed tiles (the list ends at the first empty entry): a workgroup
+// for every row set that could be cut cost 9 us where none was (48 sequences at 32 / 32 heads).
+constexpr int kMergeGrid = 2048;  // eight workgroups of four waves on each of 256 CUs
 
 template <int D, int kBM, bool QBF16>
 __global__ __launch_bounds__(256) void extend_merge(const ExtendArgs args) {
   const ExtendArgs a = args;
   constexpr int kTPR = D / 4;              // threads per row
-  constexpr int kRows = 256 / kTPR;        // rows per workgroup
-  constexpr int kBlocks = kBM / kRows;     // workgroups per row tile and kv head
-  const int blk = (int)blockIdx.x % kBlocks;
-  const int rest = (int)blockIdx.x / kBlocks;
-  const int h = rest % a.hkv;
-  const int MA_CONST* e = cptr(reinterpret_cast<const int*>(a.pieces.merges + rest / a.hkv));
-  const int b = e[0];
-  if (b < 0) return;
-  const int rt = e[1], slot = e[2], parts = e[3];
-  const QueryRows qr = clamp_query_rows(cptr(a.qsl)[b], cptr(a.qsl)[b + 1], a.num_tokens);
+  constexpr int kRows = 256 / kTPR;        // rows per step of a workgroup
+  constexpr int kBlocks = kBM / kRows;     // steps per row tile and kv head
   const int d = ((int)threadIdx.x % kTPR) * 4;
-  const int r = blk * kRows + (int)threadIdx.x / kTPR;
-  const int R = rt * kBM + r;
-  const int t = R / a.group;
-  const int g = R - t * a.group;
-  if (d >= a.head_dim || t >= qr.ntok) return;
   const int64_t pitch = (int64_t)a.hkv * kBM;  // rows of one slot
-  const int64_t row0 = ((int64_t)slot * a.hkv + h) * kBM + r;
-  const float MA_GLOBAL* lse = gptr(a.pieces.lse) + row0;
-  const float MA_GLOBAL* po = gptr(a.pieces.o) + row0 * D + d;
-  float m = -INFINITY, w = 0.f;
-  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int units = a.pieces.merge_capacity * a.hkv * kBlocks;
+  for (int u = (int)blockIdx.x; u < units; u += (int)gridDim.x) {
+    const int blk = u % kBlocks;
+    const int rest = u / kBlocks;
+    const int h = rest % a.hkv;
+    const int MA_CONST* e = cptr(reinterpret_cast<const int*>(a.pieces.merges + rest / a.hkv));
+    const int b = e[0];
+    if (b < 0) return;
+    const int rt = e[1], slot = e[2], parts = e[3];
+    const QueryRows qr = clamp_query_rows(cptr(a.qsl)[b], cptr(a.qsl)[b + 1], a.num_tokens);
+    const int r = blk * kRows + (int)threadIdx.x / kTPR;
+    const int R = rt * kBM + r;
+    const int t = R / a.group;
+    const int g = R - t * a.group;
+    if (d >= a.head_dim || t >= qr.ntok) continue;
+    const int64_t row0 = ((int64_t)slot * a.hkv + h) * kBM + r;
+    const float MA_GLOBAL* lse = gptr(a.pieces.lse) + row0;
+    const float MA_GLOBAL* po = gptr(a.pieces.o) + row0 * D + d;
+    float m = -INFINITY, w = 0.f;
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
-  for (int p = 0; p < parts; ++p) {
-    const float l = lse[p * pitch];
-    const f32x4 o = *reinterpret_cast<const f32x4 MA_GLOBAL*>(po + p * pitch * D);
-    const float m_new = fmaxf(m, l);
-    const float base = (m_new == -INFINITY) ? 0.f : m_new;
-    const float s_old = __builtin_amdgcn_exp2f(m - base);
-    const float s_new = __builtin_amdgcn_exp2f(l - base);
-    acc = acc * s_old + o * s_new;
-    w = w * s_old + s_new;
-    m = m_new;
+    for (int p = 0; p < parts; ++p) {
+      const float l = lse[p * pitch];
+      const f32x4 o = *reinterpret_cast<const f32x4 MA_GLOBAL*>(po + p * pitch * D);
+      const float m_new = fmaxf(m, l);
+      const float base = (m_new == -INFINITY) ? 0.f : m_new;
+      const float s_old = __builtin_amdgcn_exp2f(m - base);
+      const float s_new = __builtin_amdgcn_exp2f(l - base);
+      acc = acc * s_old + o * s_new;
+      w = w * s_old + s_new;
+      m = m_new;
+    }
+    const float inv = (w > 0.f) ? a.v_scale / w : 0.f;
+    const int64_t off = (int64_t)(qr.tok0 + t) * a.out_stride_tok + (int64_t)(h * a.group + g) * a.out_stride_head + d;
+    store_out4<QBF16>(a.out, off, acc, inv, a.out_f32);
   }
-  const float inv = (w > 0.f) ? a.v_scale / w : 0.f;
-  const int64_t off = (int64_t)(qr.tok0 + t) * a.out_stride_tok + (int64_t)(h * a.group + g) * a.out_stride_head + d;
-  store_out4<QBF16>(a.out, off, acc, inv, a.out_f32);
 }
 
 // Extend above 256 dims (extend_wide.hip): rows per workgroup, keys per tile, and the launch

@@ -85,8 +85,9 @@ struct ExtendPlanArgs {
   int tile_rows, tile_keys;  // the extend kernel's rows per workgroup and keys per tile
   int capacity;              // entries of items (or of pieces)
   int64_t* items;
-  // key pieces (shares > 0): CUs per kv head, partial slots per kv head, and the lists
-  int shares, slots;
+  // key pieces (shares > 0): CUs per kv head, and the lists (`capacity` also counts the
+  // partial slots per kv head)
+  int shares;
   ExtendPiece* pieces;
   ExtendMerge* merges;
   int merge_capacity;
@@ -152,7 +153,7 @@ __device__ __forceinline__ void plan_pieces(const ExtendPlanArgs& a, int m, int*
   };
   const int round = wave / kWavesPerSearch;  // 0, 1: the search for one and two rounds
   const int probe = wave % kWavesPerSearch;
-  const int room = min((round + 1) * a.shares, a.slots);
+  const int room = min((round + 1) * a.shares, a.capacity);
   int lo = kSplitMinTiles, hi = max(cmax, kSplitMinTiles);  // the least cap that fits is in [lo, hi]
   for (int span = hi - lo; span > 0; span /= kWavesPerSearch) {  // the same passes in every wave
     // probes cut lo .. hi into kWavesPerSearch parts, each probed at its last value
@@ -802,9 +803,10 @@ __global__ __launch_bounds__(kXWaves * 64, 1) void extend_kernel(const ExtendArg
 }
 
 template <int D>
-static hipError_t launch_merge_d(bool qbf16, int merges, hipStream_t st, const ExtendArgs& a) {
+static hipError_t launch_merge_d(bool qbf16, hipStream_t st, const ExtendArgs& a) {
   constexpr int kBM = D == kWideDim ? kWideRows : XShape<D>::BM;
-  const dim3 grid((unsigned)(merges * a.hkv * (kBM * D / 1024)));
+  const int64_t units = (int64_t)a.pieces.merge_capacity * a.hkv * (kBM * D / 1024);
+  const dim3 grid((unsigned)std::min<int64_t>(units, kMergeGrid));
   if (qbf16) hipLaunchKernelGGL((extend_merge<D, kBM, true>), grid, dim3(256), 0, st, a);
   else hipLaunchKernelGGL((extend_merge<D, kBM, false>), grid, dim3(256), 0, st, a);
   return hipGetLastError();
@@ -869,15 +871,17 @@ extern "C" size_t ma_extend_workspace_bytes(int64_t num_tokens, int num_q_heads,
   return ((size_t)n * sizeof(int64_t) + 255) & ~(size_t)255;
 }
 
-// Compute units of the current device, read once per device.
+// Compute units of the current device, read once per device; those of an MI355X where no
+// device answers (the workspace sizes can be asked for without one).
 static int compute_units() {
   constexpr int kMaxDevices = 64;
+  constexpr int kNominal = 256;
   static std::atomic<int> cus[kMaxDevices];
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return kNominal;
   int n = cus[dev].load(std::memory_order_relaxed);
   if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return kNominal;
     cus[dev].store(n, std::memory_order_relaxed);
   }
   return n;
@@ -887,27 +891,32 @@ static int compute_units() {
 // work list of whole row tiles); shares 0 when the call has too many row tiles for them.
 struct PiecePlan {
   bool direct;  // no plan kernel
-  int shares, slots, capacity, merges;
+  int shares, slots, merges;
   size_t pieces_at, merges_at, lse_at, o_at, bytes;
 };
 static PiecePlan piece_plan(int64_t items, int batch, int hkv, int kdim, size_t list) {
   PiecePlan p{};
   p.bytes = list;
   const int cus = compute_units();
-  if (cus <= 0 || kdim == 0) return p;
-  const int shares = std::max(1, cus / hkv);
-  // `items` counts a partly filled tile per sequence; beyond one round of row tiles the plan
-  // kernel's ordering balances whole tiles within a few percent
-  if (items > kSplitMaxItems || items - batch > shares) return p;
+  if (kdim == 0 || hkv > cus) return p;
+  const int shares = cus / hkv;
+  // Whole row tiles from one round of them on: `items` counts a partly filled tile per
+  // sequence, so a batch of `shares` sequences or more fills the chip by itself, and what
+  // the pieces could level their launch and merge cost again (whole / pieces at D = 128, 1 to
+  // 20 new tokens each: 48 sequences after 60 keys at 32 / 8 heads 24.4 / 29.6 us, after 6,000
+  // 267 / 287; 48 at 32 / 32 heads 65 / 89; below, 24 at 32 / 8 heads 17.8 / 16.7 and 166 / 136).
+  if (batch >= std::max(shares, 2) || items - batch > shares || items > kSplitMaxItems) return p;
+  static_assert(kSplitSlotRounds >= 2, "a plan holds every whole row tile: items <= 2 * shares here");
   p.direct = items <= kDirectItems && batch <= kDirectBatch;
   const int bm = extend_tile_rows(kdim);
   p.shares = shares;
-  p.slots = std::max((int)items, kSplitSlotRounds * shares);
-  p.capacity = p.direct ? p.slots : (int)items + p.slots;
-  p.merges = p.direct ? (int)items : std::min((int)items, p.slots / 2);
+  // The planners cut row tiles only into at most this many pieces in all, so at most half as
+  // many tiles; uncut, the list holds at most `items` entries, by the line above no more.
+  p.slots = kSplitSlotRounds * shares;
+  p.merges = std::min((int)items, p.slots / 2);
   auto align = [](size_t x) { return (x + 255) & ~(size_t)255; };
   p.pieces_at = list;
-  p.merges_at = align(p.pieces_at + (p.direct ? 0 : (size_t)p.capacity * sizeof(ExtendPiece)));
+  p.merges_at = align(p.pieces_at + (p.direct ? 0 : (size_t)p.slots * sizeof(ExtendPiece)));
   p.lse_at = align(p.merges_at + (size_t)p.merges * sizeof(ExtendMerge));
   p.o_at = align(p.lse_at + (size_t)p.slots * hkv * bm * sizeof(float));
   p.bytes = align(p.o_at + (size_t)p.slots * hkv * bm * kdim * sizeof(float));
@@ -977,18 +986,16 @@ extern "C" int ma_paged_extend(
   p.tile_keys = kdim == kWideDim ? kWideKeys : kdim == 256 ? XShape<256>::BN : XShape<128>::BN;
   p.capacity = (int)items; p.items = reinterpret_cast<int64_t*>(workspace);
   // key pieces where the batch has few row tiles and the workspace holds their partials
-  PiecePlan pp{};
   ExtendPieces pieces{};
-  pp = piece_plan(items, batch, num_kv_heads, kdim, need);
-  if (pp.shares > 0 && workspace_bytes >= pp.bytes &&
-      (int64_t)pp.capacity * num_kv_heads <= 0x7fffffff / (kXWaves * 64)) {
+  const PiecePlan pp = piece_plan(items, batch, num_kv_heads, kdim, need);
+  if (pp.shares > 0 && workspace_bytes >= pp.bytes) {
     char* ws = reinterpret_cast<char*>(workspace);
-    p.shares = pp.shares; p.slots = pp.slots; p.capacity = pp.capacity; p.merge_capacity = pp.merges;
+    p.shares = pp.shares; p.capacity = pp.slots; p.merge_capacity = pp.merges;
     p.pieces = reinterpret_cast<ExtendPiece*>(ws + pp.pieces_at);
     p.merges = reinterpret_cast<ExtendMerge*>(ws + pp.merges_at);
     pieces.list = pp.direct ? nullptr : p.pieces;
     pieces.merges = p.merges; pieces.merge_capacity = pp.merges;
-    pieces.shares = pp.shares; pieces.capacity = pp.capacity;
+    pieces.shares = pp.shares; pieces.capacity = pp.slots;
     pieces.lse = reinterpret_cast<float*>(ws + pp.lse_at);
     pieces.o = reinterpret_cast<float*>(ws + pp.o_at);
   }
@@ -1021,10 +1028,10 @@ extern "C" int ma_paged_extend(
                     : extend_wide_launch(qbf16, kv_dtype, grid, (hipStream_t)stream, a);
   if (e != hipSuccess) return set_error(MA_ELAUNCH, "extend launch failed: %s", hipGetErrorString(e));
   if (pieces.shares > 0) {
-    e = kdim == 64    ? launch_merge_d<64>(qbf16, pp.merges, (hipStream_t)stream, a)
-        : kdim == 128 ? launch_merge_d<128>(qbf16, pp.merges, (hipStream_t)stream, a)
-        : kdim == 256 ? launch_merge_d<256>(qbf16, pp.merges, (hipStream_t)stream, a)
-                      : launch_merge_d<kWideDim>(qbf16, pp.merges, (hipStream_t)stream, a);
+    e = kdim == 64    ? launch_merge_d<64>(qbf16, (hipStream_t)stream, a)
+        : kdim == 128 ? launch_merge_d<128>(qbf16, (hipStream_t)stream, a)
+        : kdim == 256 ? launch_merge_d<256>(qbf16, (hipStream_t)stream, a)
+                      : launch_merge_d<kWideDim>(qbf16, (hipStream_t)stream, a);
     if (e != hipSuccess) return set_error(MA_ELAUNCH, "extend merge launch failed: %s", hipGetErrorString(e));
   }
   return MA_OK;

@@ -234,3 +234,25 @@ def test_small_decode_rule_matches_the_library():
     assert ops.decode_kernel(64, 16, 4, 512, 8192) == "any_kernel"        # not a tuned head dim
     assert ops.decode_kernel(8, 64, 8, 128, 8192) == "any_kernel"         # 8 x 8 x 256 = 16384 tiles
     assert ops.decode_kernel(8, 64, 8, 128, 8193) == "splitkv_partial"
+
+
+# 256 compute units, at most two pieces each: rows of a tile x (head dim of the kernel + LSE) fp32
+PIECES_MAX = {64: 512 * 256 * 65 * 4, 128: 512 * 256 * 129 * 4, 256: 512 * 128 * 257 * 4, 512: 512 * 128 * 513 * 4}
+LISTS_MAX = 256 << 10
+
+
+@pytest.mark.parametrize("dim,kdim", [(64, 64), (48, 64), (128, 128), (96, 128), (256, 256), (192, 256), (512, 512), (272, 512)])
+@pytest.mark.parametrize("hq,hkv", [(32, 8), (64, 64), (32, 32), (8, 1), (12, 3), (256, 256), (300, 300)])
+def test_extend_piece_workspace_is_bounded(lib, dim, kdim, hq, hkv):
+    for batch in (1, 2, 4, 7, 8, 31, 32, 33, 70, 127, 255, 256, 300, 900, 1000, 1023, 16384):
+        for per_seq in (1, 5, 130, 3000):
+            tokens = batch * per_seq
+            whole = lib.ma_extend_workspace_bytes(tokens, hq, hkv, batch)
+            split = lib.ma_extend_split_workspace_bytes(tokens, hq, hkv, batch, dim)
+            assert whole <= split <= max(whole, PIECES_MAX[kdim] + LISTS_MAX), (batch, per_seq, split)
+            # as many sequences as CUs of a kv head fill the chip with whole row tiles
+            if batch >= max(256 // hkv, 2) or hkv > 256:
+                assert split == whole, (batch, per_seq, split)
+    # one sequence of few tokens can be cut at any number of kv heads the chip has CUs for
+    if hkv <= 256:
+        assert lib.ma_extend_split_workspace_bytes(5, hq, hkv, 1, dim) > lib.ma_extend_workspace_bytes(5, hq, hkv, 1)
