@@ -118,7 +118,7 @@ __device__ __forceinline__ int block_exclusive_scan(int x, int* sums, int* total
   return before + incl - x;
 }
 
-// Cut the m row tiles (m <= kSplitMaxItems, one per thread) into key pieces and list them,
+// Cut the m row tiles (one per thread) into key pieces and list them,
 // longest first. The pieces of a tile are its key tiles in near-equal shares of at most
 // `cap`. Three caps are priced (pieces_cost): whole tiles, and the least caps with which
 // the pieces make one and two rounds on the CUs, each searched for by eight waves.
@@ -133,6 +133,9 @@ __device__ __forceinline__ void plan_pieces(const ExtendPlanArgs& a, int m, int*
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
+  // query ranges that overlap make more row tiles than num_tokens does; the list and `cost`
+  // end here
+  m = min(m, min(kSplitMaxItems, a.capacity));
   int b = -1, rt = 0, c = 0;
   if (tid < m) c = decode(tid, &b, &rt) - kPlanFixedCost;
   cost[tid] = c;

@@ -136,3 +136,20 @@ def test_pieces_replay_in_a_hip_graph_with_new_lengths():
         graph.replay()
         torch.cuda.synchronize()
         assert float((out.double() - _reference(c, True, -1)).abs().max()) < 4e-3
+
+
+def test_overlapping_query_ranges_stay_inside_the_plan():
+    """Ranges that all cover the same tokens make 1,300 row tiles of 213 expected: more than
+    the plan holds. Every range computes the same rows, so any of them gives the result."""
+    print("[case] overlapping query ranges", flush=True)
+    heads, hkv, dim, T, B = 8, 1, 128, 400, 200
+    c = _make([50], [T], heads, hkv, dim, BF16, BF16)
+    ref = _reference(c, True, -1)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    c["table"] = c["table"].expand(B, -1).contiguous()
+    c["qsl_t"] = torch.tensor([0, T] * (B // 2) + [0], **i32)  # b even: [0, T); b odd: empty
+    c["pre_t"], c["seq_t"] = torch.full((B,), 50, **i32), torch.full((B,), 50 + T, **i32)
+    out = torch.full(c["q"].shape, float("nan"), dtype=torch.float32, device=DEV)
+    _call(c, True, -1, _ops().extend_workspace(torch.device(DEV), T, heads, hkv, B, dim), out)
+    torch.cuda.synchronize()
+    assert float((out.double() - ref).abs().max()) < 4e-3
