@@ -32,7 +32,8 @@ struct ExtendPieces {
   const ExtendPiece* list;  // the plan kernel's list, or null: each workgroup plans (plan_direct)
   ExtendMerge* merges;      // the cut row tiles, then entries with sequence -1
   int merge_capacity;
-  int shares;    // CUs per kv head; 0: whole row tiles from the work list
+  int shares;       // CUs per kv head; 0: whole row tiles from the work list
+  float slot_cost;  // piece_slot_cost of the kernel
   int capacity;  // pieces per kv head that the list, the grid and the partial slots hold
   float* o;      // [slot][kv head][row of the tile][D] fp32
   float* lse;    // [slot][kv head][row of the tile]
@@ -101,13 +102,14 @@ __device__ __forceinline__ int seq_row_tiles(int ntok, int group, int bm) {
 // Estimated time, in key tiles, of n pieces of at most `longest` of `all` key tiles on
 // `shares` CUs per kv head: the longest piece, or the mean piece times the rounds the
 // pieces make, each with a workgroup's start and end, plus the writing and reading back of
-// the `split` pieces that leave partials.
-__device__ __forceinline__ float pieces_cost(float all, float n, float longest, float split, float shares) {
-  constexpr float kStart = 5.f;       // a workgroup's start and end: about 8 us, a key tile 1.2-1.9 us
-  constexpr float kMergeSlot = 8.f;   // one partial per CU, written and read back: about 14 us
+// the `split` pieces that leave partials, `slot_cost` for one per CU.
+__device__ __forceinline__ float pieces_cost(float all, float n, float longest, float split, float shares,
+                                             float slot_cost) {
+  constexpr float kStart = 5.f;  // a workgroup's start and end: 6 to 8 us, a key tile 0.9 to 1.9 us
   const float mean = (all + kStart * n) / fmaxf(n, 1.f);
-  return fmaxf(longest + kStart, mean * ceilf(n / shares)) + kMergeSlot * split / shares;
+  return fmaxf(longest + kStart, mean * ceilf(n / shares)) + slot_cost * split / shares;
 }
+
 // Inclusive prefix sum over the wave's lanes, and the wave's maximum, of values >= 0, by
 // DPP moves (a few cycles a step; a cross-lane read through LDS takes over a hundred).
 template <int CTRL, int ROWS>
@@ -196,7 +198,7 @@ __device__ __forceinline__ ExtendPiece plan_direct(const ExtendArgs& a, int w, i
   // Three candidates: whole tiles, and the least caps with which the pieces make one and
   // two rounds on the CUs.
   int cap = max(cmax, 1);
-  float est = pieces_cost((float)all, (float)m, (float)cmax, 0.f, (float)a.pieces.shares);
+  float est = pieces_cost((float)all, (float)m, (float)cmax, 0.f, (float)a.pieces.shares, a.pieces.slot_cost);
 #pragma unroll 1
   for (int r = 1; r <= 2; ++r) {
     const int room = min(r * a.pieces.shares, a.pieces.capacity);
@@ -217,7 +219,8 @@ __device__ __forceinline__ ExtendPiece plan_direct(const ExtendArgs& a, int w, i
     }
     split = __builtin_amdgcn_readlane(wave_scan(split), 63);
     longest = wave_max(longest);
-    const float e = pieces_cost((float)all, (float)n, (float)longest, (float)split, (float)a.pieces.shares);
+    const float e = pieces_cost((float)all, (float)n, (float)longest, (float)split, (float)a.pieces.shares,
+                                a.pieces.slot_cost);
     if (e < est) {
       est = e;
       cap = lo;

@@ -88,6 +88,7 @@ struct ExtendPlanArgs {
   // key pieces (shares > 0): CUs per kv head, and the lists (`capacity` also counts the
   // partial slots per kv head)
   int shares;
+  float slot_cost;
   ExtendPiece* pieces;
   ExtendMerge* merges;
   int merge_capacity;
@@ -188,13 +189,14 @@ __device__ __forceinline__ void plan_pieces(const ExtendPlanArgs& a, int m, int*
     if (lane == 0) {
       found_cap[round] = hi;
       found_est[round] = n > room ? INFINITY
-                                  : pieces_cost((float)all, (float)n, (float)longest, (float)split, (float)a.shares);
+                                  : pieces_cost((float)all, (float)n, (float)longest, (float)split, (float)a.shares,
+                                                a.slot_cost);
     }
   }
   hist[tid] = 0;
   __syncthreads();
   int cap = max(cmax, 1);
-  float est = pieces_cost((float)all, (float)m, (float)cmax, 0.f, (float)a.shares);
+  float est = pieces_cost((float)all, (float)m, (float)cmax, 0.f, (float)a.shares, a.slot_cost);
 #pragma unroll
   for (int r = 0; r < 2; ++r)
     if (found_est[r] < est) {
@@ -890,6 +892,16 @@ static int compute_units() {
   return n;
 }
 
+// One partial per CU, written and read back, in key tiles of the kernel: 17 MB at 64 dims, 34
+// at 128 and 256, 67 above, against tiles of 64 keys up to 128 dims and of 32 above. Taken
+// from 620 calls (1 to 8 sequences of 5 to 900 tokens after 0 to 3,000 keys), as the cost at
+// which they took least in all; at 64 / 128 / 256 / 512 dims in ms:
+//    4: 3.05 / 4.09 / 6.29 / 9.65   8: 3.01 / 4.06 / 6.25 / 9.59   12: 3.04 / 4.10 / 6.19 / 9.58
+//   16: 3.08 / 4.17 / 6.22 / 9.61   no cuts: 3.98 / 5.77 / 8.81 / 14.25
+// With 8 at 256 dims 12 calls of 175 took over 2% longer than on whole tiles (up to 14%), with
+// 12 three (up to 4%).
+static float piece_slot_cost(int kdim) { return kdim <= 128 ? 8.f : 12.f; }
+
 // Key pieces of a call: sizes and offsets in the workspace (whose first `list` bytes are the
 // work list of whole row tiles); shares 0 when the call has too many row tiles for them.
 struct PiecePlan {
@@ -993,12 +1005,12 @@ extern "C" int ma_paged_extend(
   const PiecePlan pp = piece_plan(items, batch, num_kv_heads, kdim, need);
   if (pp.shares > 0 && workspace_bytes >= pp.bytes) {
     char* ws = reinterpret_cast<char*>(workspace);
-    p.shares = pp.shares; p.capacity = pp.slots; p.merge_capacity = pp.merges;
+    p.shares = pp.shares; p.slot_cost = piece_slot_cost(kdim); p.capacity = pp.slots; p.merge_capacity = pp.merges;
     p.pieces = reinterpret_cast<ExtendPiece*>(ws + pp.pieces_at);
     p.merges = reinterpret_cast<ExtendMerge*>(ws + pp.merges_at);
     pieces.list = pp.direct ? nullptr : p.pieces;
     pieces.merges = p.merges; pieces.merge_capacity = pp.merges;
-    pieces.shares = pp.shares; pieces.capacity = pp.slots;
+    pieces.shares = pp.shares; pieces.slot_cost = p.slot_cost; pieces.capacity = pp.slots;
     pieces.lse = reinterpret_cast<float*>(ws + pp.lse_at);
     pieces.o = reinterpret_cast<float*>(ws + pp.o_at);
   }

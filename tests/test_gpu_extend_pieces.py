@@ -53,6 +53,25 @@ def _call(c, causal, window, workspace, out):
         k_scale=0.5, v_scale=2.0, causal=causal, sliding_window_size=window, out=out, workspace=workspace, page_size=1)
 
 
+def _cut_tiles(ws, T, heads, hkv, dim, B):
+    """(row tiles a call cut, pieces of them), read back from its merge entries: after the
+    work list, and after the piece list (32 bytes an entry, two entries per CU of a kv head)
+    where a plan kernel makes one (over 128 row tiles expected, or over 64 sequences)."""
+    at = _ops().extend_workspace_bytes(T, heads, hkv, B)
+    shares = torch.cuda.get_device_properties(0).multi_processor_count // hkv
+    bm = 256 if dim <= 128 else 128
+    items = -(-T * (heads // hkv) // bm) + B
+    listed = items > 128 or B > 64
+    if listed:
+        at += (2 * shares * 32 + 255) & ~255
+    n = min(items, shares)
+    entries = ws[at:at + 16 * n].view(torch.int32).view(n, 4).tolist()
+    cut = [e for e in entries if e[0] >= 0]
+    assert entries[:len(cut)] == cut  # the empty entries come last
+    assert all(e[3] > 1 for e in cut)
+    return listed, len(cut), sum(e[3] for e in cut)
+
+
 CASES = [  # prefix, ext, heads, kv heads, dim, q dtype, kv dtype, causal, window
     ([5000], [70], 32, 8, 128, BF16, BF16, True, -1),          # one tile and a half, many pieces
     ([9000], [300], 8, 1, 128, BF16, E4M3, True, -1),          # one kv head: a share of every CU
@@ -153,3 +172,27 @@ def test_overlapping_query_ranges_stay_inside_the_plan():
     _call(c, True, -1, _ops().extend_workspace(torch.device(DEV), T, heads, hkv, B, dim), out)
     torch.cuda.synchronize()
     assert float((out.double() - ref).abs().max()) < 4e-3
+
+
+@pytest.mark.parametrize("prefix,ext,heads,hkv,dim,cuts", [
+    ([60] * 4, [180] * 4, 16, 4, 192, False),   # partials cost more than the 9 key tiles they would level
+    ([60] * 4, [180] * 4, 16, 4, 256, False),
+    ([3000] * 4, [180] * 4, 16, 4, 256, True),
+    ([900] * 4, [180] * 4, 32, 8, 128, True),
+    ([100] * 130, [10] * 130, 8, 1, 128, False),  # two key tiles each
+    ([900] * 40, [10] * 40, 32, 8, 128, None),  # more sequences than CUs of a kv head: no pieces at all
+])
+def test_the_plan_cuts_where_it_pays(prefix, ext, heads, hkv, dim, cuts):
+    print(f"[case] plan of {len(prefix)} x {ext[0]} after {prefix[0]} h={heads}/{hkv} d={dim}", flush=True)
+    ops = _ops()
+    c = _make(prefix, ext, heads, hkv, dim, BF16, BF16)
+    T, B = c["q"].shape[0], len(prefix)
+    ws = ops.extend_workspace(torch.device(DEV), T, heads, hkv, B, dim)
+    if cuts is None:
+        assert ws.numel() == ops.extend_workspace_bytes(T, heads, hkv, B)
+        return
+    _call(c, True, -1, ws, torch.empty_like(c["q"]))
+    torch.cuda.synchronize()
+    _, cut, pieces = _cut_tiles(ws, T, heads, hkv, dim, B)
+    assert (cut > 0) == cuts
+    assert pieces <= 2 * (torch.cuda.get_device_properties(0).multi_processor_count // hkv)
