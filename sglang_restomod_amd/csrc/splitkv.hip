@@ -1253,12 +1253,16 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
   }
   const int rows_total = max_q_per_seq * a.group;
   // Two row blocks per group read K and V once for all rows. Over fp8 KV at D = 256 that
-  // kernel is long, and up to two tiles per wave at the caller's bound one-block groups end
-  // first. Per call, one block against two (12 / 2 heads, 4 rows, e5m2): 16 sequences of 190
-  // keys 20.0 / 22.8 us, 4 of 6k 27.5 / 29.4, one of 22k 35.7 / 41.7; beyond, 16 of 6k 43.9 /
-  // 43.4 and 64 of 1.5k 45.7 / 45.4.
-  const bool few256 = head_dim == 256 && kv_dtype >= DT_E4M3 && max_seq_len > 0 &&
-                      (int64_t)a.batch * a.hkv * ((max_seq_len + 31) / 32) <= (int64_t)num_workgroups * kWaves * 2;
+  // kernel is long, and one-block groups end first up to about four tiles per wave. Per call,
+  // one block against two (e4m3): 12 / 2 heads, 4 rows, 16 sequences of 190 keys (0.1 tiles)
+  // 18.1 / 21.6 us, two of 22k (2.7) 32.6 / 39.9, 6 of 9k (3.3) 35.5 / 36.4, 3 of 30k (5.6)
+  // 47.9 / 43.9; 16 / 4 heads, 8 rows, 64 of 300 (2.4) 34.8 / 39.2, 4 of 6k (3.0) 30.9 /
+  // 36.1, 12 of 3k (4.5) 43.8 / 39.9, 30 of 4k (15) 107 / 72. Without a bound the tiles are
+  // not known and the groups stay at one block: two blocks took a quarter longer on short
+  // contexts, where a call with long ones can give its bound.
+  const bool few256 = head_dim == 256 && kv_dtype >= DT_E4M3 &&
+                      (max_seq_len == 0 || (int64_t)a.batch * a.hkv * ((max_seq_len + 31) / 32) <=
+                                               (int64_t)num_workgroups * kWaves * 4);
   const int nb = rows_total <= 16 || few256 ? 1 : 2;
   a.rows = 16 * nb;
   a.row_groups = (rows_total + a.rows - 1) / a.rows;

@@ -37,13 +37,7 @@ CASES = [  # prefix, new tokens, heads, kv heads, dim, q dtype, kv dtype, window
 ]
 
 
-@pytest.mark.parametrize("hinted", [True, False])
-@pytest.mark.parametrize("prefix,new,heads,hkv,dim,q_dtype,kv,window,hint", CASES)
-def test_verify_matches_float64(prefix, new, heads, hkv, dim, q_dtype, kv, window, hint, hinted):
-    from sglang_restomod_amd.attention.mi355x import ops
-
-    print(f"[case] verify split prefix={prefix[:4]} new={new[:4]} h={heads}/{hkv} d={dim} q={q_dtype} kv={kv} "
-          f"window={window} hint={hint} hinted={hinted}", flush=True)
+def _case(prefix, new, heads, hkv, dim, q_dtype, kv):
     g = torch.Generator(device=DEV).manual_seed(11)
     seq = [p + n for p, n in zip(prefix, new)]
     slots = sum(seq) + 1
@@ -56,17 +50,47 @@ def test_verify_matches_float64(prefix, new, heads, hkv, dim, q_dtype, kv, windo
     k, v = (torch.randn(slots, hkv, dim, generator=g, device=DEV).to(kv) for _ in range(2))
     q = (3 * torch.randn(sum(new), heads, dim, generator=g, device=DEV)).to(q_dtype)
     qsl = [sum(new[:i]) for i in range(len(new) + 1)]
+    return q, k, v, table, seq, qsl
+
+
+def _run(case, prefix, window, hint, bound):
+    from sglang_restomod_amd.attention.mi355x import ops
+
+    q, k, v, table, seq, qsl = case
     i32 = dict(dtype=torch.int32, device=DEV)
     out = torch.full(q.shape, float("nan"), dtype=torch.float32, device=DEV)
     ops.paged_verify_forward(
         q, k, v, table, torch.tensor(seq, **i32), torch.tensor(qsl, **i32), torch.tensor(prefix, **i32),
-        max_q_per_seq=hint, softmax_scale=dim ** -0.5, k_scale=0.5, v_scale=2.0, sliding_window_size=window, out=out,
-        page_size=1, max_seq_len_hint=max(seq) if hinted else None)
+        max_q_per_seq=hint, softmax_scale=q.shape[2] ** -0.5, k_scale=0.5, v_scale=2.0, sliding_window_size=window,
+        out=out, page_size=1, max_seq_len_hint=bound)
     torch.cuda.synchronize()
+    return out
+
+
+@pytest.mark.parametrize("hinted", [True, False])
+@pytest.mark.parametrize("prefix,new,heads,hkv,dim,q_dtype,kv,window,hint", CASES)
+def test_verify_matches_float64(prefix, new, heads, hkv, dim, q_dtype, kv, window, hint, hinted):
+    print(f"[case] verify split prefix={prefix[:4]} new={new[:4]} h={heads}/{hkv} d={dim} q={q_dtype} kv={kv} "
+          f"window={window} hint={hint} hinted={hinted}", flush=True)
+    case = _case(prefix, new, heads, hkv, dim, q_dtype, kv)
+    q, k, v, table, seq, qsl = case
+    out = _run(case, prefix, window, hint, max(seq) if hinted else None)
     ref = torch_f64.attend(q, k.float(), v.float(), [table[b] for b in range(len(seq))], qsl, prefix, seq,
                            softmax_scale=dim ** -0.5, k_scale=0.5, v_scale=2.0, sliding_window=window)
     # 2e-3 is the repository's bound for v_scale near 1
     assert float((out.double() - ref).abs().max()) < 4e-3
+
+
+@pytest.mark.parametrize("heads,hkv,tokens,prefix", [(12, 2, 4, [190] * 16), (16, 4, 8, [300] * 20), (12, 2, 4, [9000])])
+def test_fp8_d256_without_a_bound_runs_one_block_groups(heads, hkv, tokens, prefix):
+    """The row groups decide how the work is shared out, so the same groups give the same
+    bits: a call without a bound, and one whose bound is below four tiles per wave."""
+    print(f"[case] verify d=256 without a bound h={heads}/{hkv} tokens={tokens} prefix={prefix[:2]}", flush=True)
+    case = _case(prefix, [tokens] * len(prefix), heads, hkv, 256, BF16, E4M3)
+    got = _run(case, prefix, -1, tokens, None)
+    assert torch.equal(got, _run(case, prefix, -1, tokens, prefix[0] + tokens))
+    # a bound far past the lengths takes two blocks, which sum in another order
+    assert not torch.equal(got, _run(case, prefix, -1, tokens, 300_000))
 
 
 @pytest.mark.parametrize("heads,hkv,dim,kv", [(8, 1, 128, BF16), (12, 2, 256, E4M3), (16, 4, 512, F16), (5, 1, 80, BF16)])
