@@ -1125,6 +1125,17 @@ extern "C" size_t ma_splitkv_workspace_bytes(int num_workgroups, int head_dim) {
 #endif
 constexpr int64_t kSmallDecodeTiles = MA_SMALL_DECODE_TILES;
 
+// A small verify whose row blocks are too many to split runs one workgroup per row block,
+// whose keys one workgroup walks (about 8 us per 1,000 e4m3 keys, 10 in fp16): up to this
+// bound even one long sequence among short ones ends no later than on the persistent kernel.
+// 32 / 8 heads, D = 128, e4m3 / fp16, row blocks against the persistent kernel: 32 sequences,
+// one of 1,200 keys and the rest of 60, 14.0 / 16.1 us against 13.7 / 14.9 (16.0 / 16.9 before
+// its workgroups merged in LDS); one of 2,000 19.7 / 23.4 against 14.8 / 15.8; 16, one of 4,000,
+// 33.7 / 42.2 against 17.8 / 18.2. All of one length the row blocks end first further up: 32
+// of 1,200 18.7 / 28.7 against 27.9 / 37.6, of 2,000 26.5 / 45.4 against 35.7 / 54.9; the bound
+// does not tell the two apart.
+constexpr int kWholeVerifyKeys = 1280;
+
 // ---------------------------------------------------------------------------
 // Static scratch of the allocation-free decode (ma_grouped_decode_noalloc): the split-KV
 // workspace of a persistent grid of up to kScratchWorkgroups workgroups at the largest
@@ -1199,6 +1210,12 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
   if ((int64_t)a.num_tokens * a.group > 0x7fffffff) return set_error(MA_EINVAL, "num_tokens x GQA group exceeds 2^31");
   if (max_seq_len < 0) return set_error(MA_EINVAL, "max_seq_len must be >= 0 (0: not known)");
   const bool decode = a.qsl == nullptr;
+  const int64_t row_blocks = ((int64_t)max_q_per_seq * a.group + kAnyRows - 1) / kAnyRows;
+  const int64_t base = (int64_t)a.batch * a.hkv * row_blocks;  // one workgroup per row block
+  // Row blocks whose keys may be split over workgroups: fewer than the CUs. A verify up to 128
+  // dims (two workgroups a CU) splits below half the CUs only: at half of them (16 sequences of
+  // 6k keys, 8 kv heads, D = 96, e4m3) the split measured 69.5 against 64.1 us.
+  const bool can_split = (decode || head_dim > 128 ? base : 2 * base) < num_workgroups;
   // a small decode, or a small verify of one 16-row block: the split-KV tiles at the longest
   // length the caller knows, in tiles of 128 dims. A verify over bf16 KV stays on the
   // persistent kernel, which keeps P to 16 bits (two bf16 halves) and bf16 V exact.
@@ -1206,7 +1223,7 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
   if (!generic && max_seq_len > 0 && (decode || (kv_dtype != DT_BF16 && (int64_t)max_q_per_seq * a.group <= kAnyRows))) {
     const int64_t row_groups = (a.group + 31) / 32;
     const int64_t tiles = (int64_t)a.batch * a.hkv * row_groups * ((max_seq_len + 31) / 32);
-    small = tiles * (head_dim > 128 ? 2 : 1) <= kSmallDecodeTiles;
+    small = tiles * (head_dim > 128 ? 2 : 1) <= kSmallDecodeTiles && (decode || can_split || max_seq_len <= kWholeVerifyKeys);
   }
   if (generic || small) {
     // one workgroup per 16 rows (token, GQA head), its four waves splitting the keys and
@@ -1218,15 +1235,12 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
     g.tt = a.tt; g.row_index = a.row_index; g.seq_lens = a.seq_lens; g.qsl = a.qsl; g.prefix = a.prefix;
     g.num_tokens = a.num_tokens; g.batch = a.batch; g.hq = a.hq; g.hkv = a.hkv; g.group = a.group;
     g.head_dim = head_dim;
-    g.row_blocks = (int)(((int64_t)max_q_per_seq * a.group + kAnyRows - 1) / kAnyRows);
+    g.row_blocks = (int)row_blocks;
     g.causal = a.causal; g.window = a.window; g.scale_log2 = a.scale_log2; g.v_scale = a.v_scale;
     g.out = a.out; g.out_stride_tok = a.out_stride_tok; g.out_stride_head = a.out_stride_head; g.out_f32 = a.out_f32;
     g.pieces = 1;
-    const int64_t base = (int64_t)a.batch * a.hkv * g.row_blocks;  // one workgroup per row block
     const int64_t cap_slots = (int64_t)num_workgroups * kPieceWgPerCu;
-    // a verify up to 128 dims (two workgroups a CU) below half the CUs only: at half of them
-    // (16 sequences of 6k keys, 8 kv heads, D = 96, e4m3) the split measured 69.5 against 64.1 us
-    if ((decode || head_dim > 128 ? base : 2 * base) < num_workgroups && workspace && workspace_bytes >= any_piece_bytes(cap_slots, head_dim) &&
+    if (can_split && workspace && workspace_bytes >= any_piece_bytes(cap_slots, head_dim) &&
         !(reinterpret_cast<uintptr_t>(workspace) & 255)) {
       // pieces: enough workgroups to cover the chip twice, no more than one 16-key tile per
       // wave at the longest length known (the caller's bound, else the table's width),

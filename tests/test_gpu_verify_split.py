@@ -93,6 +93,18 @@ def test_fp8_d256_without_a_bound_runs_one_block_groups(heads, hkv, tokens, pref
     assert not torch.equal(got, _run(case, prefix, -1, tokens, 300_000))
 
 
+@pytest.mark.parametrize("prefix,new,dim,kv", [
+    ([4000] + [100] * 15, 2, 128, E4M3), ([2000] + [50] * 31, 4, 128, F16), ([2000] + [50] * 31, 2, 64, E5M2),
+])
+def test_a_long_sequence_among_many_short_ones_is_shared(prefix, new, dim, kv):
+    """Row blocks too many to split, over a bound that one workgroup would walk for longer
+    than the persistent kernel takes: the persistent kernel, as without a bound (same bits)."""
+    print(f"[case] verify of {len(prefix)} ragged sequences new={new} d={dim} kv={kv}", flush=True)
+    case = _case(prefix, [new] * len(prefix), 32, 8, dim, F16 if kv == F16 else BF16, kv)
+    got = _run(case, prefix, -1, new, max(prefix) + new)
+    assert torch.equal(got, _run(case, prefix, -1, new, None))
+
+
 @pytest.mark.parametrize("heads,hkv,dim,kv", [(8, 1, 128, BF16), (12, 2, 256, E4M3), (16, 4, 512, F16), (5, 1, 80, BF16)])
 def test_decode_of_one_long_sequence(heads, hkv, dim, kv):
     """Hundreds of key pieces of one row block: more than one round of the merge's loads."""
