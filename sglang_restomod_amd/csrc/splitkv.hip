@@ -1242,13 +1242,17 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
     const int64_t cap_slots = (int64_t)num_workgroups * kPieceWgPerCu;
     if (can_split && workspace && workspace_bytes >= any_piece_bytes(cap_slots, head_dim) &&
         !(reinterpret_cast<uintptr_t>(workspace) & 255)) {
-      // pieces: enough workgroups to cover the chip twice, no more than one 16-key tile per
-      // wave at the longest length known (the caller's bound, else the table's width),
-      // within the workspace's piece slots; each piece is an equal share of its sequence's
-      // own keys, so any bound gives the same result
+      // pieces: enough workgroups to cover the chip twice (a verify: once), no more than one
+      // 16-key tile per wave at the longest length known (the caller's bound, else the table's
+      // width), within the workspace's piece slots; each piece is an equal share of its
+      // sequence's own keys, so any bound gives a correct result. A verify's 16 full rows make
+      // its partials and its merge up to 16 times a decode's: 2 tokens at 16 / 4 heads, D = 512,
+      // e4m3, pieces over the chip twice / once / not split: 16 sequences of 700 keys 31.7 /
+      // 22.1 / 27.0 us, 4 of 6k 37.7 / 29.0 / 138, 16 of 190 without a bound 24.0 / 16.4 / 14.4;
+      // 32 / 8 heads, D = 96: 4 of 700 11.5 / 10.8 / 10.7, 4 of 6k 27.1 / 23.6 / 50.5.
       const int64_t width = max_seq_len > 0 ? (int64_t)max_seq_len : (a.tt.stride << a.tt.page_shift);
       const int64_t by_len = (width + kAnyWaves * kAnyKeys - 1) / (kAnyWaves * kAnyKeys);
-      const int64_t want = (cap_slots + base - 1) / base;
+      const int64_t want = decode ? (cap_slots + base - 1) / base : num_workgroups / base;
       const int64_t pieces =
           width > kPieceMinKeys ? std::min(std::min(want, by_len), std::min<int64_t>(cap_slots / base, kAnyMaxPieces)) : 1;
       if (pieces > 1) {

@@ -53,7 +53,7 @@ def _case(prefix, new, heads, hkv, dim, q_dtype, kv):
     return q, k, v, table, seq, qsl
 
 
-def _run(case, prefix, window, hint, bound):
+def _run(case, prefix, window, hint, bound, workspace=None):
     from sglang_restomod_amd.attention.mi355x import ops
 
     q, k, v, table, seq, qsl = case
@@ -62,7 +62,7 @@ def _run(case, prefix, window, hint, bound):
     ops.paged_verify_forward(
         q, k, v, table, torch.tensor(seq, **i32), torch.tensor(qsl, **i32), torch.tensor(prefix, **i32),
         max_q_per_seq=hint, softmax_scale=q.shape[2] ** -0.5, k_scale=0.5, v_scale=2.0, sliding_window_size=window,
-        out=out, page_size=1, max_seq_len_hint=bound)
+        out=out, page_size=1, max_seq_len_hint=bound, workspace=workspace)
     torch.cuda.synchronize()
     return out
 
@@ -103,6 +103,23 @@ def test_a_long_sequence_among_many_short_ones_is_shared(prefix, new, dim, kv):
     case = _case(prefix, [new] * len(prefix), 32, 8, dim, F16 if kv == F16 else BF16, kv)
     got = _run(case, prefix, -1, new, max(prefix) + new)
     assert torch.equal(got, _run(case, prefix, -1, new, None))
+
+
+@pytest.mark.parametrize("prefix,heads,hkv,dim,padded,bounded", [
+    ([700] * 16, 16, 4, 512, 512, True), ([600] * 16, 16, 4, 192, 256, False), ([700] * 4, 32, 8, 96, 128, True),
+])
+def test_verify_pieces_cover_the_chip_once(prefix, heads, hkv, dim, padded, bounded):
+    """One piece per CU at most, counted in the partial slots the call writes."""
+    from sglang_restomod_amd.attention.mi355x import ops
+
+    print(f"[case] verify pieces {len(prefix)} x {prefix[0]} h={heads}/{hkv} d={dim}", flush=True)
+    case = _case(prefix, [2] * len(prefix), heads, hkv, dim, BF16, BF16)
+    ws = ops.splitkv_workspace(torch.device(DEV), head_dim=dim).fill_(0xA5)
+    _run(case, prefix, -1, 2, prefix[0] + 2 if bounded else None, ws)
+    slots = ws.numel() // (16 * (padded + 1) * 4)
+    used = (ws[:slots * 16 * padded * 4].view(slots, -1) != 0xA5).any(1)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert len(prefix) * hkv < int(used.sum()) <= cus
 
 
 @pytest.mark.parametrize("heads,hkv,dim,kv", [(8, 1, 128, BF16), (12, 2, 256, E4M3), (16, 4, 512, F16), (5, 1, 80, BF16)])
