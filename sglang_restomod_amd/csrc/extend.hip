@@ -389,7 +389,11 @@ __global__ __launch_bounds__(kXWaves * 64, 1) void extend_kernel(const ExtendArg
   __shared__ __attribute__((aligned(1024))) unsigned char vring[S][kStageB];
 
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // scalar: 0.6% on the D = 128 batches
+  // The wave index in a scalar register (0.6% on the D = 128 batches), except where K and V
+  // move on different waves: the D = 64 fp8 kernel took 275 us that way on 16 sequences of
+  // about 200 tokens after 8,000 keys, 257 with a vector index.
+  int wave = threadIdx.x >> 6;
+  if constexpr (!kSplitDMA) wave = __builtin_amdgcn_readfirstlane(wave);
   const int c = lane & 15;
   const int j = lane >> 4;
   // Head-dim order of the QK contraction: MFMA step kk of lane group j holds dims
