@@ -1116,14 +1116,17 @@ extern "C" size_t ma_splitkv_workspace_bytes(int num_workgroups, int head_dim) {
 // cost more than they save. Measured at D = 128, 32 / 8 heads, B 1-32 and contexts of
 // 512-8192: the pieces are faster up to 16384 tiles (B = 8 at 8192 keys: 51.8 against
 // 61.5 us per call; B = 32 at 2048: 45.6 against 59.4) and slower beyond (B = 16 at 8192:
-// 110 against 101); B = 1 at 512 keys takes 16.5 us per call either way. A tile of 256
-// dims counts twice: 12 / 2 heads 4 x 22k keys (5.6k tiles) 27 against 34 us, 16 / 4 heads
-// 16 x 6k keys (12k tiles) 92 against 81. A verify of one 16-row block over fp16 or fp8 KV
+// 110 against 101); B = 1 at 512 keys takes 16.5 us per call either way. At 256 dims over
+// K rows of more than 1 KB (and for a verify) a tile counts twice, pieces against split-KV: 16 / 4 heads, bf16,
+// 16 x 6k keys (12k tiles) 85 / 78 us, 30k keys x 4 (15k) 100 / 91, against e4m3 41 / 47 and
+// 49 / 55, 12 / 2 heads, bf16, 64 x 3k (12k) 71 / 78 and 8 sequences, one of 30k keys and the
+// rest of 100 (15k), 29 / 42. A verify of one 16-row block over fp16 or fp8 KV
 // is the same work: 32 / 8 heads, 16 x 1.5k keys 24.8 against 32.0 us.
 #ifndef MA_SMALL_DECODE_TILES
 #define MA_SMALL_DECODE_TILES 16384
 #endif
 constexpr int64_t kSmallDecodeTiles = MA_SMALL_DECODE_TILES;
+constexpr int64_t kWideRowBytes = 1024;
 
 // A small verify whose row blocks are too many to split runs one workgroup per row block,
 // whose keys one workgroup walks (about 8 us per 1,000 e4m3 keys, 10 in fp16): up to this
@@ -1217,13 +1220,14 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
   // 6k keys, 8 kv heads, D = 96, e4m3) the split measured 69.5 against 64.1 us.
   const bool can_split = (decode || head_dim > 128 ? base : 2 * base) < num_workgroups;
   // a small decode, or a small verify of one 16-row block: the split-KV tiles at the longest
-  // length the caller knows, in tiles of 128 dims. A verify over bf16 KV stays on the
+  // length the caller knows. A verify over bf16 KV stays on the
   // persistent kernel, which keeps P to 16 bits (two bf16 halves) and bf16 V exact.
   bool small = false;
   if (!generic && max_seq_len > 0 && (decode || (kv_dtype != DT_BF16 && (int64_t)max_q_per_seq * a.group <= kAnyRows))) {
     const int64_t row_groups = (a.group + 31) / 32;
     const int64_t tiles = (int64_t)a.batch * a.hkv * row_groups * ((max_seq_len + 31) / 32);
-    small = tiles * (head_dim > 128 ? 2 : 1) <= kSmallDecodeTiles && (decode || can_split || max_seq_len <= kWholeVerifyKeys);
+    const bool twice = head_dim > 128 && (!decode || (int64_t)a.hkv * head_dim * elt > kWideRowBytes);
+    small = tiles * (twice ? 2 : 1) <= kSmallDecodeTiles && (decode || can_split || max_seq_len <= kWholeVerifyKeys);
   }
   if (generic || small) {
     // one workgroup per 16 rows (token, GQA head), its four waves splitting the keys and

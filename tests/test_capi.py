@@ -234,6 +234,10 @@ def test_small_decode_rule_matches_the_library():
     assert ops.decode_kernel(64, 16, 4, 512, 8192) == "any_kernel"        # not a tuned head dim
     assert ops.decode_kernel(8, 64, 8, 128, 8192) == "any_kernel"         # 8 x 8 x 256 = 16384 tiles
     assert ops.decode_kernel(8, 64, 8, 128, 8193) == "splitkv_partial"
+    assert ops.decode_kernel(64, 12, 2, 256, 3000) == "any_kernel"        # 12,032 tiles over K rows of 1 KB
+    assert ops.decode_kernel(16, 16, 4, 256, 6000) == "splitkv_partial"   # 12,032 over 2 KB: they count twice
+    assert ops.decode_kernel(16, 16, 4, 256, 6000, kv_bytes=1) == "any_kernel"
+    assert ops.decode_kernel(10, 16, 4, 256, 6000) == "any_kernel"
 
 
 # 256 compute units, at most two pieces each: rows of a tile x (head dim of the kernel + LSE) fp32
