@@ -13,6 +13,7 @@ constexpr int kAnyWaves = 4;        // waves per workgroup
 constexpr int kAnyRows = 16;        // query rows per wave
 constexpr int kAnyKeys = 16;        // keys per tile
 constexpr int kAnyMaxDim = 512;
+constexpr int kAnyFewPieces = 8;    // up to this many pieces the merge runs 1024 / DP rows a workgroup
 constexpr int kAnyMaxPieces = 512;  // key pieces of one row block (the merge keeps their weights in LDS)
 
 struct AnyArgs {

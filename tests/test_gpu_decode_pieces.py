@@ -191,3 +191,13 @@ def test_d256_between_half_and_all_of_the_small_tiles(kv, hkv, group, batch):
     assert torch.equal(hinted, plain) != pieces
     assert pieces == (hkv * 256 * c["k"].element_size() <= 1024)
     _check(c, hinted, "d256 hinted")
+
+
+@pytest.mark.parametrize("dim,group", [(64, 4), (128, 16), (256, 6), (512, 3), (80, 5)])
+@pytest.mark.parametrize("batch,hkv", [(8, 8), (7, 8), (1, 1)])
+def test_merge_of_few_and_of_many_pieces(dim, group, batch, hkv):
+    """8 pieces a row block (the last count the merge by rows takes), 9, and hundreds."""
+    lens = ([2000, 0, 700, 1] * 2)[:batch] if batch > 1 else [9000]
+    c = _build(29, dim, lens, hkv, group, torch.bfloat16)
+    out = torch.full(c["q"].shape, float("nan"), dtype=torch.float32, device=DEV)
+    _check(c, _run(c, page_size=1, max_seq_len_hint=max(lens), out=out), f"merge batch={batch} hkv={hkv}")
