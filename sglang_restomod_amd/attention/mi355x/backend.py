@@ -123,7 +123,7 @@ class MI355XAttnBackend(_EngineBase):
         self.forward_metadata: Optional[MI355XForwardMetadata] = None
         self._workspace: Optional[torch.Tensor] = None
         self._extend_ws: Optional[torch.Tensor] = None
-        self._captured_ws: list = []  # extend workspaces whose addresses captured graphs hold
+        self._outgrown_ws: list = []  # extend workspaces that a larger one replaced
         # graph buffers (init_cuda_graph_state)
         self._cg_max_bs = 0
         self._cg_row_index: Optional[torch.Tensor] = None
@@ -268,30 +268,36 @@ class MI355XAttnBackend(_EngineBase):
 
     def _workspace_for(self, mode: str, num_tokens: int, hq: int, hkv: int, batch: int) -> torch.Tensor:
         """The split-KV workspace for verify; for extend whichever buffer holds the call's
-        work list and key pieces (the split-KV workspace, or one of its own that grows). A
-        capture never allocates: it takes a buffer that holds at least the work list, and
-        that buffer then lives as long as the backend (the graph keeps its address)."""
+        work list and key pieces (the split-KV workspace, or one of its own). The pieces of
+        one set of kv heads take the same bytes at every call, so its own buffer hardly ever
+        grows, and one that did lives on with the backend: a graph may hold its address, or a
+        kernel on another stream still read it. In a capture, and where the device has no
+        room, a call without a buffer for its pieces runs whole row tiles."""
         ws = self.splitkv_workspace()
         if mode == MODE_VERIFY:
             return ws
         want = ops.extend_split_workspace_bytes(num_tokens, hq, hkv, batch, self.head_dim)
-        if ws.numel() >= want:
-            return ws
         own = self._extend_ws
-        capturing = torch.cuda.is_current_stream_capturing()
-        if own is None or own.numel() < want:
-            if capturing:
-                need = ops.extend_workspace_bytes(num_tokens, hq, hkv, batch)
-                if ws.numel() >= need and (own is None or own.numel() < ws.numel()):
-                    return ws
-                if own is None or own.numel() < need:
-                    raise RuntimeError(f"an extend of {num_tokens} tokens needs {need} workspace bytes; "
-                                       "capture smaller batches")
-            else:
-                own = self._extend_ws = torch.empty(want, dtype=torch.uint8, device=self.device)
-        if capturing and not any(own is kept for kept in self._captured_ws):
-            self._captured_ws.append(own)
-        return own
+        for buf in (ws, own):
+            if buf is not None and buf.numel() >= want:
+                return buf
+        largest = ws if own is None or own.numel() < ws.numel() else own
+        need = ops.extend_workspace_bytes(num_tokens, hq, hkv, batch)
+        if torch.cuda.is_current_stream_capturing():
+            if largest.numel() < need:
+                raise RuntimeError(f"an extend of {num_tokens} tokens needs {need} workspace bytes; "
+                                   "capture smaller batches")
+            return largest
+        try:
+            buf = torch.empty(-(-want >> 20) << 20, dtype=torch.uint8, device=self.device)
+        except torch.OutOfMemoryError:
+            if largest.numel() < need:
+                raise
+            return largest
+        if own is not None:
+            self._outgrown_ws.append(own)
+        self._extend_ws = buf
+        return buf
 
     def init_cuda_graph_state(self, max_bs: int, max_num_tokens: int, kv_indices_buf=None) -> None:
         dev = self.device

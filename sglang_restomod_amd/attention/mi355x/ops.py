@@ -163,18 +163,31 @@ def _i64(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     return t.to(torch.int64).contiguous()
 
 
+# Buffers that a larger one of their stream has replaced: a captured graph may hold their
+# addresses. Each buffer is half again as large as the last, so all of a stream's take less
+# than three times its largest.
+_OUTGROWN_WORKSPACES: list = []
+
+
+def _mib(nbytes: int) -> int:
+    return -(-nbytes >> 20) << 20  # whole MiB
+
+
 def workspace_buffer(device: torch.device, nbytes: int, stream: Optional[int] = None) -> torch.Tensor:
     """A growable byte buffer per (device, stream), shared by the entry points that take a
     workspace; calls on one stream are ordered, so they can share it. ``stream``: the
-    current stream's handle when the caller already has it."""
+    current stream's handle when the caller already has it. It is not initialised, and lives
+    until the process ends."""
     if nbytes <= 0:
         return None
     key = (str(device), _stream_ptr(device) if stream is None else stream)
     buf = _WORKSPACES.get(key)
     if buf is None or buf.numel() < nbytes:
-        cap = 1 << max(20, (nbytes - 1).bit_length())
-        buf = torch.zeros(cap, dtype=torch.uint8, device=device)
-        _WORKSPACES[key] = buf
+        least = 1 << 20 if buf is None else 3 * buf.numel() // 2
+        new = torch.empty(_mib(max(nbytes, least)), dtype=torch.uint8, device=device)
+        if buf is not None:
+            _OUTGROWN_WORKSPACES.append(buf)
+        _WORKSPACES[key] = buf = new
     return buf
 
 
@@ -516,7 +529,11 @@ def paged_extend_forward(
     stream = _stream_ptr(dev)
     if workspace is None:
         nbytes = lib.ma_extend_split_workspace_bytes(T, Hq, Hkv, B, D)
-        ws = workspace_buffer(dev, nbytes, stream)
+        try:
+            ws = workspace_buffer(dev, nbytes, stream)
+        except torch.OutOfMemoryError:  # no room for key pieces: whole row tiles
+            nbytes = lib.ma_extend_workspace_bytes(T, Hq, Hkv, B)
+            ws = workspace_buffer(dev, nbytes, stream)
     else:
         nbytes = lib.ma_extend_workspace_bytes(T, Hq, Hkv, B)
         if workspace.dtype != torch.uint8 or workspace.device != dev or workspace.numel() < nbytes:

@@ -284,3 +284,90 @@ def test_native_kv_write_matches_the_pool_write(kv_dtype, monkeypatch):
     assert engines[1].pool.writes == 0 and engines[0].pool.writes == 2
     for x, y in zip(outs[0], outs[1]):
         assert torch.equal(x, y)
+
+
+def test_extend_in_a_hip_graph_between_other_extends():
+    """A captured extend keeps its workspace (with its key pieces) while eager extends of other
+    sizes run between the replays."""
+    print("[case] extend graph", flush=True)
+    gen = torch.Generator().manual_seed(9)
+    eng = fakes.Engine(DEV, hq=32, hkv=8, head_dim=128, kv_dtype=torch.bfloat16, pool_size=30000, max_reqs=12,
+                       context_len=4096)
+    layer = _layer(torch.bfloat16, 32, 8, 128)
+    be = _backend(eng)
+    be.init_cuda_graph_state(max_bs=4, max_num_tokens=1024)
+
+    def eager(rows, ext):
+        fb = eng.batch("EXTEND", rows, new_tokens=ext)
+        T = sum(ext)
+        q, k, v = _rand(gen, T, 32 * 128), _rand(gen, T, 8, 128), _rand(gen, T, 8, 128)
+        be.init_forward_metadata(fb)
+        out = be.forward_extend(q, k, v, layer, fb)
+        _check_extend(eng, layer, fb, q, out, fb.before, ext, f"extend {ext}")
+
+    eager([4, 5], [300, 40])  # the workspace exists before the capture
+    rows, ext = [0, 1], [700, 90]
+    fb = eng.batch("EXTEND", rows, new_tokens=ext)
+    T = sum(ext)
+    eng.fill(0, fb.out_cache_loc, _rand(gen, T, 8, 128), _rand(gen, T, 8, 128), layer)
+    q = _rand(gen, T, 32 * 128)
+    be.init_forward_metadata_capture_cuda_graph(2, T, fb.req_pool_indices, fb.seq_lens, None, fb.forward_mode, None)
+    md = be.forward_metadata
+    held = be._extend_ws
+    assert held is not None
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = be.forward_extend(q, None, None, layer, fb, save_kv_cache=False)
+    for step, other in enumerate([[7], [64, 2000], [5] * 3]):
+        eager(list(range(4, 4 + len(other))), other)
+        q.copy_(_rand(gen, T, 32 * 128))
+        be.forward_metadata = md
+        graph.replay()
+        torch.cuda.synchronize()
+        _check_extend(eng, layer, fb, q, out, [0, 0], ext, f"replay {step}")
+        assert be._extend_ws is held
+
+
+def test_the_shared_workspace_of_a_graph_outlives_its_growth():
+    """A decode captured on the stream's shared buffer replays after an extend on that stream
+    took a larger one, and leaves memory allocated since alone."""
+    from sglang_restomod_amd.attention.mi355x import ops
+
+    print("[case] shared workspace of a graph", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(2)
+    n, hq, hkv = 700, 12, 3
+    k, v = (torch.randn(n + 1, hkv, 128, generator=g, device=DEV, dtype=torch.float32).half() for _ in range(2))
+    table = (torch.randperm(n, generator=g, device=DEV) + 1).to(torch.int32).view(1, n)
+    q = torch.randn(200, hq, 128, generator=g, device=DEV).half()
+    i32 = dict(dtype=torch.int32, device=DEV)
+    seq = torch.tensor([n], **i32)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    out = torch.empty(1, hq, 128, device=DEV, dtype=torch.float16)
+
+    def decode():  # without a bound: the persistent kernel, with descriptors and partials in the buffer
+        ops.grouped_decode_forward(q[:1], k, v, table, seq, softmax_scale=128 ** -0.5, out=out, page_size=1)
+
+    key = (str(q.device), stream.cuda_stream)
+    ops._WORKSPACES.pop(key, None)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        decode()
+        want = out.clone()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            decode()
+        before = ops._WORKSPACES[key]
+        assert ops.paged_extend_forward(q, k, v, table, seq, torch.tensor([0, 200], **i32),
+                                        torch.tensor([500], **i32), softmax_scale=128 ** -0.5,
+                                        page_size=1).isfinite().all()
+        assert ops._WORKSPACES[key].numel() > before.numel()
+        size = before.numel()
+        del before
+        since = torch.zeros(size, dtype=torch.uint8, device=DEV)  # would take the block, had it been freed
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
+            assert not bool(since.any())
