@@ -2,6 +2,9 @@
 
 from __future__ import annotations
 
+import re
+from pathlib import Path
+
 from sglang_restomod_amd import isa_check
 
 KERNEL = """_ZN2ma15splitkv_partialEv:
@@ -67,9 +70,21 @@ def test_out_of_line_block_is_checked_in_execution_order(tmp_path):
 
 
 def test_scalar_cache_writes_are_found(tmp_path):
-    body = "\ts_store_dword s0, s[2:3], 0x0\n\ts_dcache_wb\n\tglobal_store_dword v0, v1, s[0:1]\n"
-    found = isa_check.scalar_cache_writes(_write(tmp_path, body))
-    assert len(found) == 2 and all(f.startswith("s_") for f in found)
+    scalar = isa_check.SCALAR_PREFIX
+    for op in isa_check.SCALAR_WRITE_OPS:
+        body = f"\t{scalar}{op}_dword s0, s[2:3], 0x0\n\t{scalar}{op}\n\tglobal_store_dword v0, v1, s[0:1]\n"
+        found = isa_check.scalar_cache_writes(_write(tmp_path, body))
+        assert found == [f"{scalar}{op}_dword", f"{scalar}{op}"]
+
+
+def test_no_source_names_a_scalar_cache_write():
+    root = Path(__file__).resolve().parent.parent
+    named = re.compile(r"\b" + isa_check.SCALAR_PREFIX + "(?:" + "|".join(isa_check.SCALAR_WRITE_OPS) + ")")
+    files = [p for d in ("sglang_restomod_amd", "include", "tests", "oracle", "perf") for p in (root / d).rglob("*")
+             if p.suffix in (".py", ".hip", ".h")]
+    files += [root / "bench.py", root / "__graft_entry__.py"]
+    assert len(files) > 50
+    assert [str(p) for p in files if named.search(p.read_text())] == []
 
 
 def test_built_library_sources_are_clean():
