@@ -90,15 +90,25 @@ CASES = [  # prefix, ext, heads, kv heads, dim, q dtype, kv dtype, causal, windo
     ([900, 64], [40, 97], 8, 2, 512, BF16, E4M3, False, -1),
     ([700], [50], 8, 1, 320, F16, E5M2, True, -1),
     ([700, 5], [50, 300], 16, 4, 272, BF16, BF16, True, -1),
-    ([255, 0], [1, 256], 32, 8, 128, BF16, BF16, True, -1),    # pieces of the least length
-    ([500], [2100], 8, 1, 128, BF16, BF16, True, -1),          # over 64 row tiles: the plan kernel lists the pieces
-    ([3000] * 40 + [0] * 30, [5] * 40 + [0, 2] * 15, 16, 2, 128, F16, F16, True, -1),  # over 64 sequences
+    ([700, 0], [1, 256], 32, 8, 128, BF16, BF16, True, -1),    # pieces of the least length, and whole tiles
+    ([500], [2100], 8, 1, 128, BF16, BF16, True, -1),          # over 64 row tiles: two per lane of the planning wave
+    # the plan kernel lists the pieces: over 128 row tiles, or over 64 sequences
+    ([600], [2100], 16, 1, 128, BF16, BF16, True, -1),
+    ([3000], [2040], 16, 1, 128, BF16, E4M3, True, 2500),
+    ([3000] * 40 + [0] * 30, [5] * 40 + [0, 2] * 15, 16, 2, 128, F16, F16, True, -1),
+    ([2500, 7] + [40] * 68, [60, 200] + [3] * 68, 8, 1, 64, BF16, E5M2, True, -1),
+    ([2500, 0] + [40] * 68, [90, 64] + [0, 9] * 34, 12, 2, 256, BF16, BF16, True, -1),
+    ([4000] + [100] * 70, [33] + [2] * 70, 6, 1, 192, F16, E4M3, False, -1),
+    ([2500] * 2 + [30] * 70, [40, 3] + [1] * 70, 8, 1, 96, BF16, BF16, True, 900),
+    ([1800, 300] + [20] * 66, [70, 30] + [2] * 66, 8, 2, 512, BF16, BF16, True, -1),
+    ([1500] + [64] * 80, [33] + [4, 1] * 40, 4, 1, 320, F16, F16, True, 400),
+    ([40, 1500] + [9] * 70, [64, 50] + [3] * 70, 8, 2, 512, BF16, E4M3, False, -1),
 ]
 
 
 @pytest.mark.parametrize("prefix,ext,heads,hkv,dim,q_dtype,kv,causal,window", CASES)
 def test_pieces_match_float64_and_whole_tiles(prefix, ext, heads, hkv, dim, q_dtype, kv, causal, window):
-    print(f"[case] pieces prefix={prefix} ext={ext} h={heads}/{hkv} d={dim} q={q_dtype} kv={kv} causal={causal} "
+    print(f"[case] pieces of {len(prefix)} prefix={prefix[:5]} ext={ext[:5]} h={heads}/{hkv} d={dim} q={q_dtype} kv={kv} causal={causal} "
           f"window={window}", flush=True)
     ops = _ops()
     c = _make(prefix, ext, heads, hkv, dim, q_dtype, kv)
@@ -118,6 +128,10 @@ def test_pieces_match_float64_and_whole_tiles(prefix, ext, heads, hkv, dim, q_dt
     # repository's bound for v_scale near 1
     for out in outs:
         assert float((out.double() - ref).abs().max()) < 4e-3
+    listed, cut, pieces = _cut_tiles(large, T, heads, hkv, dim, B)
+    print(f"[plan] listed={listed} cut={cut} pieces={pieces}", flush=True)
+    assert cut > 0 and pieces > cut
+    assert listed == (B > 64 or -(-T * (heads // hkv) // (256 if dim <= 128 else 128)) + B > 128)
     # the pieces sum the same products in another order
     whole, cut = ((o.double() - ref).norm() for o in outs)
     assert float(cut) <= 1.1 * float(whole) + 1e-9
@@ -175,8 +189,9 @@ def test_overlapping_query_ranges_stay_inside_the_plan():
 
 
 @pytest.mark.parametrize("prefix,ext,heads,hkv,dim,cuts", [
-    ([60] * 4, [180] * 4, 16, 4, 192, False),   # partials cost more than the 9 key tiles they would level
-    ([60] * 4, [180] * 4, 16, 4, 256, False),
+    # partials cost more than the key tiles they would level (9 at most)
+    ([40, 60, 34, 42], [266, 112, 118, 237], 16, 4, 192, False),
+    ([40, 60, 34, 42], [266, 112, 118, 237], 16, 4, 256, False),
     ([3000] * 4, [180] * 4, 16, 4, 256, True),
     ([900] * 4, [180] * 4, 32, 8, 128, True),
     ([100] * 130, [10] * 130, 8, 1, 128, False),  # two key tiles each

@@ -26,6 +26,16 @@ CASES = [  # prefix, new tokens, heads, kv heads, dim, q dtype, kv dtype, window
     ([4000], [4], 8, 1, 64, BF16, E5M2, -1, 4),
     ([3, 5, 2], [1, 2, 3], 8, 8, 128, BF16, BF16, -1, 3),          # fewer tiles than a workgroup has waves
     ([31] * 70, [2] * 70, 8, 2, 128, F16, F16, -1, 2),             # over 64 sequences: two scans
+    # with a bound, key pieces at the tuned head dims (one 16-row block over fp16 or fp8): empty
+    # sequences, a window, rows past the hint, and whole row blocks too many to split
+    ([6000, 0, 700], [4, 2, 1], 32, 8, 128, F16, F16, -1, 4),
+    ([6000, 0, 700], [4, 2, 0], 32, 8, 128, BF16, E4M3, 900, 4),
+    ([5000, 30], [2, 1], 32, 8, 64, BF16, E5M2, -1, 2),
+    ([4000, 900], [2, 3], 16, 4, 256, BF16, E4M3, -1, 3),
+    ([4000, 900], [1, 4], 16, 4, 256, F16, F16, -1, 4),
+    ([3000, 2000, 9], [9, 3, 1], 32, 8, 128, F16, F16, -1, 3),
+    ([3000, 10], [40, 2], 8, 8, 64, BF16, E4M3, -1, 16),
+    ([300, 1200] * 20, [4, 2] * 20, 32, 8, 128, F16, F16, -1, 4),
     # any-head-dim pieces: rows within and past the hint, empty sequences, windows
     ([6000], [4], 16, 4, 512, BF16, BF16, -1, 4),
     ([6000, 0, 70], [4, 3, 0], 16, 4, 512, F16, F16, -1, 4),
@@ -105,20 +115,23 @@ def test_a_long_sequence_among_many_short_ones_is_shared(prefix, new, dim, kv):
     assert torch.equal(got, _run(case, prefix, -1, new, None))
 
 
-@pytest.mark.parametrize("prefix,heads,hkv,dim,padded,bounded", [
-    ([700] * 16, 16, 4, 512, 512, True), ([600] * 16, 16, 4, 192, 256, False), ([700] * 4, 32, 8, 96, 128, True),
+@pytest.mark.parametrize("prefix,heads,hkv,dim,padded,bounded,kv", [
+    ([700] * 16, 16, 4, 512, 512, True, BF16), ([600] * 16, 16, 4, 192, 256, False, BF16),
+    ([700] * 4, 32, 8, 96, 128, True, E4M3), ([700] * 4, 32, 8, 128, 128, True, F16),
+    ([700] * 16, 16, 4, 256, 256, True, E5M2), ([700] * 8, 32, 8, 64, 64, True, E4M3),
 ])
-def test_verify_pieces_cover_the_chip_once(prefix, heads, hkv, dim, padded, bounded):
+def test_verify_pieces_cover_the_chip_once(prefix, heads, hkv, dim, padded, bounded, kv):
     """One piece per CU at most, counted in the partial slots the call writes."""
     from sglang_restomod_amd.attention.mi355x import ops
 
     print(f"[case] verify pieces {len(prefix)} x {prefix[0]} h={heads}/{hkv} d={dim}", flush=True)
-    case = _case(prefix, [2] * len(prefix), heads, hkv, dim, BF16, BF16)
+    case = _case(prefix, [2] * len(prefix), heads, hkv, dim, F16 if kv == F16 else BF16, kv)
     ws = ops.splitkv_workspace(torch.device(DEV), head_dim=dim).fill_(0xA5)
     _run(case, prefix, -1, 2, prefix[0] + 2 if bounded else None, ws)
-    slots = ws.numel() // (16 * (padded + 1) * 4)
-    used = (ws[:slots * 16 * padded * 4].view(slots, -1) != 0xA5).any(1)
+    # twice as many slots as CUs, from the workspace's start (the tuned dims' workspace holds more)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
+    slots = 2 * cus
+    used = (ws[:slots * 16 * padded * 4].view(slots, -1) != 0xA5).any(1)
     assert len(prefix) * hkv < int(used.sum()) <= cus
 
 
