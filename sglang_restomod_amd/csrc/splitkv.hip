@@ -341,11 +341,14 @@ __global__ __launch_bounds__(256, 1) void splitkv_partial(const SplitKVArgs args
   __shared__ __attribute__((aligned(16))) unsigned char kring[kWaves][S][kStage];
 
   const int lane = threadIdx.x & 63;
-  // Wave-uniform values in scalar registers where vector registers are short (two row blocks,
-  // D = 256: 300 -> 100 register-file moves, 1-2% faster); with one row block at D = 128 the
-  // fp8 decode measured 1.4% slower that way (774 against 785 us on 128 sequences).
+  // Wave-uniform values in scalar registers where vector registers are short (D = 256: 300 ->
+  // 100 register-file moves, 1-2% faster). Below, scalar registers are the ones that run out:
+  // with two row blocks 217-221 of them spilled at D = 64, and at D = 128 over fp8 (16 with a
+  // vector index), 87-90 at D = 128 over 16-bit KV (10), and verifies of 32 rows took 2% longer at
+  // D = 64 over 16-bit KV, 1% in fp16 and 0.4% in bf16 at D = 128, the same over fp8. With one
+  // row block the D = 128 fp8 decode took 1.4% longer (785 against 774 us on 128 sequences).
   int wave = threadIdx.x >> 6;
-  if constexpr (NB == 2 || D == 256) wave = __builtin_amdgcn_readfirstlane(wave);
+  if constexpr (D == 256) wave = __builtin_amdgcn_readfirstlane(wave);
   const int c = lane & 15;
   const int j = lane >> 4;
   const int W = blockIdx.x * kWaves + wave;
