@@ -403,7 +403,7 @@ def _measure(index, steps, warmup, cpu_seconds, kv_format="e4m3"):
     if w.mode == "decode":
         from sglang_restomod_amd.attention.mi355x import ops
 
-        res["kernel"] = ops.decode_kernel(w.batch, w.heads, w.heads_kv, w.dim, max(w.seq_lens_cpu), w.k_pool.element_size())
+        res["kernel"] = ops.decode_kernel(w.batch, w.heads, w.heads_kv, w.dim, max(w.seq_lens_cpu), w.k_pool.dtype)
     if w.mode != "extend":
         # the same number of K and V rows, gathered from random slots with no arithmetic
         row_bytes = w.dim * w.k_pool.element_size()

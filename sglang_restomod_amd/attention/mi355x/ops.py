@@ -33,24 +33,25 @@ HEAD_DIM_MULTIPLE = 16
 
 
 # A decode with at most this many 32-key split-KV tiles (over every sequence, kv head and
-# 32-row group, at the caller's length bound; a tile of 256 dims counts twice over K rows of
-# more than 1 KB) runs as key pieces on the any-head-dim kernel (MA_SMALL_DECODE_TILES in
+# 32-row group, at the caller's length bound; a tile of 256 dims counts twice over bf16,
+# and over K rows of more than 1 KB) runs as key pieces on the any-head-dim kernel (MA_SMALL_DECODE_TILES in
 # csrc/splitkv.hip).
 SMALL_DECODE_TILES = 16384
 
 
 def decode_kernel(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int,
-                  max_seq_len_hint: Optional[int], kv_bytes: int = 2) -> str:
+                  max_seq_len_hint: Optional[int], kv_dtype: torch.dtype = torch.bfloat16) -> str:
     """Which kernel carries a decode call: ``"splitkv_partial"`` (the persistent split-KV
     kernel) or ``"any_kernel"`` (head dims other than 64/128/256, and small decodes given a
-    length bound). The library makes the same choice. ``kv_bytes``: bytes of a K element."""
+    length bound). The library makes the same choice."""
     if int(head_dim) not in TUNED_HEAD_DIMS:
         return "any_kernel"
     if not max_seq_len_hint or max_seq_len_hint <= 0:
         return "splitkv_partial"
     group = int(num_q_heads) // int(num_kv_heads)
     tiles = int(batch) * int(num_kv_heads) * ((group + 31) // 32) * ((int(max_seq_len_hint) + 31) // 32)
-    twice = int(head_dim) > 128 and int(num_kv_heads) * int(head_dim) * int(kv_bytes) > 1024
+    twice = int(head_dim) > 128 and (
+        kv_dtype == torch.bfloat16 or int(num_kv_heads) * int(head_dim) * kv_dtype.itemsize > 1024)
     return "any_kernel" if tiles * (2 if twice else 1) <= SMALL_DECODE_TILES else "splitkv_partial"
 
 

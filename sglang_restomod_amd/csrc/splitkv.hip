@@ -1120,10 +1120,11 @@ extern "C" size_t ma_splitkv_workspace_bytes(int num_workgroups, int head_dim) {
 // 512-8192: the pieces are faster up to 16384 tiles (B = 8 at 8192 keys: 51.8 against
 // 61.5 us per call; B = 32 at 2048: 45.6 against 59.4) and slower beyond (B = 16 at 8192:
 // 110 against 101); B = 1 at 512 keys takes 16.5 us per call either way. At 256 dims over
-// K rows of more than 1 KB (and for a verify) a tile counts twice, pieces against split-KV: 16 / 4 heads, bf16,
-// 16 x 6k keys (12k tiles) 85 / 78 us, 30k keys x 4 (15k) 100 / 91, against e4m3 41 / 47 and
-// 49 / 55, 12 / 2 heads, bf16, 64 x 3k (12k) 71 / 78 and 8 sequences, one of 30k keys and the
-// rest of 100 (15k), 29 / 42. A verify of one 16-row block over fp16 or fp8 KV
+// K rows of more than 1 KB (and for a verify) a tile counts twice, pieces against split-KV:
+// 16 / 4 heads, fp16, 16 x 6k keys (12k tiles) 84 / 77 us, 30k keys x 4 (15k) 100 / 91, against
+// e4m3 41 / 47 and 49 / 55, 12 / 2 heads, fp16, 64 x 3k (12k) 70 / 78 and 8 sequences, one of
+// 30k keys and the rest of 100 (15k), 29 / 42. It does so over any bf16 rows too (71 / 78 and
+// 29 / 42 there): the persistent kernel keeps P to 16 bits. A verify of one 16-row block over fp16 or fp8 KV
 // is the same work: 32 / 8 heads, 16 x 1.5k keys 24.8 against 32.0 us.
 #ifndef MA_SMALL_DECODE_TILES
 #define MA_SMALL_DECODE_TILES 16384
@@ -1229,7 +1230,7 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
   if (!generic && max_seq_len > 0 && (decode || (kv_dtype != DT_BF16 && (int64_t)max_q_per_seq * a.group <= kAnyRows))) {
     const int64_t row_groups = (a.group + 31) / 32;
     const int64_t tiles = (int64_t)a.batch * a.hkv * row_groups * ((max_seq_len + 31) / 32);
-    const bool twice = head_dim > 128 && (!decode || (int64_t)a.hkv * head_dim * elt > kWideRowBytes);
+    const bool twice = head_dim > 128 && (!decode || kv_dtype == DT_BF16 || (int64_t)a.hkv * head_dim * elt > kWideRowBytes);
     small = tiles * (twice ? 2 : 1) <= kSmallDecodeTiles && (decode || can_split || max_seq_len <= kWholeVerifyKeys);
   }
   if (generic || small) {

@@ -8,6 +8,7 @@ import os
 import re
 
 import pytest
+import torch
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -234,9 +235,12 @@ def test_small_decode_rule_matches_the_library():
     assert ops.decode_kernel(64, 16, 4, 512, 8192) == "any_kernel"        # not a tuned head dim
     assert ops.decode_kernel(8, 64, 8, 128, 8192) == "any_kernel"         # 8 x 8 x 256 = 16384 tiles
     assert ops.decode_kernel(8, 64, 8, 128, 8193) == "splitkv_partial"
-    assert ops.decode_kernel(64, 12, 2, 256, 3000) == "any_kernel"        # 12,032 tiles over K rows of 1 KB
-    assert ops.decode_kernel(16, 16, 4, 256, 6000) == "splitkv_partial"   # 12,032 over 2 KB: they count twice
-    assert ops.decode_kernel(16, 16, 4, 256, 6000, kv_bytes=1) == "any_kernel"
+    # 12,032 tiles at 256 dims: they count twice over bf16 and over K rows of more than 1 KB
+    for heads, hkv, batch, bound in ((12, 2, 64, 3000), (16, 4, 16, 6000)):
+        want = {torch.bfloat16: "splitkv_partial", torch.float16: "any_kernel" if hkv == 2 else "splitkv_partial",
+                torch.float8_e4m3fn: "any_kernel", torch.float8_e5m2: "any_kernel"}
+        for kv, kernel in want.items():
+            assert ops.decode_kernel(batch, heads, hkv, 256, bound, kv) == kernel
     assert ops.decode_kernel(10, 16, 4, 256, 6000) == "any_kernel"
 
 

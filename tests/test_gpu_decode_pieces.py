@@ -177,19 +177,20 @@ def test_pieces_in_a_hip_graph_replay_with_new_lengths():
 
 
 @pytest.mark.parametrize("kv,hkv,group,batch", [
-    (torch.float8_e4m3fn, 2, 6, 4), (torch.bfloat16, 2, 6, 4), (torch.bfloat16, 4, 4, 2), (torch.float8_e5m2, 4, 4, 2),
+    (torch.float8_e4m3fn, 2, 6, 4), (torch.float16, 2, 6, 4), (torch.bfloat16, 2, 6, 4), (torch.float16, 4, 4, 2),
+    (torch.float8_e5m2, 4, 4, 2),
 ])
 def test_d256_between_half_and_all_of_the_small_tiles(kv, hkv, group, batch):
     """About 15,000 tiles of 256 dims: key pieces over K rows of 1 KB, the persistent kernel
-    over longer ones. Without a bound it is always the persistent kernel, so equal bits (the
+    over longer ones and over bf16. Without a bound it is always the persistent kernel, so equal bits (the
     two share the keys out differently) tell which one ran."""
     c = _build(17, 256, [60000] + [5] * (batch - 1), hkv, group, kv)
     out32 = [torch.empty(c["q"].shape, dtype=torch.float32, device=DEV) for _ in range(2)]
     hinted = _run(c, page_size=1, out=out32[0], max_seq_len_hint=60000)
     plain = _run(c, page_size=1, out=out32[1])
-    pieces = _ops().decode_kernel(batch, hkv * group, hkv, 256, 60000, c["k"].element_size()) == "any_kernel"
+    pieces = _ops().decode_kernel(batch, hkv * group, hkv, 256, 60000, kv) == "any_kernel"
     assert torch.equal(hinted, plain) != pieces
-    assert pieces == (hkv * 256 * c["k"].element_size() <= 1024)
+    assert pieces == (kv != torch.bfloat16 and hkv * 256 * kv.itemsize <= 1024)
     _check(c, hinted, "d256 hinted")
 
 
