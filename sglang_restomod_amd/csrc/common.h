@@ -275,4 +275,30 @@ __device__ __forceinline__ int64_t kv_row(const TokenTable& t, int64_t seq_row, 
   return ((int64_t)page << t.page_shift) | (int64_t)(pos & ((1 << t.page_shift) - 1));
 }
 
+// x of the lane that DPP control CTRL names, in the rows of 16 lanes that ROWS selects; 0 where
+// there is none.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp0(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int64_t dpp0(int64_t x) {
+  const uint32_t lo = (uint32_t)dpp0<CTRL, ROWS>((int)(uint32_t)x);
+  const uint32_t hi = (uint32_t)dpp0<CTRL, ROWS>((int)(x >> 32));
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+// Inclusive prefix sum over the wave's lanes, by DPP moves (a few cycles a step; a cross-lane
+// read through LDS takes over a hundred).
+template <typename T>
+__device__ __forceinline__ T wave_scan(T x) {
+  x += dpp0<0x111, 0xf>(x);  // row_shr:1, 2, 4, 8 within rows of 16 lanes
+  x += dpp0<0x112, 0xf>(x);
+  x += dpp0<0x114, 0xf>(x);
+  x += dpp0<0x118, 0xf>(x);
+  x += dpp0<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
+  x += dpp0<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+
 }  // namespace ma

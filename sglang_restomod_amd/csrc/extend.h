@@ -110,21 +110,7 @@ __device__ __forceinline__ float pieces_cost(float all, float n, float longest, 
   return fmaxf(longest + kStart, mean * ceilf(n / shares)) + slot_cost * split / shares;
 }
 
-// Inclusive prefix sum over the wave's lanes, and the wave's maximum, of values >= 0, by
-// DPP moves (a few cycles a step; a cross-lane read through LDS takes over a hundred).
-template <int CTRL, int ROWS>
-__device__ __forceinline__ int dpp0(int x) {  // x of another lane, 0 where there is none
-  return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false);
-}
-__device__ __forceinline__ int wave_scan(int x) {
-  x += dpp0<0x111, 0xf>(x);  // row_shr:1, 2, 4, 8 within rows of 16 lanes
-  x += dpp0<0x112, 0xf>(x);
-  x += dpp0<0x114, 0xf>(x);
-  x += dpp0<0x118, 0xf>(x);
-  x += dpp0<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
-  x += dpp0<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
-  return x;
-}
+// The wave's maximum of values >= 0.
 __device__ __forceinline__ int wave_max(int x) {
   x = max(x, dpp0<0x111, 0xf>(x));
   x = max(x, dpp0<0x112, 0xf>(x));

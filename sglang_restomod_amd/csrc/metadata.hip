@@ -122,11 +122,6 @@ struct LengthsArgs {
 };
 constexpr int kLenThreads = 1024;
 
-template <int CTRL, int ROWS>
-__device__ __forceinline__ int len_dpp(int x) {
-  return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false);
-}
-
 __global__ __launch_bounds__(kLenThreads) void lengths_kernel(const LengthsArgs a) {
   __shared__ int sums[kLenThreads / 64];
   const int tid = threadIdx.x;
@@ -146,13 +141,7 @@ __global__ __launch_bounds__(kLenThreads) void lengths_kernel(const LengthsArgs 
       gptr_mut(a.seq_out)[b] = a.seq ? max(get(a.seq, a.seq64, b), n) : n;
       if (a.prefix_out) gptr_mut(a.prefix_out)[b] = pre;
     }
-    int x = ext;
-    x += len_dpp<0x111, 0xf>(x);  // row_shr:1, 2, 4, 8, then row_bcast:15 and 31
-    x += len_dpp<0x112, 0xf>(x);
-    x += len_dpp<0x114, 0xf>(x);
-    x += len_dpp<0x118, 0xf>(x);
-    x += len_dpp<0x142, 0xa>(x);
-    x += len_dpp<0x143, 0xc>(x);
+    const int x = wave_scan(ext);
     if ((tid & 63) == 63) sums[wave] = x;
     __syncthreads();
     int before = 0, all = 0;

@@ -158,23 +158,6 @@ __device__ __forceinline__ int64_t readlane_i64(int64_t v, int lane) {
   return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
-// Inclusive prefix sum over the wave's lanes, by DPP moves.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ int64_t dpp0_i64(int64_t x) {  // x of another lane, 0 where there is none
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, CTRL, ROWS, 0xf, false);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(x >> 32), CTRL, ROWS, 0xf, false);
-  return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-__device__ __forceinline__ int64_t wave_scan_i64(int64_t x) {
-  x += dpp0_i64<0x111, 0xf>(x);  // row_shr:1, 2, 4, 8 within rows of 16 lanes
-  x += dpp0_i64<0x112, 0xf>(x);
-  x += dpp0_i64<0x114, 0xf>(x);
-  x += dpp0_i64<0x118, 0xf>(x);
-  x += dpp0_i64<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
-  x += dpp0_i64<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
-  return x;
-}
-
 // The sequence holding global tile t and t's offset in it.
 template <int TS>
 __device__ __forceinline__ void scan_work(const SplitKVArgs& a, int64_t t, int& b_at, int64_t& off_at) {
@@ -183,7 +166,7 @@ __device__ __forceinline__ void scan_work(const SplitKVArgs& a, int64_t t, int& 
   for (int b0 = 0; b0 < a.batch; b0 += 64) {
     const int b = b0 + lane;
     const int64_t w = b < a.batch ? seq_work<TS>(a, b) : 0;
-    const int64_t inc = wave_scan_i64(w);
+    const int64_t inc = wave_scan(w);
     const int64_t chunk = readlane_i64(inc, 63);
     if (base + chunk > t) {
       const int L = __builtin_ctzll(__builtin_amdgcn_ballot_w64(base + inc > t));
@@ -228,7 +211,7 @@ __device__ __forceinline__ int64_t scan_total(const SplitKVArgs& a, int W, int64
       work = (int64_t)g.nt * g.rg_real * a.hkv;
       zero = g.nt == 0 && g.ntok > 0 && (b % a.nwaves) == W;
     }
-    upto = base + wave_scan_i64(work);
+    upto = base + wave_scan(work);
     base = readlane_i64(upto, 63);
     uint64_t zm = __builtin_amdgcn_ballot_w64(zero);
     while (zm) {
