@@ -196,10 +196,13 @@ size_t ma_extend_workspace_bytes(int64_t num_tokens, int num_q_heads, int num_kv
 
 /*
  * Bytes of workspace with which ma_paged_extend can also cut row tiles into key pieces
- * (at least ma_extend_workspace_bytes; equal to it where a call has row tiles enough to
- * fill the chip several times). The pieces' partial results take 128 KB or less per piece
- * and kv head, at most two pieces per compute unit. With a smaller workspace the call runs
- * whole row tiles; the result is the same up to rounding. 0 for bad arguments.
+ * (at least ma_extend_workspace_bytes; equal to it where a call's row tiles fill the chip:
+ * as many sequences as compute units per kv head, or that many tiles of their tokens). The
+ * pieces' partial results take up to 129 KB each at head dims up to 256 (65 KB at 64) and
+ * 257 KB above, at most two pieces per compute unit over all kv heads: 68 MB and 135 MB on
+ * 256 compute units, whatever the batch. With a smaller workspace the call runs whole row
+ * tiles; the result is the same up to rounding. 0 for bad arguments. Without a device the
+ * sizes are those of 256 compute units.
  */
 size_t ma_extend_split_workspace_bytes(int64_t num_tokens, int num_q_heads, int num_kv_heads, int batch,
                                        int head_dim);
@@ -220,7 +223,8 @@ size_t ma_extend_split_workspace_bytes(int64_t num_tokens, int num_q_heads, int 
  *   _paged_adapter.py:605-606).
  *   workspace: ma_extend_workspace_bytes(num_tokens, ...) bytes or more, 256-byte aligned,
  *   no initialisation; with ma_extend_split_workspace_bytes(...) bytes a call with few row
- *   tiles also splits their keys over workgroups. Calls that overlap in time must use different workspaces.
+ *   tiles also splits their keys over workgroups. Calls that overlap in time must use
+ *   different workspaces.
  *   The new tokens' K/V must already be in the pools.
  *   out [num_tokens, num_q_heads, head_dim] in out_dtype (q_dtype or MA_DT_F32).
  */

@@ -29,14 +29,14 @@ struct ExtendMerge {
   int slot, parts; // its pieces' slots: slot .. slot + parts - 1
 };
 struct ExtendPieces {
-  const ExtendPiece* list;  // the plan kernel's list, or null: each workgroup plans (plan_direct)
+  const ExtendPiece* list;  // the plan kernel's list, or null
   ExtendMerge* merges;      // the cut row tiles, then entries with sequence -1
   int merge_capacity;
-  int shares;       // CUs per kv head; 0: whole row tiles from the work list
+  int shares;       // CUs per kv head, or 0
   float slot_cost;  // piece_slot_cost of the kernel
-  int capacity;  // pieces per kv head that the list, the grid and the partial slots hold
-  float* o;      // [slot][kv head][row of the tile][D] fp32
-  float* lse;    // [slot][kv head][row of the tile]
+  int capacity;     // pieces per kv head that the list, the grid and the partial slots hold
+  float* o;         // [slot][kv head][row of the tile][D] fp32
+  float* lse;       // [slot][kv head][row of the tile]
 };
 
 struct ExtendArgs {
@@ -52,8 +52,10 @@ struct ExtendArgs {
   const int32_t* prefix;
   int num_tokens;        // rows of q and out: query rows are clamped into [0, num_tokens)
   int batch, hq, hkv, group;
-  const int64_t* items;  // work list (row_tile_item), when pieces is null
-  ExtendPieces pieces;   // work list of key pieces (pieces.list null: whole row tiles)
+  // pieces.shares == 0: whole row tiles, from the work list `items` (row_tile_item). Else key
+  // pieces: from pieces.list, or where that is null each workgroup plans its own (plan_direct).
+  const int64_t* items;
+  ExtendPieces pieces;
   int causal, window;
   float scale_log2;
   float v_scale;
@@ -87,7 +89,7 @@ __device__ __forceinline__ KeyRange row_tile_keys(int r0, int bm, int ntok, int 
 // tokens over 64-1,500 36.4 -> 26.0 us; 800 tokens at 8 / 1 heads after 8,000 253 -> 60 us.
 // Beyond one round of row tiles the pieces gained nothing that their merge did not cost:
 // 16 sequences of 300 tokens (75 row tiles, 32 CUs per kv head) 127 us either way.
-constexpr int kSplitSlotRounds = 2;  // pieces per CU share: a partial takes 128 KB per kv head at D = 128
+constexpr int kSplitSlotRounds = 2;  // pieces per CU: a partial takes 128 KB at D = 128 and 256, 256 KB above
 constexpr int kSplitMinTiles = 4;    // least key tiles of a piece (a workgroup's start and end cost about 3)
 constexpr int kDirectItems = 128;    // row tiles up to which each workgroup plans for itself, two per lane
 constexpr int kDirectBatch = 64;     // ... and sequences, one per lane
