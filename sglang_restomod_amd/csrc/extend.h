@@ -279,6 +279,8 @@ __global__ __launch_bounds__(256) void extend_merge(const ExtendArgs args) {
   constexpr int kTPR = D / 4;              // threads per row
   constexpr int kRows = 256 / kTPR;        // rows per step of a workgroup
   constexpr int kBlocks = kBM / kRows;     // steps per row tile and kv head
+  // where nothing is cut, out before the loop's constants are set up (0.4 us of the call)
+  if (cptr(reinterpret_cast<const int*>(a.pieces.merges + (int)blockIdx.x / kBlocks / a.hkv))[0] < 0) return;
   const int d = ((int)threadIdx.x % kTPR) * 4;
   const int64_t pitch = (int64_t)a.hkv * kBM;  // rows of one slot
   const int units = a.pieces.merge_capacity * a.hkv * kBlocks;

@@ -923,7 +923,7 @@ static PiecePlan piece_plan(int64_t items, int batch, int hkv, int kdim, size_t 
   // sequence, so a batch of `shares` sequences or more fills the chip by itself, and what
   // the pieces could level their launch and merge cost again (whole / pieces at D = 128, 1 to
   // 20 new tokens each: 48 sequences after 60 keys at 32 / 8 heads 24.4 / 29.6 us, after 6,000
-  // 267 / 287; 48 at 32 / 32 heads 65 / 89; below, 24 at 32 / 8 heads 17.8 / 16.7 and 166 / 136).
+  // 267 / 287; 48 at 32 / 32 heads 65 / 89; below, 24 at 32 / 8 heads 17.9 / 15.4 and 166 / 137).
   if (batch >= std::max(shares, 2) || items - batch > shares || items > kSplitMaxItems) return p;
   static_assert(kSplitSlotRounds >= 2, "a plan holds every whole row tile: items <= 2 * shares here");
   p.direct = items <= kDirectItems && batch <= kDirectBatch;
