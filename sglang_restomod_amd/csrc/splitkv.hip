@@ -1214,7 +1214,10 @@ static int splitkv_run(SplitKVArgs a, int head_dim, int q_dtype, int kv_dtype, i
     const int64_t row_groups = (a.group + 31) / 32;
     const int64_t tiles = (int64_t)a.batch * a.hkv * row_groups * ((max_seq_len + 31) / 32);
     const bool twice = head_dim > 128 && (!decode || kv_dtype == DT_BF16 || (int64_t)a.hkv * head_dim * elt > kWideRowBytes);
-    small = tiles * (twice ? 2 : 1) <= kSmallDecodeTiles && (decode || can_split || max_seq_len <= kWholeVerifyKeys);
+    // (a call without the persistent kernel's workspace stays on the row blocks, which need none)
+    const bool no_ws = !workspace || workspace_bytes < ma_splitkv_workspace_bytes(num_workgroups, head_dim);
+    small = tiles * (twice ? 2 : 1) <= kSmallDecodeTiles &&
+            (decode || can_split || max_seq_len <= kWholeVerifyKeys || no_ws);
   }
   if (generic || small) {
     // one workgroup per 16 rows (token, GQA head), its four waves splitting the keys and

@@ -115,6 +115,31 @@ def test_a_long_sequence_among_many_short_ones_is_shared(prefix, new, dim, kv):
     assert torch.equal(got, _run(case, prefix, -1, new, None))
 
 
+def test_a_small_verify_needs_no_workspace():
+    """Through the C entry with none: whole row blocks, whatever the bound."""
+    from sglang_restomod_amd.attention.mi355x import _lib, ops
+
+    print("[case] verify without a workspace", flush=True)
+    prefix = [4000] + [100] * 15
+    case = _case(prefix, [2] * 16, 32, 8, 128, F16, F16)
+    q, k, v, table, seq, qsl = case
+    want = _run(case, prefix, -1, 2, max(seq))
+    i32 = dict(dtype=torch.int32, device=DEV)
+    seq_t, qsl_t, pre_t = torch.tensor(seq, **i32), torch.tensor(qsl, **i32), torch.tensor(prefix, **i32)
+    out = torch.full(q.shape, float("nan"), dtype=torch.float32, device=DEV)
+    row, head, ps, hkv, dim = ops.kv_layout(k, 1)
+    rc = _lib.load().ma_paged_verify_bounded(
+        q.data_ptr(), q.stride(0), q.stride(1), ops.q_dtype_code(q.dtype), q.shape[0], k.data_ptr(), v.data_ptr(), row,
+        head, ops.kv_dtype_code(k.dtype), table.data_ptr(), table.stride(0), None, ps, seq_t.data_ptr(),
+        qsl_t.data_ptr(), pre_t.data_ptr(), 16, 2, 32, hkv, dim, 1, -1, ops.splitkv_workgroups(q.device), dim ** -0.5,
+        0.5, 2.0, max(seq), None, 0, out.data_ptr(), _lib.MA_DT_F32, out.stride(0), out.stride(1),
+        torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.load().ma_last_error()
+    torch.cuda.synchronize()
+    # both within the bound of the float64 checks
+    assert float((out - want).abs().max()) < 8e-3
+
+
 @pytest.mark.parametrize("prefix,heads,hkv,dim,padded,bounded,kv", [
     ([700] * 16, 16, 4, 512, 512, True, BF16), ([600] * 16, 16, 4, 192, 256, False, BF16),
     ([700] * 4, 32, 8, 96, 128, True, E4M3), ([700] * 4, 32, 8, 128, 128, True, F16),
